@@ -383,27 +383,32 @@ __global__ __launch_bounds__(kDomThreads) void nds_dominance_wide(
 // bitsets in sorted order (W words each), double-buffered across rounds.
 //
 // Workgroup g owns row blocks g, g + G, g + 2G, ... (G workgroups, spread over
-// the whole sort order).  Each owned row keeps, in LDS for the whole launch,
-// its blocking word c (the first word of its dominator row that held an
-// unassigned dominator when last looked at) and rem, the dominators of word c
-// that were still unassigned then.  Round k:
+// the whole sort order).  A row's dominator words are scanned from its last
+// one (its own block, or its row end) down to word 0.  Each owned row keeps,
+// in LDS for the whole launch, its blocking word c (the highest word of its
+// dominator row that held an unassigned dominator when last looked at) and
+// rem, the dominators of word c that were still unassigned then.  Round k:
 //   A  rem &= ~A[c] against the set assigned before round k.  A row with rem
 //      left stays blocked without touching HBM.  A row whose rem emptied reads
-//      on from c: kCheckChunks chunks from the one holding c, in one batch
-//      (four lanes a row over all 16 waves when the workgroup owns four row
-//      blocks or fewer, else a lane per row).  Rows whose dominator words run
-//      out are front k; rows still clear with words left go to the
-//      workgroup's task queue in LDS as (row, c).
+//      on below c: kCheckChunks chunks, in one batch (four lanes a row over
+//      all 16 waves when the workgroup owns four row blocks or fewer, else a
+//      lane per row).  Rows whose dominator words run out are front k; rows
+//      still clear with words left go to the workgroup's task queue in LDS as
+//      (row, c).
 //   B  the workgroup's 16 waves scan the queued rows in sweeps of one round
-//      trip per row (8 lanes and 64 words a row in the first sweep, twice as
-//      many in each later one while lanes are free), each until it meets its
-//      next blocking word (the row keeps (c, rem)) or runs out of words
-//      (front k).
+//      trip per row (as many lanes a row as the queue leaves free), each until
+//      it meets its next blocking word (the row keeps (c, rem)) or runs out of
+//      words (front k).
+// Why downwards: the dominators next to a row in the sort order (f0 just
+// below its own) are on average much deeper than those with a small f0, so the
+// blocker found first stays unassigned for most of the rounds before the row's
+// own front.  On the merged objectives of the N = 32768, M = 3, D = 1024 run
+// (generation 25, 24 fronts) the rows are scanned 176 thousand times over the
+// launch instead of 1.23 million from word 0 up, and read 121 MB of words
+// instead of 225 MB.
 // Rows, cursors, fronts and tasks never leave their workgroup (the fronts go
 // out once, when the peel stops); only the assigned set and the total cross
-// workgroups, at the one grid barrier per round.  Over all rounds a row reads
-// each of its words about once, plus what a batch reads past its blocking
-// word.
+// workgroups, at the one grid barrier per round.
 //
 // Everything the workgroups exchange inside the launch (barrier words,
 // totals, the assigned sets) is accessed with device-scope atomics, which the
@@ -437,12 +442,11 @@ constexpr int kScanLoads = 8;       // phase B: words per lane in flight (8 per 
 constexpr int kMinLanes = 8;        // phase B: fewest lanes per row (64 words a trip)
 
 // LDS layout of the peel (dynamic): s_A (W u64), s_next (bpg u64), s_task
-// (2 x 64 bpg u64), s_rem (64 bpg u64), s_cur, s_front and s_end (64 bpg int
-// each).
+// (2 x 64 bpg u64), s_rem (64 bpg u64), s_cur and s_front (64 bpg int each).
 __host__ __device__ __forceinline__ size_t peel_lds_bytes(int W, int bpg)
 {
     const size_t rows = static_cast<size_t>(bpg) * 64;
-    return static_cast<size_t>(W) * 8 + static_cast<size_t>(bpg) * 8 + rows * 36;
+    return static_cast<size_t>(W) * 8 + static_cast<size_t>(bpg) * 8 + rows * 32;
 }
 
 __device__ __forceinline__ uint64_t chunk_word(const ulonglong2 (&v)[4], int i)
@@ -464,70 +468,73 @@ __device__ __forceinline__ void peel_load_chunk(const uint64_t* rowbase, int c, 
 }
 
 // Phase A read for the lane's row (live, rem emptied): the kCheckChunks
-// chunks from the one holding cur, loaded in one batch (one HBM round trip).
-// ready: no dominator word left; queued: clear so far with words left;
-// otherwise blocked at the returned cur with the unassigned dominators of
-// that word in rem.
-__device__ __forceinline__ void peel_check(const uint64_t* __restrict__ B, int Wc, int W, int rb, int lane, int end,
+// chunks that hold the words below cur, from the one holding word cur - 1
+// down, loaded in one batch (one HBM round trip).  cur >= 1 on entry.
+// ready: no dominator word left; queued: clear so far with words left below
+// the returned cur; otherwise blocked at the returned cur with the unassigned
+// dominators of that word in rem.
+__device__ __forceinline__ void peel_check(const uint64_t* __restrict__ B, int Wc, int rb, int lane,
                                            const uint64_t* s_A, int& cur, bool& ready, bool& queued, uint64_t& rem)
 {
     const uint64_t* rowbase = peel_rowbase(B, Wc, rb, lane);
-    const int c = cur >> 3;
+    const int c = (cur - 1) >> 3;
     ulonglong2 v[kCheckChunks][4];
 #pragma unroll
     for (int a = 0; a < kCheckChunks; ++a)
-        if ((c + a) * 8 < end) peel_load_chunk(rowbase, c + a, v[a]);
+        if (c - a >= 0) peel_load_chunk(rowbase, c - a, v[a]);
     // the assigned-set words of the same span, read while the row's words
-    // are in flight (indices clamped to the set; words past stop are unused)
+    // are in flight (indices clamped to words below cur)
     uint64_t am[kCheckChunks * 8];
 #pragma unroll
-    for (int j = 0; j < kCheckChunks * 8; ++j) am[j] = s_A[min(c * 8 + j, W - 1)];
-    const int stop = min((c + kCheckChunks) * 8, end);
-    int blocked = stop;
+    for (int a = 0; a < kCheckChunks; ++a)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) am[a * 8 + i] = s_A[max(min((c - a) * 8 + i, cur - 1), 0)];
+    const int stop = max((c - kCheckChunks + 1) * 8, 0);
+    int blocked = -1;
 #pragma unroll
     for (int a = kCheckChunks - 1; a >= 0; --a) {
 #pragma unroll
-        for (int i = 7; i >= 0; --i) {
-            const int ww = (c + a) * 8 + i;
+        for (int i = 0; i < 8; ++i) {
+            const int ww = (c - a) * 8 + i;
             const uint64_t x = chunk_word(v[a], i) & ~am[a * 8 + i];
-            if (ww >= cur && ww < stop && x != 0) { blocked = ww; rem = x; }
+            if (ww >= 0 && ww < cur && x != 0) { blocked = ww; rem = x; }
         }
     }
-    cur = blocked;
-    ready = (cur >= end);
-    queued = !ready && (cur == stop);
+    cur = blocked >= 0 ? blocked : stop;
+    ready = blocked < 0 && stop == 0;
+    queued = blocked < 0 && !ready;
 }
 
 // Phase B, one trip: groups of L lanes (L = 8, 16, 32 or 64) of a wave, one
-// queued row each.  Lane sl of group gi reads words base + iL + sl
-// (i < kScanLoads, base = c rounded down to a multiple of 8) of its row: 8L
-// words a trip, each 8-word run one 64-byte segment; words before c or from
-// end on count as clear.  Returns true when the row meets a word holding an
+// queued row each.  Lane sl of group gi reads words top - iL - sl
+// (i < kScanLoads, top the last word of the chunk holding c - 1) of its row:
+// 8L words a trip, each 8-word run one 64-byte segment; words from c on or
+// below 0 count as clear.  Returns true when the row meets a word holding an
 // unassigned dominator (its index in c, its unassigned bits in rem, the same
-// in every lane of the group); otherwise c moves past the words read (to end
+// in every lane of the group); otherwise c moves below the words read (to 0
 // when they run out).  Every lane of the wave calls it; lanes of a group
 // without a row pass has = false.
-__device__ __forceinline__ bool peel_trip(const uint64_t* __restrict__ B, int Wc, int W, int pr, int& c, int end,
+__device__ __forceinline__ bool peel_trip(const uint64_t* __restrict__ B, int Wc, int W, int pr, int& c,
                                           const uint64_t* s_A, int lane, int L, bool has, uint64_t& rem)
 {
     const int sl = lane & (L - 1);
     const int shift = lane - sl;
     const uint64_t gmask = (L == 64) ? ~0ull : ((1ull << L) - 1);
-    const int base = c & ~7;
+    const int top = (c - 1) | 7;
     uint64_t x[kScanLoads];
 #pragma unroll
     for (int i = 0; i < kScanLoads; ++i) {
-        const int w = base + i * L + sl;
-        x[i] = (has && w >= c && w < end) ? B[bword_index(pr, w, Wc)] : 0ull;
+        const int w = top - i * L - sl;
+        x[i] = (has && w >= 0 && w < c) ? B[bword_index(pr, w, Wc)] : 0ull;
     }
     // the assigned-set words, read while the row's words are in flight
     uint64_t am[kScanLoads];
 #pragma unroll
-    for (int i = 0; i < kScanLoads; ++i) am[i] = s_A[min(base + i * L + sl, W - 1)];
+    for (int i = 0; i < kScanLoads; ++i) am[i] = s_A[min(max(top - i * L - sl, 0), W - 1)];
 #pragma unroll
     for (int i = 0; i < kScanLoads; ++i) {
-        const int w = base + i * L + sl;
-        x[i] = (has && w >= c && w < end) ? (x[i] & ~am[i]) : 0ull;
+        const int w = top - i * L - sl;
+        x[i] = (has && w >= 0 && w < c) ? (x[i] & ~am[i]) : 0ull;
     }
     // first blocking word of this lane's group: the lowest (i, sl)
     int first = -1;
@@ -545,11 +552,11 @@ __device__ __forceinline__ bool peel_trip(const uint64_t* __restrict__ B, int Wc
     const uint32_t lo = static_cast<uint32_t>(__shfl(static_cast<int>(hit), src));
     const uint32_t hi = static_cast<uint32_t>(__shfl(static_cast<int>(hit >> 32), src));
     if (first >= 0) {
-        c = base + first;
+        c = top - first;
         rem = (static_cast<uint64_t>(hi) << 32) | lo;
         return true;
     }
-    c = min(base + kScanLoads * L, end);
+    c = max(top + 1 - kScanLoads * L, 0);
     return false;
 }
 
@@ -576,7 +583,6 @@ __device__ __forceinline__ bool peel_body(const PeelArgs& P, int g, int G, uint6
     uint64_t* s_rem = s_task + 2 * static_cast<size_t>(rows);       // (64 bpg) unassigned bits of the blocking word
     int* s_cur = reinterpret_cast<int*>(s_rem + rows);              // (64 bpg) blocking word
     int* s_front = s_cur + rows;                                    // (64 bpg) front of each owned row
-    int* s_end = s_front + rows;                                    // (64 bpg) words 0 .. end-1 can hold dominators
     __shared__ int s_nq[3];         // queue lengths, rotating over the sweeps of phase B
     __shared__ int s_count;
     const int lane = lane_id();
@@ -585,13 +591,13 @@ __device__ __forceinline__ bool peel_body(const PeelArgs& P, int g, int G, uint6
 
     for (int j = lw; j < bpg; j += kPeelWaves) {
         const int rb = g + j * G;
-        s_cur[j * 64 + lane] = 0;
+        s_cur[j * 64 + lane] = 0;               // words 0 .. cur - 1 may hold unassigned dominators
         s_rem[j * 64 + lane] = 0ull;
         s_front[j * 64 + lane] = -1;
         if (lane == 0) s_next[j] = 0ull;
         if (rb >= nblk) continue;
         const int p = rb * 64 + lane;
-        s_end[j * 64 + lane] = (P.rend && p < P.n) ? P.rend[p] : P.hi[rb] + 1;
+        s_cur[j * 64 + lane] = (P.rend && p < P.n) ? P.rend[p] : P.hi[rb] + 1;
         if (lane == 0) { st_relaxed_u64(&P.A0[rb], 0ull); st_relaxed_u64(&P.A1[rb], 0ull); }
     }
     if (!coherent_barrier(P.state, g, G, phase, P.spin_limit)) { peel_fail(P); return false; }
@@ -618,47 +624,44 @@ __device__ __forceinline__ bool peel_body(const PeelArgs& P, int g, int G, uint6
                 const uint64_t amask = s_A[rb];
                 const int p = rb * 64 + r;
                 const int slot = j * 64 + r;
-                const int end = s_end[slot];
                 const bool live = (p < P.n) && !((amask >> r) & 1ull);
-                int cur = end;
+                int cur = 0;
                 bool ready = false, queued = false, check = false;
                 uint64_t rem = 0;
                 if (live) {
                     cur = s_cur[slot];
-                    if (cur >= end) {
-                        ready = true;
-                    } else {
-                        // still blocked while dominators of its blocking word are unassigned
-                        rem = s_rem[slot] & ~s_A[cur];
-                        check = (rem == 0);
-                    }
+                    // still blocked while dominators of its blocking word are
+                    // unassigned (before its first check rem is 0 and cur may be W)
+                    rem = s_rem[slot] & ~s_A[min(cur, P.W - 1)];
+                    ready = (rem == 0) && cur == 0;
+                    check = (rem == 0) && !ready;
                 }
                 if (ballot(check)) {
-                    const int c = cur >> 3;
-                    const int cc = c + (q >> 1);
-                    const int w0 = cc * 8 + (q & 1) * 4;
+                    const int c = (cur - 1) >> 3;
+                    const int cc = c - (q >> 1);
+                    const int w0 = cc * 8 + 4 - (q & 1) * 4;
                     ulonglong2 v0 = make_ulonglong2(0ull, 0ull), v1 = v0;
-                    if (check && cc * 8 < end) {
+                    if (check && cc >= 0) {
                         const ulonglong2* src = reinterpret_cast<const ulonglong2*>(
-                            peel_rowbase(P.B, P.Wc, rb, r) + static_cast<size_t>(cc) * 512 + (q & 1) * 4);
+                            peel_rowbase(P.B, P.Wc, rb, r) + static_cast<size_t>(cc) * 512 + 4 - (q & 1) * 4);
                         v0 = src[0];
                         v1 = src[1];
                     }
                     // the assigned-set words, read while the row's words are in flight
                     uint64_t am[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) am[i] = s_A[min(w0 + i, P.W - 1)];
-                    const int stop = min((c + kCheckChunks) * 8, end);
+                    for (int i = 0; i < 4; ++i) am[i] = s_A[min(max(w0 + i, 0), P.W - 1)];
+                    const int stop = max((c - kCheckChunks + 1) * 8, 0);
                     const uint64_t wv[4] = {v0.x, v0.y, v1.x, v1.y};
                     int fw = -1;
                     uint64_t fx = 0;
 #pragma unroll
-                    for (int i = 3; i >= 0; --i) {
+                    for (int i = 0; i < 4; ++i) {
                         const int w = w0 + i;
                         const uint64_t x = wv[i] & ~am[i];
-                        if (check && w >= cur && w < stop && x != 0) { fw = w; fx = x; }
+                        if (check && w >= 0 && w < cur && x != 0) { fw = w; fx = x; }
                     }
-                    // the row's first blocking word: from its lowest lane that has one
+                    // the row's highest blocking word: from its lowest lane that has one
                     const uint32_t gm = static_cast<uint32_t>(ballot(fw >= 0) >> (lane & ~3)) & 0xFu;
                     const int src = (lane & ~3) + (gm ? __builtin_ctz(gm) : 0);
                     const int bw = __shfl(fw, src);
@@ -670,7 +673,7 @@ __device__ __forceinline__ bool peel_body(const PeelArgs& P, int g, int G, uint6
                             rem = (static_cast<uint64_t>(hi) << 32) | lo;
                         } else {
                             cur = stop;
-                            ready = (cur >= end);
+                            ready = (stop == 0);
                             queued = !ready;
                         }
                     }
@@ -714,23 +717,20 @@ __device__ __forceinline__ bool peel_body(const PeelArgs& P, int g, int G, uint6
                 const uint64_t amask = s_A[rb];
                 const int p = rb * 64 + lane;
                 const int slot = j * 64 + lane;
-                const int end = s_end[slot];
                 const bool live = (p < P.n) && !((amask >> lane) & 1ull);
-                int cur = end;
+                int cur = 0;
                 bool ready = false, queued = false;
                 if (live) {
                     cur = s_cur[slot];
-                    if (cur >= end) {
-                        ready = true;
-                    } else {
-                        // still blocked while dominators of its blocking word are unassigned
-                        uint64_t rem = s_rem[slot] & ~s_A[cur];
-                        if (rem == 0) {
-                            peel_check(P.B, P.Wc, P.W, rb, lane, end, s_A, cur, ready, queued, rem);
-                            s_cur[slot] = cur;
-                        }
-                        s_rem[slot] = rem;
+                    // still blocked while dominators of its blocking word are
+                    // unassigned (before its first check rem is 0 and cur may be W)
+                    uint64_t rem = s_rem[slot] & ~s_A[min(cur, P.W - 1)];
+                    if (rem == 0) {
+                        if (cur == 0) ready = true;
+                        else peel_check(P.B, P.Wc, rb, lane, s_A, cur, ready, queued, rem);
+                        s_cur[slot] = cur;
                     }
+                    s_rem[slot] = rem;
                 }
                 const uint64_t ready_m = ballot(ready);
                 const uint64_t task_m = ballot(queued);
@@ -756,11 +756,9 @@ __device__ __forceinline__ bool peel_body(const PeelArgs& P, int g, int G, uint6
         // ---- phase B: the queued rows, in sweeps of one trip per row, each
         // row until it blocks or runs out of words.  Sweep s takes queue s % 2
         // (length s_nq[s % 3]) and queues the rows still clear in the other.
-        // A row gets 8 lanes (64 words a trip) in the first sweep and twice as
-        // many in each later one, up to a wave, as far as the queue leaves
-        // lanes free (8 lanes for more than 64 rows, a wave for 16 or fewer):
-        // long scans take few trips, and a row reads at most about twice the
-        // words it needs.
+        // A row gets as many lanes as the queue leaves free (a wave for 16
+        // rows or fewer, 8 lanes for more than 64): a queued row mostly runs
+        // out of words, so what it reads at once it needs.
         for (int sw = 0;; ++sw) {
             __syncthreads();
             const int nq = s_nq[sw % 3];
@@ -768,7 +766,6 @@ __device__ __forceinline__ bool peel_body(const PeelArgs& P, int g, int G, uint6
             if (threadIdx.x == 0) s_nq[(sw + 2) % 3] = 0;
             int L = 64;
             while (L > kMinLanes && nq > kPeelWaves * (64 / L)) L >>= 1;
-            L = min(L, kMinLanes << min(sw, 3));
             const int gpw = 64 / L;
             const uint64_t* q_in = s_task + (sw & 1) * static_cast<size_t>(rows);
             uint64_t* q_out = s_task + ((sw + 1) & 1) * static_cast<size_t>(rows);
@@ -779,15 +776,14 @@ __device__ __forceinline__ bool peel_body(const PeelArgs& P, int g, int G, uint6
                 const int pr = static_cast<int>(static_cast<uint32_t>(rec));
                 const int rb = pr >> 6;
                 const int slot = ((rb - g) / G) * 64 + (pr & 63);
-                const int end = has ? s_end[slot] : 0;
                 int c = static_cast<int>(rec >> 32);
                 uint64_t rem = 0;
-                const bool blocked = peel_trip(P.B, P.Wc, P.W, pr, c, end, s_A, lane, L, has, rem);
+                const bool blocked = peel_trip(P.B, P.Wc, P.W, pr, c, s_A, lane, L, has, rem);
                 if (has && (lane & (L - 1)) == 0) {
                     if (blocked) {
                         s_cur[slot] = c;
                         s_rem[slot] = rem;
-                    } else if (c >= end) {
+                    } else if (c == 0) {
                         s_front[slot] = k;
                         atomicOr(reinterpret_cast<unsigned long long*>(&s_next[(rb - g) / G]),
                                  static_cast<unsigned long long>(1ull << (pr & 63)));
