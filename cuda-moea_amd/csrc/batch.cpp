@@ -91,11 +91,13 @@ void carve_instance(Carve& c, const moea_batch_problem& p, BInst& I)
     I.chosen = c.take<int32_t>(z.n);
     I.B = c.take<uint64_t>(static_cast<size_t>(z.W) * z.Wc * 512);
     I.fs = c.take<float>(static_cast<size_t>(z.m) * z.npad);
-    I.cvs = c.take<float>(z.npad);
+    I.tables = c.take<unsigned char>(nds_table_bytes(z.nm, z.m));
     I.perm = c.take<int32_t>(z.nm);
     I.hi = c.take<int32_t>(z.W);
-    I.kind = c.take<uint8_t>(z.W);
+    I.valid = c.take<uint64_t>(8 * static_cast<size_t>(z.Wc));
     I.rend = c.take<int32_t>(z.nm);
+    I.gmask = c.take<uint64_t>(z.W);
+    I.ninfo = c.take<int32_t>(2);
     I.A = c.take<uint64_t>(2 * static_cast<size_t>(z.W));
     I.pstate = c.take<uint32_t>(kBatchPeelStateWords);
     I.wp = nullptr; I.cperm = nullptr; I.cones = nullptr; I.cone_buf = nullptr;
@@ -200,8 +202,8 @@ void fix_grids(Grids& G, const int* base)
     }
     fix(G.eval.mlp_tiles, base);
     fix(G.sel.merged256, base); fix(G.sel.rows4, base); fix(G.sel.objectives, base);
-    fix(G.nds0.rows256, base); fix(G.nds0.npad256, base); fix(G.nds0.blocks64, base);
-    fix(G.nds1.rows256, base); fix(G.nds1.npad256, base); fix(G.nds1.blocks64, base);
+    fix(G.nds0.rows256, base); fix(G.nds0.prep, base);
+    fix(G.nds1.rows256, base); fix(G.nds1.prep, base);
     fix(G.nds0.peel_first, base); fix(G.nds0.peel_jobs, base);
     fix(G.nds1.peel_first, base); fix(G.nds1.peel_jobs, base);
 }
@@ -214,8 +216,8 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
 {
     const int count = static_cast<int>(host.size());
     std::vector<long long> init256(count, 0), rows256(count, 0), sbx256(count, 0), merged256(count, 0),
-        objectives(count, 0), rows4(count, 0), mlp_tiles(count, 0), n0_rows(count, 0), n0_npad(count, 0),
-        n0_w(count, 0), n1_rows(count, 0), n1_npad(count, 0), n1_w(count, 0);
+        objectives(count, 0), rows4(count, 0), mlp_tiles(count, 0), n0_rows(count, 0), n0_prep(count, 0),
+        n1_rows(count, 0), n1_prep(count, 0);
     std::vector<std::vector<long long>> q4(kMaxM + 1, std::vector<long long>(count, 0)),
         h4(kMaxM + 1, std::vector<long long>(count, 0)), prep(kMaxM + 1, std::vector<long long>(count, 0)),
         assoc(kMaxM + 1, std::vector<long long>(count, 0)), dom0(kMaxM + 1, std::vector<long long>(count, 0)),
@@ -245,13 +247,11 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
         if (I.cones) apr[m][i] = ceil_div(nm, 4);
         else assoc[m][i] = static_cast<long long>(nb) * I.nchunks;
         n0_rows[i] = ceil_div(n, 256);
-        n0_npad[i] = ceil_div(W0 * 64, 256);
-        n0_w[i] = W0;
-        dom0[m][i] = ceil_div(4ll * Wc0 * (Wc0 + 1), 4);
+        n0_prep[i] = static_cast<long long>(Wc0) * m;
+        dom0[m][i] = static_cast<long long>(Wc0) * ceil_div(W0, kBatchDomSeg);
         n1_rows[i] = ceil_div(nm, 256);
-        n1_npad[i] = ceil_div(I.npad, 256);
-        n1_w[i] = I.W;
-        dom1[m][i] = ceil_div(4ll * I.Wc * (I.Wc + 1), 4);
+        n1_prep[i] = static_cast<long long>(I.Wc) * m;
+        dom1[m][i] = static_cast<long long>(I.Wc) * ceil_div(I.W, kBatchDomSeg);
         max_k = std::max(max_k, I.k);
         max_nm = std::max(max_nm, nm);
         peel_inst.push_back(i);
@@ -283,11 +283,9 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
     G.sel.total_merged = total_merged;
     G.sel.max_nm = static_cast<int>(max_nm);
     G.nds0.rows256 = T.add(n0_rows);
-    G.nds0.npad256 = T.add(n0_npad);
-    G.nds0.blocks64 = T.add(n0_w);
+    G.nds0.prep = T.add(n0_prep);
     G.nds1.rows256 = T.add(n1_rows);
-    G.nds1.npad256 = T.add(n1_npad);
-    G.nds1.blocks64 = T.add(n1_w);
+    G.nds1.prep = T.add(n1_prep);
     for (int m = 1; m <= kMaxM; ++m) {
         G.nds0.dom[m] = T.add(dom0[m]);
         G.nds1.dom[m] = T.add(dom1[m]);
@@ -308,8 +306,8 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
     return total_merged;
 }
 
-// Prefix tables per state: (1 + 3 + 2 kMaxM + 1 + 3 + 3 kMaxM + 3 + 3 + 2 kMaxM) grids.
-constexpr int kGridsPerState = 14 + 7 * kMaxM;
+// Prefix tables per state: (1 + 3 + 2 kMaxM + 1 + 3 + 3 kMaxM + 2 + 2 + 2 kMaxM) grids.
+constexpr int kGridsPerState = 12 + 7 * kMaxM;
 
 }  // namespace
 

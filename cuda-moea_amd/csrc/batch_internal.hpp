@@ -20,6 +20,7 @@
 namespace moea {
 
 constexpr int kBatchPeelStateWords = 1024 + 64;   // per instance: peel group barrier flags and totals
+constexpr int kBatchDomSeg = 64;                   // row blocks per dominance workgroup
 constexpr int kBatchPeelMaxLds = 80 * 1024;        // LDS bound of one batched peel block
 
 struct BInst {
@@ -76,11 +77,13 @@ struct BInst {
     // NDS scratch (2n merged rows, or n for the initial parents)
     uint64_t* B;                  // (W * Wc * 512) dominator bitmask, sorted order
     float* fs;                    // (m, npad) sorted objectives
-    float* cvs;                   // (npad)
+    unsigned char* tables;        // (Wc, m) rank tables of the dominance kernel
     int32_t* perm;                // (nm) sorted position -> local row
     int32_t* hi;                  // (W)
-    uint8_t* kind;                // (W)
+    uint64_t* valid;              // (8 Wc) feasible rows without a NaN objective, sorted order
     int32_t* rend;                // (nm) sorted row -> 1 + last word holding a dominator (0: none)
+    uint64_t* gmask;              // (W) first rows of each distinct infeasible cv, sorted order
+    int32_t* ninfo;               // (2) feasible rows, end of the infeasible rows whose cv is a number
     uint64_t* A;                  // (2 W) assigned sets of the peel (this round, next round)
     uint32_t* pstate;             // (kBatchPeelStateWords) peel barrier and totals
     long long key_off;            // first of this instance's nm entries in the batch key arrays
@@ -125,9 +128,8 @@ struct BatchLaunch {
 // the 2n merged rows.
 struct BNdsGrids {
     BGrid rows256;                // nds keys: rows per instance, 256 per block
-    BGrid npad256;                // sorted gather: 64 W per instance, 256 per block
-    BGrid blocks64;               // block info: W one-wave blocks per instance
-    BGrid dom[kMaxM + 1];         // dominance units, 4 per block, of the instances with m objectives
+    BGrid prep;                   // sorted objectives, tie bounds and rank tables: Wc x m blocks per instance
+    BGrid dom[kMaxM + 1];         // dominance: Wc x ceil(W / kBatchDomSeg) blocks, instances with m objectives
     long long total_rows;         // sum of rows (sort length)
     // peel: cooperative launch of peel_wgs blocks; block w runs
     // peel_jobs[peel_first[w] .. peel_first[w + 1]) (instance, rank, group size)
@@ -181,6 +183,7 @@ int batch_evaluate(const BatchLaunch& L, const BEvalGrids& G, int which);       
 int mlp_tile_count(int n, int hidden);            // blocks of one MLP hidden-layer launch       // evaluate.hip
 size_t batch_nds_sort_bytes(long long total_rows, int inst_bits);                             // nds.hip
 int batch_nds(const BatchLaunch& L, const BNdsGrids& G, const BNdsScratch& S, int mode, int state);  // nds.hip
+size_t nds_table_bytes(int nm, int m);                                                        // nds.hip
 int batch_peel_capacity();                                                                    // nds.hip
 int batch_peel_plan(const std::vector<int>& inst, const std::vector<int>& W, int capacity, int rows_per_block,
                     std::vector<int>& first, std::vector<int>& jobs, size_t& lds);           // nds.hip

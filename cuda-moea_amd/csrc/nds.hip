@@ -17,17 +17,24 @@
 //     infeasible one, a NaN objective compares false both ways, infeasible
 //     rows dominate by strictly smaller cv, and q <= p in every objective with
 //     f0(q) > f0(p) is impossible.
-//  2. nds_block_prep: objectives and cv in sorted order; per 64-row block b,
-//     kind[b] (all rows in segment 0?) and hi[b], the last block holding a row
-//     whose key equals the key of block b's last row (b itself unless an f0
-//     tie runs past the block).  Dominators of a row of block b all lie in
-//     blocks <= hi[b].
+//  2. nds_prep: objectives in sorted order; per 64-row block b, valid[b] (which
+//     rows are in segment 0) and hi[b], the last block holding a row whose key
+//     equals the key of block b's last row (b itself unless an f0 tie runs past
+//     the block).  Dominators of a row of block b all lie in blocks <= hi[b].
+//     Per chunk of 512 sorted rows and objective, a rank table (see RankTable).
 //  3. nds_dominance: the dominator bitmask B in sorted order, words (p, w) for
-//     w <= hi[p/64].  Tiles below the diagonal whose blocks are all segment 0
-//     and not tied need only "q_k <= p_k for k >= 1" (f0 is already strictly
-//     smaller for every q of the earlier block): M - 1 compares per pair.
-//  4. nds_peel: front peeling with per-row cursors on B in one cooperative
-//     launch; fronts are written back in input order.
+//     w <= hi[p/64], from the rank tables: a search and a table row per
+//     objective give a row's "q_k <= p_k" over a whole chunk.
+//  4. nds_peel: front peeling of the feasible rows with per-row cursors on B
+//     in one cooperative launch; the infeasible rows' fronts follow from their
+//     order alone; fronts are written back in input order.
+//
+// Infeasible rows need no bitmask: every feasible row dominates them, among
+// themselves they are ordered by cv alone, and a NaN cv neither dominates nor
+// is dominated by another infeasible row.  So with F feasible fronts the rows
+// with the j-th smallest distinct cv are front F + j and the NaN rows front F.
+// Peeled one front a round they cost a grid barrier per distinct cv: 17.2 ms
+// for 20001 rows of which a fifth are infeasible, against 0.2 ms this way.
 //
 // Data layout of B (u64 words, sorted row index p):
 //   W  = ceil(n / 64) words per row (bit q%64 of word q/64 = "q dominates p"),
@@ -50,11 +57,10 @@ namespace moea {
 namespace {
 
 constexpr int kRowEndMinM = 4;           // fewest objectives for which the sort computes row ends
-constexpr int kDomWaves = 4;             // waves (work units) per dominance workgroup
-constexpr int kDomThreads = 64 * kDomWaves;
+constexpr int kDomThreads = 512;         // dominance workgroup: each wave takes a row block at a time
+constexpr int kDomWaves = kDomThreads / 64;
+constexpr int kChunk = 512;              // sorted rows q per rank table: the 8 words of a chunk of B
 constexpr int kKeyBits = 34;             // segment (2 bits) above a 32-bit order key
-constexpr uint8_t kPlain = 0;            // every row of the block is in segment 0
-constexpr uint8_t kMixed = 1;
 
 __host__ __device__ __forceinline__ size_t bword_index(int p, int w, int Wc)
 {
@@ -90,290 +96,355 @@ __global__ void nds_keys(const float* __restrict__ f, int ldf, const float* __re
     vals[s] = s;
 }
 
-// Sorted copies of the objectives (m rows of npad) and cv of row t; padding
-// rows are 0.
-__device__ __forceinline__ void gather_sorted_row(const float* __restrict__ f, int ldf, const float* __restrict__ cv,
-                                                  int n, int m, int npad, const int32_t* __restrict__ perm,
-                                                  float* __restrict__ fs, float* __restrict__ cvs, int t)
+// The infeasible rows of the sort order, found by one wave per 64-row block:
+// gmask[b] has a bit for each row of block b that is the first of its cv (NaN
+// cv left out); info[kInfoFeasible] is the number of feasible rows and
+// info[kInfoOrdered] the end of the rows with a cv that is not NaN, each
+// written by the wave whose row comes just before (row 0's wave for 0).
+constexpr int kInfoFeasible = 0, kInfoOrdered = 1;
+
+__device__ __forceinline__ int infeasible_class(uint64_t key)
 {
-    if (t >= npad) return;
-    if (t < n) {
-        const int s = perm[t];
-        for (int k = 0; k < m; ++k) fs[static_cast<size_t>(k) * npad + t] = f[static_cast<size_t>(k) * ldf + s];
-        cvs[t] = cv[s];
-    } else {
-        for (int k = 0; k < m; ++k) fs[static_cast<size_t>(k) * npad + t] = 0.0f;
-        cvs[t] = 0.0f;
+    return ((key >> 32) & 3u) != 2 ? 0 : static_cast<uint32_t>(key) != 0xFFFFFFFFu ? 1 : 2;
+}
+
+__device__ __forceinline__ void infeasible_info(const uint64_t* __restrict__ keys, int n, int t,
+                                                uint64_t* __restrict__ gmask, int32_t* __restrict__ info)
+{
+    const bool valid = t < n;
+    const uint64_t key = valid ? keys[t] : 0;
+    const uint64_t prev = (valid && t > 0) ? keys[t - 1] : 0;
+    // 0 feasible, 1 infeasible with a number, 2 NaN cv, 3 past the end
+    const int c = valid ? infeasible_class(key) : 3;
+    const int c0 = t > 0 ? infeasible_class(prev) : 0;
+    const uint64_t starts = ballot(c == 1 && (t == 0 || prev != key));
+    if ((threadIdx.x & 63) == 0) gmask[t >> 6] = starts;
+    if (valid && c0 == 0 && c != 0) info[kInfoFeasible] = t;
+    if (valid && c0 <= 1 && c == 2) info[kInfoOrdered] = t;
+    if (t == n - 1) {
+        if (c == 0) info[kInfoFeasible] = n;
+        if (c <= 1) info[kInfoOrdered] = n;
     }
 }
 
-// One wave per 64-row block: kind[b] and hi[b] (see the header comment).  The
-// segment is bits 32-33 of the key (higher bits may carry a batch index).
-__device__ __forceinline__ void block_info_one(const uint64_t* __restrict__ keys, int n, int b,
-                                      uint8_t* __restrict__ kind, int32_t* __restrict__ hi)
+// hi[b] of the block whose last row is `last` (see the header comment), read
+// by one lane.  Ties past a block are rare, so the next key is looked at before
+// the search.
+__device__ __forceinline__ int tie_end_block(const uint64_t* __restrict__ keys, int n, int last)
 {
-    const int t = b * 64 + static_cast<int>(threadIdx.x);
-    const bool other = (t < n) && ((keys[t] >> 32) & 3u) != 0;
-    const uint64_t any_other = ballot(other);
-    if (threadIdx.x != 0) return;
-    kind[b] = any_other ? kMixed : kPlain;
-    const int last = min(n, b * 64 + 64) - 1;
     const uint64_t kl = keys[last];
-    int end = last;
-    if (((kl >> 32) & 3u) == 0) {
-        // first position after `last` whose key differs (keys ascend)
-        int lo = last + 1, hi_ = n;
-        while (lo < hi_) {
-            const int mid = (lo + hi_) >> 1;
-            if (keys[mid] == kl) lo = mid + 1;
-            else hi_ = mid;
-        }
-        end = lo - 1;
+    if (last + 1 >= n || ((kl >> 32) & 3u) != 0 || keys[last + 1] != kl) return last >> 6;
+    // first position after `last` whose key differs (keys ascend)
+    int lo = last + 2, hi = n;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (keys[mid] == kl) lo = mid + 1;
+        else hi = mid;
     }
-    hi[b] = end >> 6;
+    return (lo - 1) >> 6;
 }
 
-// One 64-thread block per 64-row block after the sort: the block's sorted
-// objectives and cv (gather_sorted_row) and its kind and tie bound
-// (block_info_one).  zero (optional, `words` of them): cleared on the way, for
-// a later launch; mf_init (optional): set to -1, the value the peel replaces
-// with its result; rend (optional, one per padded row): set to 0, the row ends
-// the dominance kernel raises.
-__global__ __launch_bounds__(64) void nds_block_prep(const float* __restrict__ f, int ldf,
-                                                     const float* __restrict__ cv, int m, int npad,
-                                                     const int32_t* __restrict__ perm, float* __restrict__ fs,
-                                                     float* __restrict__ cvs, const uint64_t* __restrict__ keys, int n,
-                                                     uint8_t* __restrict__ kind, int32_t* __restrict__ hi,
-                                                     uint32_t* __restrict__ zero, int words,
-                                                     int32_t* __restrict__ mf_init, int32_t* __restrict__ rend)
+// Rank table of one objective over a chunk of kChunk sorted rows, in sub-chunks
+// of S rows: the S values in ascending order, and for each r = 0 .. S the mask
+// of the rows among the r smallest (S bits).  A row p whose objective has r
+// values <= p_k among the S gets "q_k <= p_k" for all of them from mask r, so a
+// (row, chunk, objective) costs a search and one 64-byte read instead of 512
+// compares; "q_k == p_k" is mask r without the mask of the values < p_k.
+//   bytes [0, 2048): float values, sub-chunk h at 4 S h;
+//   then per sub-chunk S + 1 masks of S / 8 bytes in 16-byte pieces, pieces of
+//   a mask swapped by bit 3 of r where a mask has two: reads at random r then
+//   spread over all LDS banks instead of half of them.
+// A small S makes the table smaller and the sort below shorter, a large one the
+// searches fewer (9 steps per 256 rows against 8 per 128).  S = 256 holds up
+// to 8 objectives' tables in LDS (7 x 18.5 KB; the first objective needs none),
+// S = 128 up to 10 (9 x 10.3 KB).
+constexpr int rank_sub(int m) { return m <= 8 ? 256 : 128; }
+constexpr int kRankValueBytes = kChunk * 4;
+constexpr int rank_mask_bytes(int S) { return (S + 1) * (S / 8); }         // one sub-chunk's masks
+__host__ __device__ constexpr int rank_table_bytes(int S)
 {
-    gather_sorted_row(f, ldf, cv, n, m, npad, perm, fs, cvs, static_cast<int>(blockIdx.x * 64 + threadIdx.x));
-    for (int j = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x); j < words;
-         j += static_cast<int>(gridDim.x * blockDim.x))
-        zero[j] = 0u;
-    if (mf_init && blockIdx.x == 0 && threadIdx.x == 0) mf_init[0] = -1;
-    if (rend) rend[blockIdx.x * 64 + threadIdx.x] = 0;
-    block_info_one(keys, n, static_cast<int>(blockIdx.x), kind, hi);
+    return (kRankValueBytes + (kChunk / S) * ((S + 1) * (S / 8)) + 255) / 256 * 256;
 }
+// the largest of an objective count's tables per chunk, for buffers sized without it
+constexpr int kRankChunkBytes = 10 * rank_table_bytes(128) > 8 * rank_table_bytes(256) ? 10 * rank_table_bytes(128)
+                                                                                     : 8 * rank_table_bytes(256);
+static_assert(kMaxM == 10, "kRankChunkBytes covers 8 and 10 objectives");
 
-// Tile in which every earlier row q (block qb, wave-uniform) has f0 strictly
-// below every row p (lane): q dominates p iff q_k <= p_k for k = 1..M-1.
-// Returns the row word of lane p over the 64 rows q of the block.
-template <int M>
-__device__ __forceinline__ uint64_t tile_fast(const float* __restrict__ fs, int npad, int q0,
-                                     const float (&pv)[M])
+// Byte offset of 16-byte piece j of mask r.
+template <int S>
+__device__ __forceinline__ int rank_piece(int r, int j)
 {
-    constexpr int G = (M <= 5) ? 16 : 8;   // rows q per group of scalar loads
-    uint32_t acc_hi = 0, acc_lo = 0;
-    static_for([&](auto GC) {
-        constexpr int g0 = 64 - G * (decltype(GC)::value + 1);   // groups in descending order
-        float qv[M > 1 ? M - 1 : 1][G];
-#pragma unroll
-        for (int k = 1; k < M; ++k)
-#pragma unroll
-            for (int i = 0; i < G; ++i) qv[k - 1][i] = ld_uniform(fs, static_cast<size_t>(k) * npad + q0 + g0 + i);
-        static_for([&](auto IC) {
-            constexpr int i = G - 1 - decltype(IC)::value;
-            constexpr int j = g0 + i;                  // descending: bit j lands at position j
-            uint64_t dom = ~0ull;
-#pragma unroll
-            for (int k = 1; k < M; ++k) dom &= mask_not_gt(qv[k - 1][i], pv[k]);
-            if (j >= 32) acc_hi = shift_in(acc_hi, dom);
-            else acc_lo = shift_in(acc_lo, dom);
-        }, std::make_integer_sequence<int, G>{});
-    }, std::make_integer_sequence<int, 64 / G>{});
-    return (static_cast<uint64_t>(acc_hi) << 32) | acc_lo;
+    if constexpr (S == 256) return (2 * r + (j ^ ((r >> 3) & 1))) * 16;
+    else return r * 16;
 }
 
-// Any tile with the full constrained rule.  Row word of lane p over the rows q
-// of block qb (q < n, q != p); when `backward` is set, the words "p dominates
-// q" of the rows q are stored at word pb of their rows (tied tiles only).
-template <int M>
-__device__ __forceinline__ uint64_t tile_general(const float* __restrict__ fs, const float* __restrict__ cvs,
-                                        int npad, int n, int qb, int pb, const float (&pv)[M],
-                                        float cp, bool backward, uint64_t* __restrict__ B, int Wc,
-                                        int32_t* __restrict__ rend)
-{
-    const int lane = lane_id();
-    const int p = pb * 64 + lane;
-    const bool pvalid = p < n;
-    const bool pf = (cp == 0.0f);
-    const int q0 = qb * 64;
-    uint32_t acc_hi = 0, acc_lo = 0;
-    uint32_t col_lo = 0, col_hi = 0;
-    static_for([&](auto JC) {
-        constexpr int j = 63 - decltype(JC)::value;
-        const int q = q0 + j;
-        uint64_t qdp_m = 0, pdq_m = 0;
-        if (q < n) {
-            const float cq = ld_uniform(cvs, q);
-            const bool qf = (cq == 0.0f);
-            bool le_qp = true, lt_qp = false, le_pq = true, lt_pq = false;
-#pragma unroll
-            for (int k = 0; k < M; ++k) {
-                const float qk = ld_uniform(fs, static_cast<size_t>(k) * npad + q);
-                le_qp = le_qp && (qk <= pv[k]);
-                lt_qp = lt_qp || (qk < pv[k]);
-                le_pq = le_pq && (pv[k] <= qk);
-                lt_pq = lt_pq || (pv[k] < qk);
-            }
-            const bool qdp = (qf && !pf) || (!qf && !pf && (cq < cp)) || (qf && pf && le_qp && lt_qp);
-            const bool pdq = (pf && !qf) || (!pf && !qf && (cp < cq)) || (pf && qf && le_pq && lt_pq);
-            qdp_m = ballot(qdp && q != p);
-            pdq_m = ballot(pdq && pvalid && q != p);
-        }
-        if (j >= 32) acc_hi = shift_in(acc_hi, qdp_m);
-        else acc_lo = shift_in(acc_lo, qdp_m);
-        if (backward) {
-            col_lo = writelane<j>(col_lo, static_cast<uint32_t>(pdq_m));
-            col_hi = writelane<j>(col_hi, static_cast<uint32_t>(pdq_m >> 32));
-        }
-    }, std::make_integer_sequence<int, 64>{});
-    if (backward) {
-        const int q = q0 + lane;
-        if (q < n) {
-            B[bword_index(q, pb, Wc)] = (static_cast<uint64_t>(col_hi) << 32) | col_lo;
-            if (rend && (col_hi | col_lo)) atomicMax(&rend[q], pb + 1);
-        }
-    }
-    return (static_cast<uint64_t>(acc_hi) << 32) | acc_lo;
-}
-
-// The same, out of line.  Inlined, the 64 unrolled steps of tile_general raise
-// the SGPR count of the dominance kernel past what fits without spilling, and
-// the spill code runs inside the fast tiles' loop; out of line, the call costs
-// more than the spills where diagonal tiles are common (a few row blocks).
-// The row's objectives go by value, in registers (by reference they would be
-// stored to scratch in every unit).  Up to kOutlineMaxM objectives: from 7 the
-// out-of-line form lowers the occupancy and the inlined one measured faster
-// (M = 8, n = 65536: 0.97 against 1.00 ms).
-constexpr int kOutlineMaxM = 6;
-template <int M>
-struct RowObjectives {
-    float v[M];
+// What nds_prep writes besides the tables.
+struct PrepOut {
+    float* fs;               // (m, npad) sorted objectives, 0 in padding rows
+    uint64_t* valid;         // (8 Wc) rows of segment 0 per block, 0 past the last block
+    int32_t* hi;             // (W)
+    uint64_t* gmask;         // (W) see infeasible_info
+    int32_t* info;           // (2)
+    int32_t* rend;           // optional (n): row ends, cleared for the dominance kernel to raise
+    unsigned char* tables;   // (Wc, m) rank tables
 };
 
-template <int M>
-__device__ __attribute__((noinline)) uint64_t tile_general_call(const float* __restrict__ fs,
-                                                                const float* __restrict__ cvs, int npad, int n, int qb,
-                                                                int pb, RowObjectives<M> pv, float cp, bool backward,
-                                                                uint64_t* __restrict__ B, int Wc,
-                                                                int32_t* __restrict__ rend)
+// One workgroup of kChunk threads: chunk qc, objective k.
+template <int S>
+__device__ __forceinline__ void prep_chunk(const float* __restrict__ f, int ldf, int n, int m, int npad,
+                                           const int32_t* __restrict__ perm, const uint64_t* __restrict__ keys,
+                                           int qc, int k, const PrepOut& O)
 {
-    return tile_general<M>(fs, cvs, npad, n, qb, pb, pv.v, cp, backward, B, Wc, rend);
-}
-
-template <int M>
-__device__ __forceinline__ RowObjectives<M> row_pv(const float (&pv)[M])
-{
-    RowObjectives<M> r;
-#pragma unroll
-    for (int k = 0; k < M; ++k) r.v[k] = pv[k];
-    return r;
-}
-
-// Work unit u -> (row block pb, chunk qc), qc <= pb / 8.  Units are grouped by
-// a = pb / 8: group a holds 8 row blocks x (a + 1) chunks.
-__device__ __forceinline__ void decode_unit(long long u, int& pb, int& qc)
-{
-    long long a = static_cast<long long>((sqrt(1.0 + static_cast<double>(u)) - 1.0) * 0.5);
-    while (4 * a * (a + 1) > u) --a;
-    while (4 * (a + 1) * (a + 2) <= u) ++a;
-    const long long rem = u - 4 * a * (a + 1);
-    pb = static_cast<int>(8 * a + rem / (a + 1));
-    qc = static_cast<int>(rem % (a + 1));
-}
-
-// One wave per unit (pb, qc): the 8 words (p, 8qc .. 8qc+7) of the 64 rows of
-// block pb, accumulated in registers and written as one 64-byte segment per
-// lane.  In the diagonal chunk only words <= pb are written; words past pb
-// belong to tied tiles, whose backward direction the wave of the later block
-// stores.  rend (optional): each row's end, one past its last non-zero word,
-// raised with atomicMax from every unit that holds a non-zero word of it.
-template <int M, bool kOutline = false>
-__device__ __forceinline__ void dom_unit(const float* __restrict__ fs, const float* __restrict__ cvs, int npad,
-                                int n, int W, int Wc, const uint8_t* __restrict__ kind,
-                                const int32_t* __restrict__ hi, uint64_t* __restrict__ B, long long u,
-                                int32_t* __restrict__ rend = nullptr)
-{
-    int pb, qc;
-    decode_unit(u, pb, qc);
-    pb = wave_uniform(pb);
-    qc = wave_uniform(qc);
-    if (pb >= W) return;
+    __shared__ __align__(16) float s_v[kChunk];
+    __shared__ int s_rank[kChunk];
+    const int tid = static_cast<int>(threadIdx.x);
     const int lane = lane_id();
-    const int p = pb * 64 + lane;
-    float pv[M];
-#pragma unroll
-    for (int k = 0; k < M; ++k) pv[k] = fs[static_cast<size_t>(k) * npad + p];
-    const float cp = cvs[p];
-    const bool p_plain = ld_uniform(kind, pb) == kPlain;
-
-    uint64_t w0 = 0, w1 = 0, w2 = 0, w3 = 0, w4 = 0, w5 = 0, w6 = 0, w7 = 0;
-#pragma unroll 1
-    for (int t = 0; t < 8; ++t) {
-        const int qb = qc * 8 + t;
-        uint64_t word = 0;
-        if (qb < pb) {
-            const bool tied = ld_uniform(hi, qb) >= pb;
-            if (!tied && p_plain && ld_uniform(kind, qb) == kPlain) word = tile_fast<M>(fs, npad, qb * 64, pv);
-            else if constexpr (kOutline && M <= kOutlineMaxM) word = tile_general_call<M>(fs, cvs, npad, n, qb, pb, row_pv(pv), cp, tied, B, Wc, rend);
-            else word = tile_general<M>(fs, cvs, npad, n, qb, pb, pv, cp, tied, B, Wc, rend);
-        } else if (qb == pb) {
-            if constexpr (kOutline && M <= kOutlineMaxM) word = tile_general_call<M>(fs, cvs, npad, n, qb, pb, row_pv(pv), cp, false, B, Wc, rend);
-            else word = tile_general<M>(fs, cvs, npad, n, qb, pb, pv, cp, false, B, Wc, rend);
+    const int w = wave_uniform(tid >> 6);
+    const int t = qc * kChunk + tid;
+    const float v = t < n ? f[static_cast<size_t>(k) * ldf + perm[t]] : 0.0f;
+    if (t < npad) O.fs[static_cast<size_t>(k) * npad + t] = v;
+    if (k == 0) {
+        // the wave's 64 rows are block 8 qc + w
+        const int b = qc * 8 + w;
+        const uint64_t seg0 = ballot(t < n && ((keys[min(t, n - 1)] >> 32) & 3u) == 0);
+        if (lane == 0) O.valid[b] = seg0;
+        if (b * 64 < n) {
+            infeasible_info(keys, n, t, O.gmask, O.info);
+            if (lane == 0) O.hi[b] = tie_end_block(keys, n, min(n, b * 64 + 64) - 1);
+            if (O.rend && t < n) O.rend[t] = 0;
         }
-        // rotate: after 8 steps w0..w7 hold tiles 0..7
-        w0 = w1; w1 = w2; w2 = w3; w3 = w4; w4 = w5; w5 = w6; w6 = w7; w7 = word;
     }
-    uint64_t* dst = B + ((static_cast<size_t>(pb) * Wc + qc) * 64 + lane) * 8;
-    if (qc * 8 + 7 < pb) {
-        ulonglong2* d2 = reinterpret_cast<ulonglong2*>(dst);
-        d2[0] = make_ulonglong2(w0, w1);
-        d2[1] = make_ulonglong2(w2, w3);
-        d2[2] = make_ulonglong2(w4, w5);
-        d2[3] = make_ulonglong2(w6, w7);
-    } else {
-        const int last = pb - qc * 8;   // words 0..last of this chunk
-        dst[0] = w0;
-        if (last >= 1) dst[1] = w1;
-        if (last >= 2) dst[2] = w2;
-        if (last >= 3) dst[3] = w3;
-        if (last >= 4) dst[4] = w4;
-        if (last >= 5) dst[5] = w5;
-        if (last >= 6) dst[6] = w6;
-        if (last >= 7) dst[7] = w7;
+    // rows without a number are never looked up (valid masks them): any order does
+    const float x = (t < n && !isnan(v)) ? v : INFINITY;
+    s_v[tid] = x;
+    __syncthreads();
+    // rank of each value among its sub-chunk, ties by position
+    const int h = wave_uniform(tid / S);
+    const int w0 = h * (S / 64);
+    int rank = 0;
+#pragma unroll 1
+    for (int b = 0; b < S / 64; ++b) {
+        const float4* src = reinterpret_cast<const float4*>(s_v + h * S + b * 64);
+        const int own = w - w0;
+        if (b == own) {
+#pragma unroll 4
+            for (int j = 0; j < 16; ++j) {
+                const float4 u = src[j];
+                rank += (u.x < x || (u.x == x && 4 * j < lane)) ? 1 : 0;
+                rank += (u.y < x || (u.y == x && 4 * j + 1 < lane)) ? 1 : 0;
+                rank += (u.z < x || (u.z == x && 4 * j + 2 < lane)) ? 1 : 0;
+                rank += (u.w < x || (u.w == x && 4 * j + 3 < lane)) ? 1 : 0;
+            }
+        } else if (b < own) {
+#pragma unroll 4
+            for (int j = 0; j < 16; ++j) {
+                const float4 u = src[j];
+                rank += (u.x <= x) + (u.y <= x) + (u.z <= x) + (u.w <= x);
+            }
+        } else {
+#pragma unroll 4
+            for (int j = 0; j < 16; ++j) {
+                const float4 u = src[j];
+                rank += (u.x < x) + (u.y < x) + (u.z < x) + (u.w < x);
+            }
+        }
     }
-    if (rend && p < n) {
-        const int top = w7 ? 8 : w6 ? 7 : w5 ? 6 : w4 ? 5 : w3 ? 4 : w2 ? 3 : w1 ? 2 : w0 ? 1 : 0;
-        if (top) atomicMax(&rend[p], qc * 8 + top);
+    s_rank[tid] = rank;
+    unsigned char* tab = O.tables + (static_cast<size_t>(qc) * m + k) * rank_table_bytes(S);
+    reinterpret_cast<float*>(tab)[h * S + rank] = x;
+    // wave w: its 64 rows' word of every mask of their sub-chunk, 64 masks at a
+    // time with a lane per mask (bit e: row e's rank < r)
+    int re[64];
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 64; ++e) re[e] = wave_uniform(s_rank[w * 64 + e]);
+    unsigned char* masks = tab + kRankValueBytes + h * rank_mask_bytes(S);
+    const int jj = w - w0;
+#pragma unroll 1
+    for (int r0 = 0; r0 <= S; r0 += 64) {
+        const int r = r0 + lane;
+        uint32_t lo = 0, hi = 0;
+#pragma unroll
+        for (int e = 31; e >= 0; --e) {
+            lo = shift_in(lo, ballot(re[e] < r));
+            hi = shift_in(hi, ballot(re[e + 32] < r));
+        }
+        if (r <= S)
+            *reinterpret_cast<uint64_t*>(masks + rank_piece<S>(r, jj >> 1) + (jj & 1) * 8) =
+                (static_cast<uint64_t>(hi) << 32) | lo;
     }
 }
 
-template <int M>
-__global__ __launch_bounds__(kDomThreads) void nds_dominance(
-    const float* __restrict__ fs, const float* __restrict__ cvs, int npad, int n, int W, int Wc,
-    const uint8_t* __restrict__ kind, const int32_t* __restrict__ hi, uint64_t* __restrict__ B,
-    long long units, int32_t* __restrict__ rend)
+// Grid (Wc, m).  zero (optional, `words` of them): cleared on the way, for a
+// later launch; mf_init: set to -1, the value the peel replaces with its result.
+template <int S>
+__global__ __launch_bounds__(kChunk) void nds_prep(const float* __restrict__ f, int ldf, int n, int m, int npad,
+                                                   const int32_t* __restrict__ perm,
+                                                   const uint64_t* __restrict__ keys, PrepOut O,
+                                                   uint32_t* __restrict__ zero, int words,
+                                                   int32_t* __restrict__ mf_init)
 {
-    const int wave = wave_uniform(static_cast<int>(threadIdx.x >> 6));
-    const long long u = static_cast<long long>(blockIdx.x) * kDomWaves + wave;
-    if (u >= units) return;
-    dom_unit<M>(fs, cvs, npad, n, W, Wc, kind, hi, B, u, rend);
+    if (blockIdx.x == 0 && blockIdx.y == 0) {
+        for (int j = static_cast<int>(threadIdx.x); j < words; j += kChunk) zero[j] = 0u;
+        if (threadIdx.x == 0) mf_init[0] = -1;
+    }
+    prep_chunk<S>(f, ldf, n, m, npad, perm, keys, static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), O);
 }
 
-// The same for many row blocks, where nearly every tile is a fast one: the
-// general tiles out of line keep the fast loop free of spill code.
-template <int M>
-__global__ __launch_bounds__(kDomThreads) void nds_dominance_wide(
-    const float* __restrict__ fs, const float* __restrict__ cvs, int npad, int n, int W, int Wc,
-    const uint8_t* __restrict__ kind, const int32_t* __restrict__ hi, uint64_t* __restrict__ B,
-    long long units, int32_t* __restrict__ rend)
+// Number of the S ascending values v[0 .. S) that are <= x (kLess: < x).
+template <int S, bool kLess>
+__device__ __forceinline__ int rank_search(const float* v, float x)
 {
-    const int wave = wave_uniform(static_cast<int>(threadIdx.x >> 6));
-    const long long u = static_cast<long long>(blockIdx.x) * kDomWaves + wave;
-    if (u >= units) return;
-    dom_unit<M, true>(fs, cvs, npad, n, W, Wc, kind, hi, B, u, rend);
+    int pos = 0;
+#pragma unroll
+    for (int step = S / 2; step >= 1; step >>= 1) {
+        const float u = v[pos + step - 1];
+        pos += (kLess ? u < x : u <= x) ? step : 0;
+    }
+    const float u = v[pos];
+    return pos + ((kLess ? u < x : u <= x) ? 1 : 0);
+}
+
+// The 512 bits of a table for x: rows with a value <= x (kLess: < x).
+template <int S, bool kLess>
+__device__ __forceinline__ void rank_bits(const unsigned char* tab, float x, uint64_t (&out)[8])
+{
+    int r[kChunk / S];
+#pragma unroll
+    for (int h = 0; h < kChunk / S; ++h) r[h] = rank_search<S, kLess>(reinterpret_cast<const float*>(tab) + h * S, x);
+#pragma unroll
+    for (int h = 0; h < kChunk / S; ++h) {
+        const unsigned char* masks = tab + kRankValueBytes + h * rank_mask_bytes(S);
+#pragma unroll
+        for (int j = 0; j < S / 128; ++j) {
+            const ulonglong2 u = *reinterpret_cast<const ulonglong2*>(masks + rank_piece<S>(r[h], j));
+            out[h * (S / 64) + 2 * j] = u.x;
+            out[h * (S / 64) + 2 * j + 1] = u.y;
+        }
+    }
+}
+
+// A chunk whose f0 ties with row block pb, or that holds pb itself (or rows
+// after it): every objective's <=, without the rows equal in all of them.  The
+// first objective's table is read where nds_prep left it.
+template <int M, int S>
+__device__ __forceinline__ void tied_bits(const unsigned char* tab0, const unsigned char* s_tab, const float (&pv)[M],
+                                          uint64_t (&bits)[8])
+{
+    uint64_t eq[8], lt[8], le[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) eq[j] = ~0ull;
+#pragma unroll 1
+    for (int k = 0; k < M; ++k) {
+        const unsigned char* tab = k == 0 ? tab0 : s_tab + (k - 1) * rank_table_bytes(S);
+        float x = pv[0];
+#pragma unroll
+        for (int c = 1; c < M; ++c) x = (k == c) ? pv[c] : x;
+        rank_bits<S, false>(tab, x, le);
+        rank_bits<S, true>(tab, x, lt);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            bits[j] &= le[j];
+            eq[j] &= le[j] & ~lt[j];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) bits[j] &= ~eq[j];
+}
+
+// One workgroup: chunk qc against the row blocks [pb0, pb1), a row block per
+// wave at a time.  s_tab: LDS for the tables of objectives 1 .. M - 1.  A chunk
+// that ends before block pb with no f0 tie has f0 strictly below pb's, so its
+// words need objectives 1 .. M - 1 only.  rend (optional): each row's end, one
+// past its last non-zero word, raised with atomicMax.
+//
+// Bound: the bitmask's write (n^2 / 16 bytes).  Rows of one wave hit unrelated
+// ranks, so searches and mask reads go to LDS, where a random 16-byte read of a
+// wave costs about 12 cycles.
+template <int M>
+__device__ __forceinline__ void dom_chunk(const float* __restrict__ fs, int npad, int n, int W, int Wc,
+                                          const uint64_t* __restrict__ valid, const int32_t* __restrict__ hi,
+                                          const unsigned char* __restrict__ tables, uint64_t* __restrict__ B,
+                                          int32_t* __restrict__ rend, int qc, int pb0, int pb1, unsigned char* s_tab)
+{
+    constexpr int S = rank_sub(M);
+    constexpr int kTab = rank_table_bytes(S);
+    if (hi[pb1 - 1] < 8 * qc) return;            // hi ascends: no row block here reaches the chunk
+    const unsigned char* tab0 = tables + static_cast<size_t>(qc) * M * kTab;
+    if constexpr (M > 1) {
+        const uint4* src = reinterpret_cast<const uint4*>(tab0 + kTab);
+        uint4* dst = reinterpret_cast<uint4*>(s_tab);
+#pragma unroll 4
+        for (int j = static_cast<int>(threadIdx.x); j < (M - 1) * kTab / 16; j += kDomThreads) dst[j] = src[j];
+        __syncthreads();
+    }
+    const int lane = lane_id();
+    uint64_t vq[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) vq[j] = ld_uniform(valid, static_cast<size_t>(qc) * 8 + j);
+    const int tie_to = ld_uniform(hi, min(8 * qc + 7, W - 1));   // last block that ties with the chunk
+    for (int pb = pb0 + wave_uniform(static_cast<int>(threadIdx.x >> 6)); pb < pb1; pb += kDomWaves) {
+        if (ld_uniform(hi, pb) < 8 * qc) continue;
+        const uint64_t vp = ld_uniform(valid, pb);
+        // rows outside segment 0: feasible ones with a NaN objective have no
+        // dominators, infeasible ones no words that are read
+        const int p = pb * 64 + lane;
+        float pv[M];
+#pragma unroll
+        for (int k = 0; k < M; ++k) pv[k] = fs[static_cast<size_t>(k) * npad + p];
+        const bool in0 = (vp >> lane) & 1ull;
+        uint64_t bits[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) bits[j] = in0 ? vq[j] : 0ull;
+        if (8 * qc + 7 < pb && tie_to < pb) {
+#pragma unroll
+            for (int k = 1; k < M; ++k) {
+                uint64_t le[8];
+                rank_bits<S, false>(s_tab + (k - 1) * kTab, pv[k], le);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) bits[j] &= le[j];
+            }
+        } else {
+            tied_bits<M, S>(tab0, s_tab, pv, bits);
+        }
+        ulonglong2* dst = reinterpret_cast<ulonglong2*>(B + ((static_cast<size_t>(pb) * Wc + qc) * 64 + lane) * 8);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dst[j] = make_ulonglong2(bits[2 * j], bits[2 * j + 1]);
+        if (rend && p < n) {
+            int top = 0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (bits[j]) top = j + 1;
+            if (top) atomicMax(&rend[p], qc * 8 + top);
+        }
+    }
+}
+
+// LDS of the dominance kernel: the tables of objectives 1 .. m - 1.
+constexpr size_t dom_lds_bytes(int m) { return static_cast<size_t>(m > 1 ? m - 1 : 0) * rank_table_bytes(rank_sub(m)); }
+
+// Grid (ceil(W / seg), Wc).
+template <int M>
+__global__ __launch_bounds__(kDomThreads) void nds_dominance(const float* __restrict__ fs, int npad, int n, int W,
+                                                            int Wc, const uint64_t* __restrict__ valid,
+                                                            const int32_t* __restrict__ hi,
+                                                            const unsigned char* __restrict__ tables,
+                                                            uint64_t* __restrict__ B, int32_t* __restrict__ rend,
+                                                            int seg)
+{
+    extern __shared__ __align__(16) unsigned char s_tab[];
+    const int pb0 = static_cast<int>(blockIdx.x) * seg;
+    dom_chunk<M>(fs, npad, n, W, Wc, valid, hi, tables, B, rend, static_cast<int>(blockIdx.y), pb0,
+                 min(pb0 + seg, W), s_tab);
+}
+
+// Row blocks per dominance workgroup: enough workgroups to fill the chip, and
+// enough row blocks in each to pay for loading its tables.
+int dom_segment(int W, int Wc)
+{
+    const long long units = static_cast<long long>(W) * Wc / 2;
+    const long long per = units / 1024 / kDomWaves * kDomWaves;
+    return static_cast<int>(std::max<long long>(kDomWaves, std::min<long long>(64, per)));
 }
 
 // Peel state (device), u32 words: [0, kBarWords) group barrier,
@@ -388,17 +459,15 @@ __global__ __launch_bounds__(kDomThreads) void nds_dominance_wide(
 // in LDS for the whole launch, its blocking word c (the highest word of its
 // dominator row that held an unassigned dominator when last looked at) and
 // rem, the dominators of word c that were still unassigned then.  Round k:
-//   A  rem &= ~A[c] against the set assigned before round k.  A row with rem
-//      left stays blocked without touching HBM.  A row whose rem emptied reads
-//      on below c: kCheckChunks chunks, in one batch (four lanes a row over
-//      all 16 waves when the workgroup owns four row blocks or fewer, else a
-//      lane per row).  Rows whose dominator words run out are front k; rows
-//      still clear with words left go to the workgroup's task queue in LDS as
-//      (row, c).
-//   B  the workgroup's 16 waves scan the queued rows in sweeps of one round
-//      trip per row (as many lanes a row as the queue leaves free), each until
-//      it meets its next blocking word (the row keeps (c, rem)) or runs out of
-//      words (front k).
+//   A  rem &= ~A[c] against the set assigned before round k, a lane per row,
+//      in LDS alone.  A row with rem left stays blocked; the others go to the
+//      workgroup's queue in LDS as (row, c).
+//   B  the workgroup's 16 waves scan the queued rows downwards from c in sweeps
+//      of one round trip per row, each until it meets its next blocking word
+//      (the row keeps (c, rem)) or runs out of words (front k).  The first
+//      sweep reads kFirstLanes chunks a row, which ends most scans; the later
+//      ones as many as the queue leaves lanes for (a wave, 512 words, for 16
+//      rows or fewer), as a row that got past the first mostly runs out.
 // Why downwards: the dominators next to a row in the sort order (f0 just
 // below its own) are on average much deeper than those with a small f0, so the
 // blocker found first stays unassigned for most of the rounds before the row's
@@ -429,6 +498,8 @@ struct PeelArgs {
     const int32_t* rend;     // (n,) optional: one past each row's last non-zero word (sorted order)
     uint32_t spin_limit;     // polls before a barrier wait gives up
     uint32_t* error;         // optional sticky flag: set to 1 when a bounded wait gave up
+    const uint64_t* gmask;   // (W,) first rows of each distinct infeasible cv (infeasible_info)
+    const int32_t* info;     // feasible rows, end of the infeasible rows whose cv is a number
 };
 
 constexpr int32_t kPeelFailed = -2;
@@ -437,126 +508,66 @@ constexpr int kPeelStateWords = kBarWords + 16;
 static_assert(kPeelStateWords <= kBatchPeelStateWords, "batched peel state too small");
 constexpr int kPeelThreads = 1024;
 constexpr int kPeelWaves = kPeelThreads / 64;
-constexpr int kCheckChunks = 2;     // phase A: chunks read in one batch from the cursor's chunk
-constexpr int kScanLoads = 8;       // phase B: words per lane in flight (8 per lane of a row)
-constexpr int kMinLanes = 8;        // phase B: fewest lanes per row (64 words a trip)
+constexpr int kFirstLanes = 4;      // lanes (chunks) per row of the first sweep
+constexpr int kMinLanes = 8;        // and of the later ones, at least
 
-// LDS layout of the peel (dynamic): s_A (W u64), s_next (bpg u64), s_task
-// (2 x 64 bpg u64), s_rem (64 bpg u64), s_cur and s_front (64 bpg int each).
+// LDS layout of the peel (dynamic): s_A (W u64), s_next (bpg u64), s_rem
+// (64 bpg u64), s_task (2 x 64 bpg rows and cursors), s_cur and s_front (64 bpg
+// int each).
 __host__ __device__ __forceinline__ size_t peel_lds_bytes(int W, int bpg)
 {
     const size_t rows = static_cast<size_t>(bpg) * 64;
-    return static_cast<size_t>(W) * 8 + static_cast<size_t>(bpg) * 8 + rows * 32;
+    return (static_cast<size_t>(W) + 7) / 8 * 64 + static_cast<size_t>(bpg) * 8 + rows * 32;
 }
 
-__device__ __forceinline__ uint64_t chunk_word(const ulonglong2 (&v)[4], int i)
-{
-    const ulonglong2 h = v[i >> 1];
-    return (i & 1) ? h.y : h.x;
-}
-
-__device__ __forceinline__ const uint64_t* peel_rowbase(const uint64_t* __restrict__ B, int Wc, int rb, int lane)
-{
-    return B + (static_cast<size_t>(rb) * Wc * 64 + lane) * 8;
-}
-
-__device__ __forceinline__ void peel_load_chunk(const uint64_t* rowbase, int c, ulonglong2 (&v)[4])
-{
-    const ulonglong2* src = reinterpret_cast<const ulonglong2*>(rowbase + static_cast<size_t>(c) * 512);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = src[i];
-}
-
-// Phase A read for the lane's row (live, rem emptied): the kCheckChunks
-// chunks that hold the words below cur, from the one holding word cur - 1
-// down, loaded in one batch (one HBM round trip).  cur >= 1 on entry.
-// ready: no dominator word left; queued: clear so far with words left below
-// the returned cur; otherwise blocked at the returned cur with the unassigned
-// dominators of that word in rem.
-__device__ __forceinline__ void peel_check(const uint64_t* __restrict__ B, int Wc, int rb, int lane,
-                                           const uint64_t* s_A, int& cur, bool& ready, bool& queued, uint64_t& rem)
-{
-    const uint64_t* rowbase = peel_rowbase(B, Wc, rb, lane);
-    const int c = (cur - 1) >> 3;
-    ulonglong2 v[kCheckChunks][4];
-#pragma unroll
-    for (int a = 0; a < kCheckChunks; ++a)
-        if (c - a >= 0) peel_load_chunk(rowbase, c - a, v[a]);
-    // the assigned-set words of the same span, read while the row's words
-    // are in flight (indices clamped to words below cur)
-    uint64_t am[kCheckChunks * 8];
-#pragma unroll
-    for (int a = 0; a < kCheckChunks; ++a)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) am[a * 8 + i] = s_A[max(min((c - a) * 8 + i, cur - 1), 0)];
-    const int stop = max((c - kCheckChunks + 1) * 8, 0);
-    int blocked = -1;
-#pragma unroll
-    for (int a = kCheckChunks - 1; a >= 0; --a) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int ww = (c - a) * 8 + i;
-            const uint64_t x = chunk_word(v[a], i) & ~am[a * 8 + i];
-            if (ww >= 0 && ww < cur && x != 0) { blocked = ww; rem = x; }
-        }
-    }
-    cur = blocked >= 0 ? blocked : stop;
-    ready = blocked < 0 && stop == 0;
-    queued = blocked < 0 && !ready;
-}
-
-// Phase B, one trip: groups of L lanes (L = 8, 16, 32 or 64) of a wave, one
-// queued row each.  Lane sl of group gi reads words top - iL - sl
-// (i < kScanLoads, top the last word of the chunk holding c - 1) of its row:
-// 8L words a trip, each 8-word run one 64-byte segment; words from c on or
-// below 0 count as clear.  Returns true when the row meets a word holding an
-// unassigned dominator (its index in c, its unassigned bits in rem, the same
-// in every lane of the group); otherwise c moves below the words read (to 0
-// when they run out).  Every lane of the wave calls it; lanes of a group
-// without a row pass has = false.
-__device__ __forceinline__ bool peel_trip(const uint64_t* __restrict__ B, int Wc, int W, int pr, int& c,
+// One trip: groups of L lanes (a power of two) of a wave, one queued row each.
+// Lane sl of a row's group reads chunk (c - 1) / 8 - sl of the row, a 64-byte
+// segment; words from c on count as clear.  Returns true when the row meets a
+// word holding an unassigned dominator (its index in c, its unassigned bits in
+// rem, the same in every lane of the group); otherwise c moves below the words
+// read (to 0 when they run out).  Every lane of the wave calls it; lanes of a
+// group without a row pass has = false.  c >= 1 for a row.
+__device__ __forceinline__ bool peel_trip(const uint64_t* __restrict__ B, int Wc, int p, int& c,
                                           const uint64_t* s_A, int lane, int L, bool has, uint64_t& rem)
 {
     const int sl = lane & (L - 1);
     const int shift = lane - sl;
-    const uint64_t gmask = (L == 64) ? ~0ull : ((1ull << L) - 1);
-    const int top = (c - 1) | 7;
-    uint64_t x[kScanLoads];
+    const int ch0 = (c - 1) >> 3;
+    const int ch = ch0 - sl;
+    const bool in = has && ch >= 0;
+    ulonglong2 v[4];
+    if (in) {
+        const ulonglong2* src = reinterpret_cast<const ulonglong2*>(B + bword_index(p, ch * 8, Wc));
 #pragma unroll
-    for (int i = 0; i < kScanLoads; ++i) {
-        const int w = top - i * L - sl;
-        x[i] = (has && w >= 0 && w < c) ? B[bword_index(pr, w, Wc)] : 0ull;
+        for (int i = 0; i < 4; ++i) v[i] = src[i];
     }
     // the assigned-set words, read while the row's words are in flight
-    uint64_t am[kScanLoads];
+    const int w0 = in ? ch * 8 : 0;
+    uint64_t am[8];
 #pragma unroll
-    for (int i = 0; i < kScanLoads; ++i) am[i] = s_A[min(max(top - i * L - sl, 0), W - 1)];
-#pragma unroll
-    for (int i = 0; i < kScanLoads; ++i) {
-        const int w = top - i * L - sl;
-        x[i] = (has && w >= 0 && w < c) ? (x[i] & ~am[i]) : 0ull;
-    }
-    // first blocking word of this lane's group: the lowest (i, sl)
-    int first = -1;
+    for (int i = 0; i < 8; ++i) am[i] = s_A[w0 + i];
+    int fw = -1;
     uint64_t hit = 0;
+    if (in) {
 #pragma unroll
-    for (int i = kScanLoads - 1; i >= 0; --i) {
-        const uint64_t gm = (ballot(x[i] != 0) >> shift) & gmask;
-        if (gm) {
-            first = i * L + __builtin_ctzll(gm);
-            hit = x[i];
+        for (int i = 0; i < 8; ++i) {
+            const uint64_t x = ((i & 1) ? v[i >> 1].y : v[i >> 1].x) & ~am[i];
+            if (w0 + i < c && x != 0) { fw = w0 + i; hit = x; }
         }
     }
-    // the blocking word's bits, from the lane that read it
-    const int src = shift + (first & (L - 1));
+    // the row's highest blocking word: from its lowest lane that has one
+    const uint64_t gmask = (L == 64) ? ~0ull : ((1ull << L) - 1);
+    const uint64_t gm = (ballot(fw >= 0) >> shift) & gmask;
+    const int src = shift + (gm ? __builtin_ctzll(gm) : 0);
+    const int bw = __shfl(fw, src);
     const uint32_t lo = static_cast<uint32_t>(__shfl(static_cast<int>(hit), src));
     const uint32_t hi = static_cast<uint32_t>(__shfl(static_cast<int>(hit >> 32), src));
-    if (first >= 0) {
-        c = top - first;
+    if (gm) {
+        c = bw;
         rem = (static_cast<uint64_t>(hi) << 32) | lo;
         return true;
     }
-    c = max(top + 1 - kScanLoads * L, 0);
+    c = max((ch0 + 1 - L) * 8, 0);
     return false;
 }
 
@@ -569,6 +580,80 @@ __device__ __forceinline__ void peel_fail(const PeelArgs& P)
     if (P.error) __hip_atomic_fetch_or(P.error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// The end of the peel, once the feasible rows' fronts (0 .. F - 1) are known or
+// the stop rule has ended them: with `tail`, the infeasible rows get front
+// F + (index of their distinct cv) as long as fewer than stop_at rows are
+// assigned before (at least one front when no row is feasible), rows with a
+// NaN cv front F.  Every owned row's front goes out in input order; block 0
+// of the group leaves the last front.  s_A (free by now) takes the prefix
+// counts of the first rows.
+__device__ __forceinline__ void peel_finish(const PeelArgs& P, int g, int G, int nf, int ne, int last_front,
+                                            bool tail, const int* s_front, uint64_t* s_A)
+{
+    const int lane = lane_id();
+    const int lw = wave_uniform(static_cast<int>(threadIdx.x >> 6));
+    int cut = nf;                 // first infeasible row that is not assigned
+    int* s_start = reinterpret_cast<int*>(s_A);   // (W) first rows before each block
+    __shared__ int s_cut, s_base[kPeelWaves], s_run;
+    if (tail) {
+        // the first group that begins at or after `from` finds enough rows assigned
+        const int from = max(nf + 1, P.stop_at - (P.n - ne));
+        if (threadIdx.x == 0) { s_cut = ne; s_run = 0; }
+        __syncthreads();
+        for (int w0 = 0; w0 < P.W; w0 += kPeelThreads) {
+            const int w = w0 + static_cast<int>(threadIdx.x);
+            const uint64_t m = w < P.W ? P.gmask[w] : 0ull;
+            uint64_t late = m;
+            if (w * 64 < from) late = (from - w * 64 >= 64) ? 0ull : m & (~0ull << (from - w * 64));
+            if (late) atomicMin(&s_cut, w * 64 + __builtin_ctzll(late));
+            // prefix of the counts over the block's words
+            const int cnt = __builtin_popcountll(m);
+            int incl = cnt;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int u = __shfl_up(incl, o);
+                if (lane >= o) incl += u;
+            }
+            if (lane == 63) s_base[lw] = incl;
+            __syncthreads();
+            int before = s_run;
+            for (int v = 0; v < lw; ++v) before += s_base[v];
+            if (w < P.W) s_start[w] = before + incl - cnt;
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                int all = s_run;
+                for (int v = 0; v < kPeelWaves; ++v) all += s_base[v];
+                s_run = all;
+            }
+            __syncthreads();
+        }
+        cut = s_cut;
+    }
+    const auto groups_to = [&](int t) {           // first rows at sorted positions <= t
+        const uint64_t m = P.gmask[t >> 6];
+        const int b = t & 63;
+        return s_start[t >> 6] + __builtin_popcountll(m & (b == 63 ? ~0ull : (1ull << (b + 1)) - 1));
+    };
+    if (g == 0 && threadIdx.x == 0) {
+        int last = last_front;
+        if (tail && ne > nf) last += groups_to(cut - 1);
+        else if (tail && P.n > ne) last += 1;
+        // the launch before the peel set the output to -1; a block that gave
+        // up in this last barrier may already have marked the run failed, and
+        // that mark stays
+        int32_t expected = -1;
+        __hip_atomic_compare_exchange_strong(P.out_max_front, &expected, last, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+    }
+    for (int j = lw; j < P.blocks_per_group; j += kPeelWaves) {
+        const int p = (g + j * G) * 64 + lane;
+        if (p >= P.n) continue;
+        int fr = s_front[j * 64 + lane];
+        if (tail && p >= nf) fr = p >= ne ? last_front + 1 : p < cut ? last_front + groups_to(p) : -1;
+        P.fronts[P.perm[p]] = fr;
+    }
+}
+
 // One peel over the G blocks of a group; g is this block's rank.  Returns
 // false when a barrier gave up (the launch is broken; the block exits after
 // recording the failure).
@@ -576,18 +661,19 @@ __device__ __forceinline__ bool peel_body(const PeelArgs& P, int g, int G, uint6
 {
     const int nblk = P.W;
     const int bpg = P.blocks_per_group;
-    uint64_t* s_A = s_dyn;                                          // (W) assigned before this round
-    uint64_t* s_next = s_A + nblk;                                  // (bpg) rows of own blocks assigned this round
+    uint64_t* s_A = s_dyn;                                          // (W) assigned before this round, whole chunks
+    uint64_t* s_next = s_A + (nblk + 7) / 8 * 8;                    // (bpg) rows of own blocks assigned this round
     const int rows = bpg * 64;
-    uint64_t* s_task = s_next + bpg;                                // (2 x 64 bpg) queued (cursor << 32 | row)
-    uint64_t* s_rem = s_task + 2 * static_cast<size_t>(rows);       // (64 bpg) unassigned bits of the blocking word
-    int* s_cur = reinterpret_cast<int*>(s_rem + rows);              // (64 bpg) blocking word
+    uint64_t* s_rem = s_next + bpg;                                 // (64 bpg) unassigned bits of the blocking word
+    int2* s_task = reinterpret_cast<int2*>(s_rem + rows);           // (2 x 64 bpg) queued (row, cursor)
+    int* s_cur = reinterpret_cast<int*>(s_task + 2 * static_cast<size_t>(rows));   // (64 bpg) blocking word
     int* s_front = s_cur + rows;                                    // (64 bpg) front of each owned row
     __shared__ int s_nq[3];         // queue lengths, rotating over the sweeps of phase B
     __shared__ int s_count;
     const int lane = lane_id();
     const int lw = wave_uniform(static_cast<int>(threadIdx.x >> 6));
     uint32_t phase = 0;
+    const int nf = P.info[kInfoFeasible], ne = P.info[kInfoOrdered];
 
     for (int j = lw; j < bpg; j += kPeelWaves) {
         const int rb = g + j * G;
@@ -601,6 +687,10 @@ __device__ __forceinline__ bool peel_body(const PeelArgs& P, int g, int G, uint6
         if (lane == 0) { st_relaxed_u64(&P.A0[rb], 0ull); st_relaxed_u64(&P.A1[rb], 0ull); }
     }
     if (!coherent_barrier(P.state, g, G, phase, P.spin_limit)) { peel_fail(P); return false; }
+    if (nf == 0) {
+        peel_finish(P, g, G, nf, ne, -1, true, s_front, s_A);
+        return true;
+    }
 
     int total_prev = 0;
     for (int k = 0;; ++k) {
@@ -610,187 +700,81 @@ __device__ __forceinline__ bool peel_body(const PeelArgs& P, int g, int G, uint6
         if (threadIdx.x == 0) { s_count = 0; s_nq[0] = 0; s_nq[1] = 0; }
         __syncthreads();
 
-        // ---- phase A
+        // ---- phase A: lane per row, in LDS
         int my_new = 0;
-        if (bpg * 4 <= kPeelWaves) {
-            // four lanes a row: wave lw takes rows 16 (lw & 3) .. 16 (lw & 3) + 15
-            // of row block lw / 4, and lane q = lane & 3 of a row reads words
-            // 4q .. 4q + 3 of the two chunks from the one holding its cursor
-            const int j = lw >> 2;
+        for (int j = lw; j < bpg; j += kPeelWaves) {
             const int rb = g + j * G;
-            if (j < bpg && rb < nblk) {
-                const int q = lane & 3;
-                const int r = (lw & 3) * 16 + (lane >> 2);
-                const uint64_t amask = s_A[rb];
-                const int p = rb * 64 + r;
-                const int slot = j * 64 + r;
-                const bool live = (p < P.n) && !((amask >> r) & 1ull);
-                int cur = 0;
-                bool ready = false, queued = false, check = false;
-                uint64_t rem = 0;
-                if (live) {
-                    cur = s_cur[slot];
-                    // still blocked while dominators of its blocking word are
-                    // unassigned (before its first check rem is 0 and cur may be W)
-                    rem = s_rem[slot] & ~s_A[min(cur, P.W - 1)];
-                    ready = (rem == 0) && cur == 0;
-                    check = (rem == 0) && !ready;
-                }
-                if (ballot(check)) {
-                    const int c = (cur - 1) >> 3;
-                    const int cc = c - (q >> 1);
-                    const int w0 = cc * 8 + 4 - (q & 1) * 4;
-                    ulonglong2 v0 = make_ulonglong2(0ull, 0ull), v1 = v0;
-                    if (check && cc >= 0) {
-                        const ulonglong2* src = reinterpret_cast<const ulonglong2*>(
-                            peel_rowbase(P.B, P.Wc, rb, r) + static_cast<size_t>(cc) * 512 + 4 - (q & 1) * 4);
-                        v0 = src[0];
-                        v1 = src[1];
-                    }
-                    // the assigned-set words, read while the row's words are in flight
-                    uint64_t am[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) am[i] = s_A[min(max(w0 + i, 0), P.W - 1)];
-                    const int stop = max((c - kCheckChunks + 1) * 8, 0);
-                    const uint64_t wv[4] = {v0.x, v0.y, v1.x, v1.y};
-                    int fw = -1;
-                    uint64_t fx = 0;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int w = w0 + i;
-                        const uint64_t x = wv[i] & ~am[i];
-                        if (check && w >= 0 && w < cur && x != 0) { fw = w; fx = x; }
-                    }
-                    // the row's highest blocking word: from its lowest lane that has one
-                    const uint32_t gm = static_cast<uint32_t>(ballot(fw >= 0) >> (lane & ~3)) & 0xFu;
-                    const int src = (lane & ~3) + (gm ? __builtin_ctz(gm) : 0);
-                    const int bw = __shfl(fw, src);
-                    const uint32_t lo = static_cast<uint32_t>(__shfl(static_cast<int>(fx), src));
-                    const uint32_t hi = static_cast<uint32_t>(__shfl(static_cast<int>(fx >> 32), src));
-                    if (check) {
-                        if (gm) {
-                            cur = bw;
-                            rem = (static_cast<uint64_t>(hi) << 32) | lo;
-                        } else {
-                            cur = stop;
-                            ready = (stop == 0);
-                            queued = !ready;
-                        }
-                    }
-                }
-                const bool lead = (q == 0);
-                if (live && !ready && lead) {
-                    s_cur[slot] = cur;
-                    s_rem[slot] = rem;
-                }
-                const uint64_t ready_m = ballot(ready && lead);
-                const uint64_t task_m = ballot(queued && lead);
-                if (ready && lead) s_front[slot] = k;
-                if (task_m) {
-                    int base = 0;
-                    if (lane == 0) base = atomicAdd(&s_nq[0], __builtin_popcountll(task_m));
-                    base = __builtin_amdgcn_readfirstlane(base);
-                    if (queued && lead) {
-                        const int below = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
-                            static_cast<uint32_t>(task_m >> 32),
-                            __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(task_m), 0u)));
-                        s_task[base + below] = (static_cast<uint64_t>(cur) << 32) | static_cast<uint32_t>(p);
-                    }
-                }
-                if (ready_m) {
-                    // the rows' bits sit at lanes 0, 4, ..., 60: bits 0 .. 15 of the wave's rows
-                    uint64_t rbits = 0;
-#pragma unroll
-                    for (int t = 0; t < 16; ++t) rbits |= ((ready_m >> (4 * t)) & 1ull) << t;
-                    if (lane == 0) {
-                        atomicOr(reinterpret_cast<unsigned long long*>(&s_next[j]),
-                                 static_cast<unsigned long long>(rbits << ((lw & 3) * 16)));
-                        my_new += __builtin_popcountll(rbits);
-                    }
+            if (rb >= nblk) break;
+            const uint64_t amask = s_A[rb];
+            const int p = rb * 64 + lane;
+            const int slot = j * 64 + lane;
+            const bool live = (p < nf) && !((amask >> lane) & 1ull);
+            bool ready = false, queued = false;
+            int cur = 0;
+            if (live) {
+                cur = s_cur[slot];
+                // still blocked while dominators of its blocking word are
+                // unassigned (before its first scan rem is 0 and cur may be W)
+                const uint64_t rem = s_rem[slot] & ~s_A[min(cur, nblk - 1)];
+                s_rem[slot] = rem;
+                ready = (rem == 0) && cur == 0;
+                queued = (rem == 0) && !ready;
+            }
+            if (ready) s_front[slot] = k;
+            const uint64_t ready_m = ballot(ready);
+            const uint64_t task_m = ballot(queued);
+            if (task_m) {
+                int base = 0;
+                if (lane == 0) base = atomicAdd(&s_nq[0], __builtin_popcountll(task_m));
+                base = __builtin_amdgcn_readfirstlane(base);
+                if (queued) {
+                    const int below = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                        static_cast<uint32_t>(task_m >> 32),
+                        __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(task_m), 0u)));
+                    s_task[base + below] = make_int2(slot, cur);
                 }
             }
-        } else {
-            // lane per row
-            for (int j = lw; j < bpg; j += kPeelWaves) {
-                const int rb = g + j * G;
-                if (rb >= nblk) break;
-                const uint64_t amask = s_A[rb];
-                const int p = rb * 64 + lane;
-                const int slot = j * 64 + lane;
-                const bool live = (p < P.n) && !((amask >> lane) & 1ull);
-                int cur = 0;
-                bool ready = false, queued = false;
-                if (live) {
-                    cur = s_cur[slot];
-                    // still blocked while dominators of its blocking word are
-                    // unassigned (before its first check rem is 0 and cur may be W)
-                    uint64_t rem = s_rem[slot] & ~s_A[min(cur, P.W - 1)];
-                    if (rem == 0) {
-                        if (cur == 0) ready = true;
-                        else peel_check(P.B, P.Wc, rb, lane, s_A, cur, ready, queued, rem);
-                        s_cur[slot] = cur;
-                    }
-                    s_rem[slot] = rem;
-                }
-                const uint64_t ready_m = ballot(ready);
-                const uint64_t task_m = ballot(queued);
-                if (ready) s_front[slot] = k;
-                if (task_m) {
-                    int base = 0;
-                    if (lane == 0) base = atomicAdd(&s_nq[0], __builtin_popcountll(task_m));
-                    base = __builtin_amdgcn_readfirstlane(base);
-                    if (queued) {
-                        const int below = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
-                            static_cast<uint32_t>(task_m >> 32),
-                            __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(task_m), 0u)));
-                        s_task[base + below] = (static_cast<uint64_t>(cur) << 32) | static_cast<uint32_t>(p);
-                    }
-                }
-                if (lane == 0) {
-                    s_next[j] = ready_m;
-                    my_new += __builtin_popcountll(ready_m);
-                }
+            if (lane == 0) {
+                s_next[j] = ready_m;
+                my_new += __builtin_popcountll(ready_m);
             }
         }
 
-        // ---- phase B: the queued rows, in sweeps of one trip per row, each
-        // row until it blocks or runs out of words.  Sweep s takes queue s % 2
-        // (length s_nq[s % 3]) and queues the rows still clear in the other.
-        // A row gets as many lanes as the queue leaves free (a wave for 16
-        // rows or fewer, 8 lanes for more than 64): a queued row mostly runs
-        // out of words, so what it reads at once it needs.
+        // ---- phase B: sweep s takes queue s % 2 (length s_nq[s % 3]) and
+        // queues the rows still clear in the other
         for (int sw = 0;; ++sw) {
             __syncthreads();
             const int nq = s_nq[sw % 3];
             if (nq == 0) break;
             if (threadIdx.x == 0) s_nq[(sw + 2) % 3] = 0;
-            int L = 64;
-            while (L > kMinLanes && nq > kPeelWaves * (64 / L)) L >>= 1;
+            int L = kFirstLanes;
+            if (sw > 0) {
+                L = 64;
+                while (L > kMinLanes && nq > kPeelWaves * (64 / L)) L >>= 1;
+            }
             const int gpw = 64 / L;
-            const uint64_t* q_in = s_task + (sw & 1) * static_cast<size_t>(rows);
-            uint64_t* q_out = s_task + ((sw + 1) & 1) * static_cast<size_t>(rows);
+            const int2* q_in = s_task + (sw & 1) * static_cast<size_t>(rows);
+            int2* q_out = s_task + ((sw + 1) & 1) * static_cast<size_t>(rows);
             for (int t0 = lw * gpw; t0 < nq; t0 += kPeelWaves * gpw) {
                 const int t = t0 + lane / L;
                 const bool has = t < nq;
-                const uint64_t rec = has ? q_in[t] : 0ull;
-                const int pr = static_cast<int>(static_cast<uint32_t>(rec));
-                const int rb = pr >> 6;
-                const int slot = ((rb - g) / G) * 64 + (pr & 63);
-                int c = static_cast<int>(rec >> 32);
+                const int2 rec = has ? q_in[t] : make_int2(0, 1);
+                const int slot = rec.x;
+                int c = rec.y;
+                const int p = (g + (slot >> 6) * G) * 64 + (slot & 63);
                 uint64_t rem = 0;
-                const bool blocked = peel_trip(P.B, P.Wc, P.W, pr, c, s_A, lane, L, has, rem);
+                const bool blocked = peel_trip(P.B, P.Wc, p, c, s_A, lane, L, has, rem);
                 if (has && (lane & (L - 1)) == 0) {
                     if (blocked) {
                         s_cur[slot] = c;
                         s_rem[slot] = rem;
                     } else if (c == 0) {
                         s_front[slot] = k;
-                        atomicOr(reinterpret_cast<unsigned long long*>(&s_next[(rb - g) / G]),
-                                 static_cast<unsigned long long>(1ull << (pr & 63)));
+                        atomicOr(reinterpret_cast<unsigned long long*>(&s_next[slot >> 6]),
+                                 static_cast<unsigned long long>(1ull << (slot & 63)));
                         ++my_new;
                     } else {
-                        q_out[atomicAdd(&s_nq[(sw + 1) % 3], 1)] =
-                            (static_cast<uint64_t>(c) << 32) | static_cast<uint32_t>(pr);
+                        q_out[atomicAdd(&s_nq[(sw + 1) % 3], 1)] = make_int2(slot, c);
                     }
                 }
             }
@@ -812,21 +796,10 @@ __device__ __forceinline__ bool peel_body(const PeelArgs& P, int g, int G, uint6
         const int snap = kPeelTotal + 4 + (k & 1);
         if (!coherent_barrier(P.state, g, G, phase, P.spin_limit, kPeelTotal, snap)) { peel_fail(P); return false; }
         const int total = static_cast<int>(ld_relaxed_u32(&P.state[snap]));
-        if (total >= P.stop_at || total == total_prev || total >= P.n) {
-            if (g == 0 && threadIdx.x == 0) {
-                // the launch before the peel set the output to -1; a block
-                // that gave up in this last barrier may already have marked
-                // the run failed, and that mark stays
-                int32_t expected = -1;
-                __hip_atomic_compare_exchange_strong(P.out_max_front, &expected,
-                                                     (total == total_prev) ? k - 1 : k, __ATOMIC_RELAXED,
-                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            // the owned rows' fronts (-1: not assigned), in input order
-            for (int j = lw; j < bpg; j += kPeelWaves) {
-                const int p = (g + j * G) * 64 + lane;
-                if (p < P.n) P.fronts[P.perm[p]] = s_front[j * 64 + lane];
-            }
+        if (total >= P.stop_at || total == total_prev || total >= nf) {
+            // the infeasible rows follow once every feasible one is assigned
+            peel_finish(P, g, G, nf, ne, (total == total_prev) ? k - 1 : k, total >= nf && total < P.stop_at, s_front,
+                        s_A);
             return true;
         }
         total_prev = total;
@@ -875,54 +848,39 @@ __global__ void b_nds_keys(const BInst* __restrict__ insts, BMap mp, int mode, u
     vals[R.key_off + s] = s;
 }
 
-__global__ void b_nds_gather(const BInst* __restrict__ insts, BMap mp, int mode,
-                             const int32_t* __restrict__ vals_sorted)
+// nds_prep of every instance: Wc x m workgroups each.
+__global__ __launch_bounds__(kChunk) void b_nds_prep(const BInst* __restrict__ insts, BMap mp, int mode,
+                                                     const uint64_t* __restrict__ keys_sorted,
+                                                     const int32_t* __restrict__ vals_sorted)
 {
     int local;
     const int i = bmap_find(mp, static_cast<int>(blockIdx.x), local);
     const BInst& I = insts[i];
     const BRows R = brows(I, mode);
-    const int npad = ((R.rows + 63) / 64) * 64;
-    const int t = local * 256 + static_cast<int>(threadIdx.x);
-    if (t >= npad) return;
-    if (t < R.rows) {
-        const int s = vals_sorted[R.key_off + t];
-        I.perm[t] = s;
-        for (int k = 0; k < I.m; ++k)
-            I.fs[static_cast<size_t>(k) * npad + t] = R.f[static_cast<size_t>(k) * R.rows + s];
-        I.cvs[t] = R.cv[s];
-    } else {
-        for (int k = 0; k < I.m; ++k) I.fs[static_cast<size_t>(k) * npad + t] = 0.0f;
-        I.cvs[t] = 0.0f;
-    }
+    const int W = (R.rows + 63) / 64;
+    const int qc = local / I.m, k = local % I.m;
+    const int t = qc * kChunk + static_cast<int>(threadIdx.x);
+    const int32_t* perm = vals_sorted + R.key_off;
+    if (k == 0 && t < R.rows) I.perm[t] = perm[t];
+    const PrepOut O{I.fs, I.valid, I.hi, I.gmask, I.ninfo, I.m >= kRowEndMinM ? I.rend : nullptr, I.tables};
+    if (rank_sub(I.m) == 256) prep_chunk<256>(R.f, R.rows, R.rows, I.m, W * 64, perm, keys_sorted + R.key_off, qc, k, O);
+    else prep_chunk<128>(R.f, R.rows, R.rows, I.m, W * 64, perm, keys_sorted + R.key_off, qc, k, O);
 }
 
-__global__ void b_nds_block_info(const BInst* __restrict__ insts, BMap mp, int mode,
-                                 const uint64_t* __restrict__ keys_sorted)
-{
-    int local;
-    const int i = bmap_find(mp, static_cast<int>(blockIdx.x), local);
-    const BInst& I = insts[i];
-    const BRows R = brows(I, mode);
-    block_info_one(keys_sorted + R.key_off, R.rows, local, I.kind, I.hi);
-    // row ends start at 0; the dominance kernel raises them (four or more objectives)
-    const int row = local * 64 + static_cast<int>(threadIdx.x);
-    if (I.m >= kRowEndMinM && row < R.rows) I.rend[row] = 0;
-}
-
+// nds_dominance of the instances with M objectives: Wc x ceil(W / kBatchDomSeg)
+// workgroups each.
 template <int M>
-__global__ __launch_bounds__(kDomThreads) void b_nds_dominance(const BInst* __restrict__ insts, BMap mp,
-                                                              int mode)
+__global__ __launch_bounds__(kDomThreads) void b_nds_dominance(const BInst* __restrict__ insts, BMap mp, int mode)
 {
+    extern __shared__ __align__(16) unsigned char s_tab[];
     int local;
     const int i = bmap_find(mp, static_cast<int>(blockIdx.x), local);
     const BInst& I = insts[i];
     const BRows R = brows(I, mode);
     const int W = (R.rows + 63) / 64, Wc = (W + 7) / 8;
-    const long long units = 4ll * Wc * (Wc + 1);
-    const long long u = static_cast<long long>(local) * kDomWaves + wave_uniform(static_cast<int>(threadIdx.x >> 6));
-    if (u >= units) return;
-    dom_unit<M>(I.fs, I.cvs, W * 64, R.rows, W, Wc, I.kind, I.hi, I.B, u, M >= kRowEndMinM ? I.rend : nullptr);
+    const int qc = local % Wc, pb0 = local / Wc * kBatchDomSeg;
+    dom_chunk<M>(I.fs, W * 64, R.rows, W, Wc, I.valid, I.hi, I.tables, I.B, M >= kRowEndMinM ? I.rend : nullptr, qc,
+                 pb0, min(pb0 + kBatchDomSeg, W), s_tab);
 }
 
 // Where a batched peel leaves the index of its last front: the selection's
@@ -952,7 +910,7 @@ __global__ __launch_bounds__(kPeelThreads) void b_nds_peel_groups(const BInst* _
         const int W = (R.rows + 63) / 64, Wc = (W + 7) / 8;
         PeelArgs P{I.B, I.hi, I.perm, R.rows, W, Wc, mode == 1 ? I.n : R.rows, (W + G - 1) / G, R.fronts,
                    I.A, I.A + W, I.pstate, peel_max_front(I, mode), I.m >= kRowEndMinM ? I.rend : nullptr,
-                   spin_limit, error};
+                   spin_limit, error, I.gmask, I.ninfo};
         __syncthreads();
         if (!peel_body(P, g, G, s_dyn)) return;
     }
@@ -971,7 +929,6 @@ __global__ void b_peel_reset(const BInst* __restrict__ insts, int mode, int stat
 
 
 constexpr int kMaxWords = 4096;   // n <= 262144: the assigned set fits in 32 KiB of LDS
-constexpr int kWideBlocks = 64;   // row blocks (n >= 4033) from which dominance uses nds_dominance_wide
 
 // Polls before a peel barrier gives up (kSpinLimit unless a test lowers it
 // with moea_debug_set_spin_limit to make the bounded wait give up on purpose).
@@ -988,13 +945,15 @@ struct NdsLayout {
     void* sort_temp;
     size_t sort_bytes;
     float* fs;
-    float* cvs;
+    unsigned char* tables;
     int32_t* hi;
-    uint8_t* kind;
+    uint64_t* valid;
     uint64_t* A0;
     uint64_t* A1;
     uint32_t* state;
     int32_t* rend;
+    uint64_t* gmask;
+    int32_t* info;
 };
 
 size_t carve_nds(void* ws, int n, NdsLayout& L)
@@ -1011,13 +970,15 @@ size_t carve_nds(void* ws, int n, NdsLayout& L)
     L.sort_bytes = sort_pairs_temp_bytes(n, kKeyBits);
     L.sort_temp = c.take_bytes(L.sort_bytes);
     L.fs = c.take<float>(static_cast<size_t>(kMaxM) * npad);
-    L.cvs = c.take<float>(npad);
+    L.tables = c.take<unsigned char>(static_cast<size_t>(Wc) * kRankChunkBytes);
     L.hi = c.take<int32_t>(W);
-    L.kind = c.take<uint8_t>(W);
+    L.valid = c.take<uint64_t>(static_cast<size_t>(Wc) * 8);
     L.A0 = c.take<uint64_t>(W);
     L.A1 = c.take<uint64_t>(W);
     L.state = c.take<uint32_t>(kPeelStateWords);
     L.rend = c.take<int32_t>(npad);
+    L.gmask = c.take<uint64_t>(W);
+    L.info = c.take<int32_t>(2);
     return c.used;
 }
 
@@ -1045,6 +1006,12 @@ int peel_grid_size(int nblk)
 }
 
 }  // namespace
+
+// Rank-table bytes of one instance with nm rows and m objectives.
+size_t nds_table_bytes(int nm, int m)
+{
+    return static_cast<size_t>(ceil_div(nm, kChunk)) * m * rank_table_bytes(rank_sub(m));
+}
 
 size_t nds_workspace_bytes(int n)
 {
@@ -1087,23 +1054,23 @@ int nds_run(const float* f, int ldf, const float* cv, int n, int m, int stop_at,
     // row ends pay for their atomics when many rows have no dominator near
     // their own block, which is the case for many objectives
     int32_t* rend = m >= kRowEndMinM ? L.rend : nullptr;
+    const PrepOut O{L.fs, L.valid, L.hi, L.gmask, L.info, rend, L.tables};
+    const dim3 pgrid(Wc, m), pblock(kChunk);
     // also clears the peel's barrier state (not read before the peel)
-    hipLaunchKernelGGL(nds_block_prep, dim3(W), dim3(64), 0, stream, f, ldf, cv, m, npad, L.perm, L.fs, L.cvs,
-                       L.keys_out, n, L.kind, L.hi, L.state, kPeelStateWords, max_front, rend);
+    if (rank_sub(m) == 256)
+        hipLaunchKernelGGL(nds_prep<256>, pgrid, pblock, 0, stream, f, ldf, n, m, npad, L.perm, L.keys_out, O, L.state,
+                           kPeelStateWords, max_front);
+    else
+        hipLaunchKernelGGL(nds_prep<128>, pgrid, pblock, 0, stream, f, ldf, n, m, npad, L.perm, L.keys_out, O, L.state,
+                           kPeelStateWords, max_front);
     MOEA_HIP(hipGetLastError());
     stage_end(kStNdsSort, stream);
 
     stage_begin(kStDominance, stream);
-    const long long units = 4ll * Wc * (Wc + 1);
-    const dim3 dgrid(static_cast<unsigned>((units + kDomWaves - 1) / kDomWaves));
-    const dim3 dblock(kDomThreads);
-    if (W >= kWideBlocks) {
-        MOEA_LAUNCH_M(m, nds_dominance_wide, dgrid, dblock, 0, stream, L.fs, L.cvs, npad, n, W, Wc, L.kind,
-                      L.hi, L.B, units, rend);
-    } else {
-        MOEA_LAUNCH_M(m, nds_dominance, dgrid, dblock, 0, stream, L.fs, L.cvs, npad, n, W, Wc, L.kind,
-                      L.hi, L.B, units, rend);
-    }
+    const int seg = dom_segment(W, Wc);
+    const dim3 dgrid(ceil_div(W, seg), Wc), dblock(kDomThreads);
+    MOEA_LAUNCH_M(m, nds_dominance, dgrid, dblock, dom_lds_bytes(m), stream, L.fs, npad, n, W, Wc, L.valid, L.hi,
+                  L.tables, L.B, rend, seg);
     MOEA_HIP(hipGetLastError());
     stage_end(kStDominance, stream);
 
@@ -1112,7 +1079,7 @@ int nds_run(const float* f, int ldf, const float* cv, int n, int m, int stop_at,
     const int bpg = ceil_div(W, grid);
     const size_t lds = peel_lds_bytes(W, bpg);
     PeelArgs args{L.B, L.hi, L.perm, n, W, Wc, stop_at, bpg, fronts, L.A0, L.A1, L.state, max_front, rend,
-                  peel_spin_limit(), error};
+                  peel_spin_limit(), error, L.gmask, L.info};
     void* kargs[] = {&args};
     stage_begin(kStPeel, stream);
     MOEA_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(nds_peel), dim3(grid),
@@ -1265,18 +1232,15 @@ int batch_nds(const BatchLaunch& L, const BNdsGrids& G, const BNdsScratch& S, in
     MOEA_HIP(hipGetLastError());
     MOEA_CHECK(sort_pairs(S.sort_temp, S.sort_bytes, S.keys_in, S.keys_out, S.vals_in, S.vals_out,
                           static_cast<int>(G.total_rows), st, kKeyBits + S.inst_bits));
-    hipLaunchKernelGGL(b_nds_gather, dim3(G.npad256.blocks), dim3(256), 0, st, L.insts, G.npad256.map, mode,
+    hipLaunchKernelGGL(b_nds_prep, dim3(G.prep.blocks), dim3(kChunk), 0, st, L.insts, G.prep.map, mode, S.keys_out,
                        S.vals_out);
-    MOEA_HIP(hipGetLastError());
-    hipLaunchKernelGGL(b_nds_block_info, dim3(G.blocks64.blocks), dim3(64), 0, st, L.insts, G.blocks64.map,
-                       mode, S.keys_out);
     MOEA_HIP(hipGetLastError());
     stage_end(kStNdsSort, st);
     stage_begin(kStDominance, st);
     for (int m = 1; m <= kMaxM; ++m) {
         if (G.dom[m].blocks <= 0) continue;
         const dim3 grid(G.dom[m].blocks), block(kDomThreads);
-        MOEA_LAUNCH_M(m, b_nds_dominance, grid, block, 0, st, L.insts, G.dom[m].map, mode);
+        MOEA_LAUNCH_M(m, b_nds_dominance, grid, block, dom_lds_bytes(m), st, L.insts, G.dom[m].map, mode);
         MOEA_HIP(hipGetLastError());
     }
     stage_end(kStDominance, st);
