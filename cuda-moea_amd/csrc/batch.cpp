@@ -91,6 +91,7 @@ void carve_instance(Carve& c, const moea_batch_problem& p, BInst& I)
     I.chosen = c.take<int32_t>(z.n);
     I.B = c.take<uint64_t>(static_cast<size_t>(z.W) * z.Wc * 512);
     I.fs = c.take<float>(static_cast<size_t>(z.m) * z.npad);
+    I.ties = c.take<int2>(z.nm);
     I.tables = c.take<unsigned char>(nds_table_bytes(z.nm, z.m));
     I.perm = c.take<int32_t>(z.nm);
     I.hi = c.take<int32_t>(z.W);

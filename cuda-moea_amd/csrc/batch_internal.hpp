@@ -77,7 +77,8 @@ struct BInst {
     // NDS scratch (2n merged rows, or n for the initial parents)
     uint64_t* B;                  // (W * Wc * 512) dominator bitmask, sorted order
     float* fs;                    // (m, npad) sorted objectives
-    unsigned char* tables;        // (Wc, m) rank tables of the dominance kernel
+    unsigned char* tables;        // (Wc, m - 1) rank tables of the dominance kernel
+    int2* ties;                   // (nm) run of equal first objectives of each row, sorted order
     int32_t* perm;                // (nm) sorted position -> local row
     int32_t* hi;                  // (W)
     uint64_t* valid;              // (8 Wc) feasible rows without a NaN objective, sorted order

@@ -57,8 +57,9 @@ namespace moea {
 namespace {
 
 constexpr int kRowEndMinM = 4;           // fewest objectives for which the sort computes row ends
-constexpr int kDomThreads = 512;         // dominance workgroup: each wave takes a row block at a time
-constexpr int kDomWaves = kDomThreads / 64;
+// Threads of a dominance workgroup, each wave a row block at a time: from six
+// objectives one workgroup's tables fill a CU's LDS, so it brings all 16 waves.
+constexpr int dom_threads(int m) { return m >= 6 ? 1024 : 512; }
 constexpr int kChunk = 512;              // sorted rows q per rank table: the 8 words of a chunk of B
 constexpr int kKeyBits = 34;             // segment (2 bits) above a 32-bit order key
 
@@ -127,21 +128,42 @@ __device__ __forceinline__ void infeasible_info(const uint64_t* __restrict__ key
     }
 }
 
-// hi[b] of the block whose last row is `last` (see the header comment), read
-// by one lane.  Ties past a block are rare, so the next key is looked at before
-// the search.
-__device__ __forceinline__ int tie_end_block(const uint64_t* __restrict__ keys, int n, int last)
+// First position whose key is not below kl (kEqual: not below or equal) in
+// keys[lo, hi), the same in every lane.
+template <bool kEqual>
+__device__ __forceinline__ int key_bound(const uint64_t* __restrict__ keys, uint64_t kl, int lo, int hi)
 {
-    const uint64_t kl = keys[last];
-    if (last + 1 >= n || ((kl >> 32) & 3u) != 0 || keys[last + 1] != kl) return last >> 6;
-    // first position after `last` whose key differs (keys ascend)
-    int lo = last + 2, hi = n;
     while (lo < hi) {
         const int mid = (lo + hi) >> 1;
-        if (keys[mid] == kl) lo = mid + 1;
+        const uint64_t v = keys[mid];
+        if (kEqual ? v <= kl : v < kl) lo = mid + 1;
         else hi = mid;
     }
-    return (lo - 1) >> 6;
+    return lo;
+}
+
+// The run of equal keys [tie[0], tie[1]) of each row t of the wave's block
+// (rows of segment 0; other rows' values are not read) and the block's hi.
+// Runs are found in the block itself; one that crosses its border is searched.
+__device__ __forceinline__ void tie_runs(const uint64_t* __restrict__ keys, int n, int b, int lane,
+                                         int2* __restrict__ ties, int32_t* __restrict__ hi)
+{
+    const int first = b * 64, end = min(n, first + 64);
+    const int t = first + lane;
+    const uint64_t key = keys[min(t, n - 1)];
+    const uint64_t prev = t > 0 ? keys[min(t, n - 1) - 1] : ~key;
+    const uint64_t starts = ballot(t < end && prev != key);
+    const uint64_t key_last = keys[end - 1];
+    const bool seg0_first = ((keys[first] >> 32) & 3u) == 0, seg0_last = ((key_last >> 32) & 3u) == 0;
+    int before = first, after = end;      // start of the block's first run, end of its last
+    if (!(starts & 1ull) && seg0_first) before = key_bound<false>(keys, keys[first], 0, first);
+    if (seg0_last && end < n && keys[end] == key_last) after = key_bound<true>(keys, key_last, end + 1, n);
+    const uint64_t upto = starts & (lane == 63 ? ~0ull : (1ull << (lane + 1)) - 1);
+    const uint64_t past = starts & ~(lane == 63 ? ~0ull : (1ull << (lane + 1)) - 1);
+    if (t < n)
+        ties[t] = make_int2(upto ? first + 63 - __builtin_clzll(upto) : before,
+                            past ? first + __builtin_ctzll(past) : after);
+    if (lane == 0) hi[b] = seg0_last ? (after - 1) >> 6 : b;
 }
 
 // Rank table of one objective over a chunk of kChunk sorted rows, in sub-chunks
@@ -156,8 +178,8 @@ __device__ __forceinline__ int tie_end_block(const uint64_t* __restrict__ keys, 
 //   spread over all LDS banks instead of half of them.
 // A small S makes the table smaller and the sort below shorter, a large one the
 // searches fewer (9 steps per 256 rows against 8 per 128).  S = 256 holds up
-// to 8 objectives' tables in LDS (7 x 18.5 KB; the first objective needs none),
-// S = 128 up to 10 (9 x 10.3 KB).
+// to 8 objectives' tables in LDS (7 x 18.5 KB; the first objective, the sort
+// order itself, needs none), S = 128 up to 10 (9 x 10.3 KB).
 constexpr int rank_sub(int m) { return m <= 8 ? 256 : 128; }
 constexpr int kRankValueBytes = kChunk * 4;
 constexpr int rank_mask_bytes(int S) { return (S + 1) * (S / 8); }         // one sub-chunk's masks
@@ -166,8 +188,8 @@ __host__ __device__ constexpr int rank_table_bytes(int S)
     return (kRankValueBytes + (kChunk / S) * ((S + 1) * (S / 8)) + 255) / 256 * 256;
 }
 // the largest of an objective count's tables per chunk, for buffers sized without it
-constexpr int kRankChunkBytes = 10 * rank_table_bytes(128) > 8 * rank_table_bytes(256) ? 10 * rank_table_bytes(128)
-                                                                                     : 8 * rank_table_bytes(256);
+constexpr int kRankChunkBytes = 9 * rank_table_bytes(128) > 7 * rank_table_bytes(256) ? 9 * rank_table_bytes(128)
+                                                                                    : 7 * rank_table_bytes(256);
 static_assert(kMaxM == 10, "kRankChunkBytes covers 8 and 10 objectives");
 
 // Byte offset of 16-byte piece j of mask r.
@@ -178,15 +200,30 @@ __device__ __forceinline__ int rank_piece(int r, int j)
     else return r * 16;
 }
 
+// Number of the S ascending values v[0 .. S) that are <= x (kLess: < x).
+template <int S, bool kLess>
+__device__ __forceinline__ int rank_search(const float* v, float x)
+{
+    int pos = 0;
+#pragma unroll
+    for (int step = S / 2; step >= 1; step >>= 1) {
+        const float u = v[pos + step - 1];
+        pos += (kLess ? u < x : u <= x) ? step : 0;
+    }
+    const float u = v[pos];
+    return pos + ((kLess ? u < x : u <= x) ? 1 : 0);
+}
+
 // What nds_prep writes besides the tables.
 struct PrepOut {
     float* fs;               // (m, npad) sorted objectives, 0 in padding rows
     uint64_t* valid;         // (8 Wc) rows of segment 0 per block, 0 past the last block
     int32_t* hi;             // (W)
+    int2* ties;              // (n) see tie_runs
     uint64_t* gmask;         // (W) see infeasible_info
     int32_t* info;           // (2)
     int32_t* rend;           // optional (n): row ends, cleared for the dominance kernel to raise
-    unsigned char* tables;   // (Wc, m) rank tables
+    unsigned char* tables;   // (Wc, m - 1) rank tables of the objectives after the first
 };
 
 // One workgroup of kChunk threads: chunk qc, objective k.
@@ -195,8 +232,9 @@ __device__ __forceinline__ void prep_chunk(const float* __restrict__ f, int ldf,
                                            const int32_t* __restrict__ perm, const uint64_t* __restrict__ keys,
                                            int qc, int k, const PrepOut& O)
 {
-    __shared__ __align__(16) float s_v[kChunk];
-    __shared__ int s_rank[kChunk];
+    __shared__ __align__(16) float s_v[kChunk];     // values by position
+    __shared__ float s_sort[kChunk];                // values of each 64-row block, ascending
+    __shared__ uint16_t s_inv[kChunk];              // position (in its sub-chunk) of each rank
     const int tid = static_cast<int>(threadIdx.x);
     const int lane = lane_id();
     const int w = wave_uniform(tid >> 6);
@@ -210,69 +248,67 @@ __device__ __forceinline__ void prep_chunk(const float* __restrict__ f, int ldf,
         if (lane == 0) O.valid[b] = seg0;
         if (b * 64 < n) {
             infeasible_info(keys, n, t, O.gmask, O.info);
-            if (lane == 0) O.hi[b] = tie_end_block(keys, n, min(n, b * 64 + 64) - 1);
+            tie_runs(keys, n, b, lane, O.ties, O.hi);
             if (O.rend && t < n) O.rend[t] = 0;
         }
+        return;
     }
     // rows without a number are never looked up (valid masks them): any order does
     const float x = (t < n && !isnan(v)) ? v : INFINITY;
     s_v[tid] = x;
+    __builtin_amdgcn_wave_barrier();
+    // rank among the wave's own 64 rows, ties by position
+    int own = 0;
+    {
+        const float4* src = reinterpret_cast<const float4*>(s_v + w * 64);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const float4 u = src[j];
+            own += (u.x < x || (u.x == x && 4 * j < lane)) ? 1 : 0;
+            own += (u.y < x || (u.y == x && 4 * j + 1 < lane)) ? 1 : 0;
+            own += (u.z < x || (u.z == x && 4 * j + 2 < lane)) ? 1 : 0;
+            own += (u.w < x || (u.w == x && 4 * j + 3 < lane)) ? 1 : 0;
+        }
+    }
+    s_sort[w * 64 + own] = x;
     __syncthreads();
-    // rank of each value among its sub-chunk, ties by position
+    // and among the sub-chunk: its other blocks are searched, earlier ones for
+    // the values <= x, later ones for those < x
     const int h = wave_uniform(tid / S);
     const int w0 = h * (S / 64);
-    int rank = 0;
-#pragma unroll 1
-    for (int b = 0; b < S / 64; ++b) {
-        const float4* src = reinterpret_cast<const float4*>(s_v + h * S + b * 64);
-        const int own = w - w0;
-        if (b == own) {
-#pragma unroll 4
-            for (int j = 0; j < 16; ++j) {
-                const float4 u = src[j];
-                rank += (u.x < x || (u.x == x && 4 * j < lane)) ? 1 : 0;
-                rank += (u.y < x || (u.y == x && 4 * j + 1 < lane)) ? 1 : 0;
-                rank += (u.z < x || (u.z == x && 4 * j + 2 < lane)) ? 1 : 0;
-                rank += (u.w < x || (u.w == x && 4 * j + 3 < lane)) ? 1 : 0;
-            }
-        } else if (b < own) {
-#pragma unroll 4
-            for (int j = 0; j < 16; ++j) {
-                const float4 u = src[j];
-                rank += (u.x <= x) + (u.y <= x) + (u.z <= x) + (u.w <= x);
-            }
-        } else {
-#pragma unroll 4
-            for (int j = 0; j < 16; ++j) {
-                const float4 u = src[j];
-                rank += (u.x < x) + (u.y < x) + (u.z < x) + (u.w < x);
-            }
-        }
-    }
-    s_rank[tid] = rank;
-    unsigned char* tab = O.tables + (static_cast<size_t>(qc) * m + k) * rank_table_bytes(S);
-    reinterpret_cast<float*>(tab)[h * S + rank] = x;
-    // wave w: its 64 rows' word of every mask of their sub-chunk, 64 masks at a
-    // time with a lane per mask (bit e: row e's rank < r)
-    int re[64];
-    __syncthreads();
+    int rank = own;
 #pragma unroll
-    for (int e = 0; e < 64; ++e) re[e] = wave_uniform(s_rank[w * 64 + e]);
+    for (int o = 1; o < S / 64; ++o) {
+        const int b = w0 + ((w - w0 + o) & (S / 64 - 1));
+        rank += (b < w) ? rank_search<64, false>(s_sort + b * 64, x) : rank_search<64, true>(s_sort + b * 64, x);
+    }
+    s_inv[h * S + rank] = static_cast<uint16_t>(tid & (S - 1));
+    unsigned char* tab = O.tables + (static_cast<size_t>(qc) * (m - 1) + k - 1) * rank_table_bytes(S);
+    reinterpret_cast<float*>(tab)[h * S + rank] = x;
+    __syncthreads();
+    // wave w: its 64 rows' word of every mask of their sub-chunk.  Mask r + 1
+    // is mask r and the bit of the row of rank r: a prefix OR over the ranks,
+    // 64 a step.
     unsigned char* masks = tab + kRankValueBytes + h * rank_mask_bytes(S);
     const int jj = w - w0;
-#pragma unroll 1
-    for (int r0 = 0; r0 <= S; r0 += 64) {
-        const int r = r0 + lane;
-        uint32_t lo = 0, hi = 0;
+    uint64_t before = 0;
 #pragma unroll
-        for (int e = 31; e >= 0; --e) {
-            lo = shift_in(lo, ballot(re[e] < r));
-            hi = shift_in(hi, ballot(re[e + 32] < r));
+    for (int r0 = 0; r0 < S; r0 += 64) {
+        const int e = s_inv[h * S + r0 + lane];
+        uint64_t acc = (e >> 6) == jj ? 1ull << (e & 63) : 0ull;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t lo = static_cast<uint32_t>(__shfl_up(static_cast<int>(acc), o));
+            const uint32_t hi = static_cast<uint32_t>(__shfl_up(static_cast<int>(acc >> 32), o));
+            if (lane >= o) acc |= (static_cast<uint64_t>(hi) << 32) | lo;
         }
-        if (r <= S)
-            *reinterpret_cast<uint64_t*>(masks + rank_piece<S>(r, jj >> 1) + (jj & 1) * 8) =
-                (static_cast<uint64_t>(hi) << 32) | lo;
+        acc |= before;
+        const int r = r0 + lane;
+        *reinterpret_cast<uint64_t*>(masks + rank_piece<S>(r + 1, jj >> 1) + (jj & 1) * 8) = acc;
+        before = (static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(acc >> 32), 63))) << 32) |
+                 static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(acc), 63));
     }
+    if (lane == 0) *reinterpret_cast<uint64_t*>(masks + rank_piece<S>(0, jj >> 1) + (jj & 1) * 8) = 0ull;
 }
 
 // Grid (Wc, m).  zero (optional, `words` of them): cleared on the way, for a
@@ -291,65 +327,88 @@ __global__ __launch_bounds__(kChunk) void nds_prep(const float* __restrict__ f, 
     prep_chunk<S>(f, ldf, n, m, npad, perm, keys, static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), O);
 }
 
-// Number of the S ascending values v[0 .. S) that are <= x (kLess: < x).
-template <int S, bool kLess>
-__device__ __forceinline__ int rank_search(const float* v, float x)
+// Mask r of sub-chunk h of a table.
+template <int S>
+__device__ __forceinline__ void rank_mask(const unsigned char* tab, int h, int r, uint64_t (&out)[S / 64])
 {
-    int pos = 0;
+    const unsigned char* masks = tab + kRankValueBytes + h * rank_mask_bytes(S);
 #pragma unroll
-    for (int step = S / 2; step >= 1; step >>= 1) {
-        const float u = v[pos + step - 1];
-        pos += (kLess ? u < x : u <= x) ? step : 0;
+    for (int j = 0; j < S / 128; ++j) {
+        const ulonglong2 u = *reinterpret_cast<const ulonglong2*>(masks + rank_piece<S>(r, j));
+        out[2 * j] = u.x;
+        out[2 * j + 1] = u.y;
     }
-    const float u = v[pos];
-    return pos + ((kLess ? u < x : u <= x) ? 1 : 0);
 }
 
-// The 512 bits of a table for x: rows with a value <= x (kLess: < x).
-template <int S, bool kLess>
-__device__ __forceinline__ void rank_bits(const unsigned char* tab, float x, uint64_t (&out)[8])
+// The first r of the 64 rows of a word (r clamped to 0 .. 64).
+__device__ __forceinline__ uint64_t first_rows(int r)
 {
-    int r[kChunk / S];
-#pragma unroll
-    for (int h = 0; h < kChunk / S; ++h) r[h] = rank_search<S, kLess>(reinterpret_cast<const float*>(tab) + h * S, x);
-#pragma unroll
-    for (int h = 0; h < kChunk / S; ++h) {
-        const unsigned char* masks = tab + kRankValueBytes + h * rank_mask_bytes(S);
-#pragma unroll
-        for (int j = 0; j < S / 128; ++j) {
-            const ulonglong2 u = *reinterpret_cast<const ulonglong2*>(masks + rank_piece<S>(r[h], j));
-            out[h * (S / 64) + 2 * j] = u.x;
-            out[h * (S / 64) + 2 * j + 1] = u.y;
-        }
-    }
+    return r <= 0 ? 0ull : r >= 64 ? ~0ull : (1ull << r) - 1;
 }
 
 // A chunk whose f0 ties with row block pb, or that holds pb itself (or rows
-// after it): every objective's <=, without the rows equal in all of them.  The
-// first objective's table is read where nds_prep left it.
+// after it): every objective's <=, without the rows equal in all of them.  f0
+// is the sort order: rows before `tie`'s end are <=, those in it equal.
 template <int M, int S>
-__device__ __forceinline__ void tied_bits(const unsigned char* tab0, const unsigned char* s_tab, const float (&pv)[M],
+__device__ __forceinline__ void tied_bits(const unsigned char* s_tab, const float (&pv)[M], int2 tie, int q0,
                                           uint64_t (&bits)[8])
 {
-    uint64_t eq[8], lt[8], le[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) eq[j] = ~0ull;
-#pragma unroll 1
-    for (int k = 0; k < M; ++k) {
-        const unsigned char* tab = k == 0 ? tab0 : s_tab + (k - 1) * rank_table_bytes(S);
-        float x = pv[0];
+    for (int h = 0; h < kChunk / S; ++h) {
+        uint64_t eq[S / 64], le[S / 64], lt[S / 64];
 #pragma unroll
-        for (int c = 1; c < M; ++c) x = (k == c) ? pv[c] : x;
-        rank_bits<S, false>(tab, x, le);
-        rank_bits<S, true>(tab, x, lt);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            bits[j] &= le[j];
-            eq[j] &= le[j] & ~lt[j];
+        for (int j = 0; j < S / 64; ++j) {
+            const int b = h * (S / 64) + j;
+            const uint64_t le0 = first_rows(tie.y - q0 - b * 64);
+            bits[b] &= le0;
+            eq[j] = le0 & ~first_rows(tie.x - q0 - b * 64);
         }
+#pragma unroll 1
+        for (int k = 1; k < M; ++k) {
+            const unsigned char* tab = s_tab + (k - 1) * rank_table_bytes(S);
+            float x = pv[M > 1 ? 1 : 0];
+#pragma unroll
+            for (int c = 2; c < M; ++c) x = (k == c) ? pv[c] : x;
+            const float* v = reinterpret_cast<const float*>(tab) + h * S;
+            rank_mask<S>(tab, h, rank_search<S, false>(v, x), le);
+            rank_mask<S>(tab, h, rank_search<S, true>(v, x), lt);
+#pragma unroll
+            for (int j = 0; j < S / 64; ++j) {
+                bits[h * (S / 64) + j] &= le[j];
+                eq[j] &= le[j] & ~lt[j];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < S / 64; ++j) bits[h * (S / 64) + j] &= ~eq[j];
+    }
+}
+
+// Four lanes of a quad with four 16-byte pieces each (words 4j .. 4j + 3):
+// afterwards lane q holds piece q of the quad's lanes 0 .. 3, by two rounds of
+// exchange.
+template <int kCtrl>
+__device__ __forceinline__ void quad_trade(uint32_t& a, uint32_t& b, bool high)
+{
+    const uint32_t got = static_cast<uint32_t>(
+        __builtin_amdgcn_mov_dpp(static_cast<int>(high ? a : b), kCtrl, 0xf, 0xf, true));
+    a = high ? got : a;
+    b = high ? b : got;
+}
+
+__device__ __forceinline__ void quad_transpose(uint32_t (&w)[16], int lane)
+{
+    constexpr int kXor1 = 0xB1, kXor2 = 0x4E;   // quad_perm [1,0,3,2] and [2,3,0,1]
+    const bool odd = lane & 1, top = lane & 2;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        quad_trade<kXor1>(w[i], w[4 + i], odd);
+        quad_trade<kXor1>(w[8 + i], w[12 + i], odd);
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) bits[j] &= ~eq[j];
+    for (int i = 0; i < 4; ++i) {
+        quad_trade<kXor2>(w[i], w[8 + i], top);
+        quad_trade<kXor2>(w[4 + i], w[12 + i], top);
+    }
 }
 
 // One workgroup: chunk qc against the row blocks [pb0, pb1), a row block per
@@ -364,18 +423,18 @@ __device__ __forceinline__ void tied_bits(const unsigned char* tab0, const unsig
 template <int M>
 __device__ __forceinline__ void dom_chunk(const float* __restrict__ fs, int npad, int n, int W, int Wc,
                                           const uint64_t* __restrict__ valid, const int32_t* __restrict__ hi,
-                                          const unsigned char* __restrict__ tables, uint64_t* __restrict__ B,
-                                          int32_t* __restrict__ rend, int qc, int pb0, int pb1, unsigned char* s_tab)
+                                          const int2* __restrict__ ties, const unsigned char* __restrict__ tables,
+                                          uint64_t* __restrict__ B, int32_t* __restrict__ rend, int qc, int pb0, int pb1, unsigned char* s_tab)
 {
     constexpr int S = rank_sub(M);
     constexpr int kTab = rank_table_bytes(S);
+    constexpr int kThreads = dom_threads(M);
     if (hi[pb1 - 1] < 8 * qc) return;            // hi ascends: no row block here reaches the chunk
-    const unsigned char* tab0 = tables + static_cast<size_t>(qc) * M * kTab;
     if constexpr (M > 1) {
-        const uint4* src = reinterpret_cast<const uint4*>(tab0 + kTab);
+        const uint4* src = reinterpret_cast<const uint4*>(tables + static_cast<size_t>(qc) * (M - 1) * kTab);
         uint4* dst = reinterpret_cast<uint4*>(s_tab);
 #pragma unroll 4
-        for (int j = static_cast<int>(threadIdx.x); j < (M - 1) * kTab / 16; j += kDomThreads) dst[j] = src[j];
+        for (int j = static_cast<int>(threadIdx.x); j < (M - 1) * kTab / 16; j += kThreads) dst[j] = src[j];
         __syncthreads();
     }
     const int lane = lane_id();
@@ -383,7 +442,7 @@ __device__ __forceinline__ void dom_chunk(const float* __restrict__ fs, int npad
 #pragma unroll
     for (int j = 0; j < 8; ++j) vq[j] = ld_uniform(valid, static_cast<size_t>(qc) * 8 + j);
     const int tie_to = ld_uniform(hi, min(8 * qc + 7, W - 1));   // last block that ties with the chunk
-    for (int pb = pb0 + wave_uniform(static_cast<int>(threadIdx.x >> 6)); pb < pb1; pb += kDomWaves) {
+    for (int pb = pb0 + wave_uniform(static_cast<int>(threadIdx.x >> 6)); pb < pb1; pb += kThreads / 64) {
         if (ld_uniform(hi, pb) < 8 * qc) continue;
         const uint64_t vp = ld_uniform(valid, pb);
         // rows outside segment 0: feasible ones with a NaN objective have no
@@ -399,17 +458,34 @@ __device__ __forceinline__ void dom_chunk(const float* __restrict__ fs, int npad
         if (8 * qc + 7 < pb && tie_to < pb) {
 #pragma unroll
             for (int k = 1; k < M; ++k) {
-                uint64_t le[8];
-                rank_bits<S, false>(s_tab + (k - 1) * kTab, pv[k], le);
+                const unsigned char* tab = s_tab + (k - 1) * kTab;
+                int r[kChunk / S];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) bits[j] &= le[j];
+                for (int h = 0; h < kChunk / S; ++h)
+                    r[h] = rank_search<S, false>(reinterpret_cast<const float*>(tab) + h * S, pv[k]);
+#pragma unroll
+                for (int h = 0; h < kChunk / S; ++h) {
+                    uint64_t le[S / 64];
+                    rank_mask<S>(tab, h, r[h], le);
+#pragma unroll
+                    for (int j = 0; j < S / 64; ++j) bits[h * (S / 64) + j] &= le[j];
+                }
             }
         } else {
-            tied_bits<M, S>(tab0, s_tab, pv, bits);
+            tied_bits<M, S>(s_tab, pv, ties[min(p, n - 1)], qc * kChunk, bits);
         }
-        ulonglong2* dst = reinterpret_cast<ulonglong2*>(B + ((static_cast<size_t>(pb) * Wc + qc) * 64 + lane) * 8);
+        // a lane quad trades pieces so that it writes whole 64-byte rows, one a
+        // store, instead of 16 bytes of four rows: a quarter of the L2 requests
+        uint32_t w[16];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) dst[j] = make_ulonglong2(bits[2 * j], bits[2 * j + 1]);
+        for (int j = 0; j < 8; ++j) {
+            w[2 * j] = static_cast<uint32_t>(bits[j]);
+            w[2 * j + 1] = static_cast<uint32_t>(bits[j] >> 32);
+        }
+        quad_transpose(w, lane);
+        uint4* dst = reinterpret_cast<uint4*>(B + ((static_cast<size_t>(pb) * Wc + qc) * 64 + (lane & ~3)) * 8) + (lane & 3);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dst[j * 4] = make_uint4(w[4 * j], w[4 * j + 1], w[4 * j + 2], w[4 * j + 3]);
         if (rend && p < n) {
             int top = 0;
 #pragma unroll
@@ -425,26 +501,28 @@ constexpr size_t dom_lds_bytes(int m) { return static_cast<size_t>(m > 1 ? m - 1
 
 // Grid (ceil(W / seg), Wc).
 template <int M>
-__global__ __launch_bounds__(kDomThreads) void nds_dominance(const float* __restrict__ fs, int npad, int n, int W,
+__global__ __launch_bounds__(dom_threads(M)) void nds_dominance(const float* __restrict__ fs, int npad, int n, int W,
                                                             int Wc, const uint64_t* __restrict__ valid,
                                                             const int32_t* __restrict__ hi,
+                                                            const int2* __restrict__ ties,
                                                             const unsigned char* __restrict__ tables,
                                                             uint64_t* __restrict__ B, int32_t* __restrict__ rend,
                                                             int seg)
 {
     extern __shared__ __align__(16) unsigned char s_tab[];
     const int pb0 = static_cast<int>(blockIdx.x) * seg;
-    dom_chunk<M>(fs, npad, n, W, Wc, valid, hi, tables, B, rend, static_cast<int>(blockIdx.y), pb0,
+    dom_chunk<M>(fs, npad, n, W, Wc, valid, hi, ties, tables, B, rend, static_cast<int>(blockIdx.y), pb0,
                  min(pb0 + seg, W), s_tab);
 }
 
 // Row blocks per dominance workgroup: enough workgroups to fill the chip, and
 // enough row blocks in each to pay for loading its tables.
-int dom_segment(int W, int Wc)
+int dom_segment(int W, int Wc, int m)
 {
+    const int waves = dom_threads(m) / 64;
     const long long units = static_cast<long long>(W) * Wc / 2;
-    const long long per = units / 1024 / kDomWaves * kDomWaves;
-    return static_cast<int>(std::max<long long>(kDomWaves, std::min<long long>(64, per)));
+    const long long per = units / 1024 / waves * waves;
+    return static_cast<int>(std::max<long long>(waves, std::min<long long>(64, per)));
 }
 
 // Peel state (device), u32 words: [0, kBarWords) group barrier,
@@ -862,7 +940,7 @@ __global__ __launch_bounds__(kChunk) void b_nds_prep(const BInst* __restrict__ i
     const int t = qc * kChunk + static_cast<int>(threadIdx.x);
     const int32_t* perm = vals_sorted + R.key_off;
     if (k == 0 && t < R.rows) I.perm[t] = perm[t];
-    const PrepOut O{I.fs, I.valid, I.hi, I.gmask, I.ninfo, I.m >= kRowEndMinM ? I.rend : nullptr, I.tables};
+    const PrepOut O{I.fs, I.valid, I.hi, I.ties, I.gmask, I.ninfo, I.m >= kRowEndMinM ? I.rend : nullptr, I.tables};
     if (rank_sub(I.m) == 256) prep_chunk<256>(R.f, R.rows, R.rows, I.m, W * 64, perm, keys_sorted + R.key_off, qc, k, O);
     else prep_chunk<128>(R.f, R.rows, R.rows, I.m, W * 64, perm, keys_sorted + R.key_off, qc, k, O);
 }
@@ -870,7 +948,7 @@ __global__ __launch_bounds__(kChunk) void b_nds_prep(const BInst* __restrict__ i
 // nds_dominance of the instances with M objectives: Wc x ceil(W / kBatchDomSeg)
 // workgroups each.
 template <int M>
-__global__ __launch_bounds__(kDomThreads) void b_nds_dominance(const BInst* __restrict__ insts, BMap mp, int mode)
+__global__ __launch_bounds__(dom_threads(M)) void b_nds_dominance(const BInst* __restrict__ insts, BMap mp, int mode)
 {
     extern __shared__ __align__(16) unsigned char s_tab[];
     int local;
@@ -879,8 +957,8 @@ __global__ __launch_bounds__(kDomThreads) void b_nds_dominance(const BInst* __re
     const BRows R = brows(I, mode);
     const int W = (R.rows + 63) / 64, Wc = (W + 7) / 8;
     const int qc = local % Wc, pb0 = local / Wc * kBatchDomSeg;
-    dom_chunk<M>(I.fs, W * 64, R.rows, W, Wc, I.valid, I.hi, I.tables, I.B, M >= kRowEndMinM ? I.rend : nullptr, qc,
-                 pb0, min(pb0 + kBatchDomSeg, W), s_tab);
+    dom_chunk<M>(I.fs, W * 64, R.rows, W, Wc, I.valid, I.hi, I.ties, I.tables, I.B,
+                 M >= kRowEndMinM ? I.rend : nullptr, qc, pb0, min(pb0 + kBatchDomSeg, W), s_tab);
 }
 
 // Where a batched peel leaves the index of its last front: the selection's
@@ -947,6 +1025,7 @@ struct NdsLayout {
     float* fs;
     unsigned char* tables;
     int32_t* hi;
+    int2* ties;
     uint64_t* valid;
     uint64_t* A0;
     uint64_t* A1;
@@ -972,6 +1051,7 @@ size_t carve_nds(void* ws, int n, NdsLayout& L)
     L.fs = c.take<float>(static_cast<size_t>(kMaxM) * npad);
     L.tables = c.take<unsigned char>(static_cast<size_t>(Wc) * kRankChunkBytes);
     L.hi = c.take<int32_t>(W);
+    L.ties = c.take<int2>(n);
     L.valid = c.take<uint64_t>(static_cast<size_t>(Wc) * 8);
     L.A0 = c.take<uint64_t>(W);
     L.A1 = c.take<uint64_t>(W);
@@ -1010,7 +1090,7 @@ int peel_grid_size(int nblk)
 // Rank-table bytes of one instance with nm rows and m objectives.
 size_t nds_table_bytes(int nm, int m)
 {
-    return static_cast<size_t>(ceil_div(nm, kChunk)) * m * rank_table_bytes(rank_sub(m));
+    return static_cast<size_t>(ceil_div(nm, kChunk)) * (m - 1) * rank_table_bytes(rank_sub(m));
 }
 
 size_t nds_workspace_bytes(int n)
@@ -1054,7 +1134,7 @@ int nds_run(const float* f, int ldf, const float* cv, int n, int m, int stop_at,
     // row ends pay for their atomics when many rows have no dominator near
     // their own block, which is the case for many objectives
     int32_t* rend = m >= kRowEndMinM ? L.rend : nullptr;
-    const PrepOut O{L.fs, L.valid, L.hi, L.gmask, L.info, rend, L.tables};
+    const PrepOut O{L.fs, L.valid, L.hi, L.ties, L.gmask, L.info, rend, L.tables};
     const dim3 pgrid(Wc, m), pblock(kChunk);
     // also clears the peel's barrier state (not read before the peel)
     if (rank_sub(m) == 256)
@@ -1067,10 +1147,10 @@ int nds_run(const float* f, int ldf, const float* cv, int n, int m, int stop_at,
     stage_end(kStNdsSort, stream);
 
     stage_begin(kStDominance, stream);
-    const int seg = dom_segment(W, Wc);
-    const dim3 dgrid(ceil_div(W, seg), Wc), dblock(kDomThreads);
+    const int seg = dom_segment(W, Wc, m);
+    const dim3 dgrid(ceil_div(W, seg), Wc), dblock(dom_threads(m));
     MOEA_LAUNCH_M(m, nds_dominance, dgrid, dblock, dom_lds_bytes(m), stream, L.fs, npad, n, W, Wc, L.valid, L.hi,
-                  L.tables, L.B, rend, seg);
+                  L.ties, L.tables, L.B, rend, seg);
     MOEA_HIP(hipGetLastError());
     stage_end(kStDominance, stream);
 
@@ -1239,7 +1319,7 @@ int batch_nds(const BatchLaunch& L, const BNdsGrids& G, const BNdsScratch& S, in
     stage_begin(kStDominance, st);
     for (int m = 1; m <= kMaxM; ++m) {
         if (G.dom[m].blocks <= 0) continue;
-        const dim3 grid(G.dom[m].blocks), block(kDomThreads);
+        const dim3 grid(G.dom[m].blocks), block(dom_threads(m));
         MOEA_LAUNCH_M(m, b_nds_dominance, grid, block, dom_lds_bytes(m), st, L.insts, G.dom[m].map, mode);
         MOEA_HIP(hipGetLastError());
     }
