@@ -585,39 +585,20 @@ __device__ __forceinline__ uint64_t nds_key_from(float f0, bool any_nan, float c
 // ----------------------------------------------------------------------------
 __device__ inline uint64_t ballot(bool pred) { return __builtin_amdgcn_ballot_w64(pred); }
 
-// v_writelane_b32 with a compile-time lane: lane J of the result takes the
-// wave-uniform `value` (an inline-constant lane keeps the instruction within
-// the constant-bus limit).
-template <int J>
-__device__ inline uint32_t writelane(uint32_t old, uint32_t value)
-{
-    uint32_t r = old;
-    const uint32_t v = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(value)));
-    asm volatile("v_writelane_b32 %0, %1, %2" : "+v"(r) : "s"(v), "n"(J));
-    return r;
-}
-
-// Compile-time loop: f(std::integral_constant<int, J>) for J in Js.
-template <typename F, int... Js>
-__device__ inline void static_for(F&& f, std::integer_sequence<int, Js...>)
-{
-    (f(std::integral_constant<int, Js>{}), ...);
-}
-
 __device__ inline int lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
 
 // Marks a value the whole wave agrees on as uniform (kept in an SGPR), so
 // loads indexed by it become scalar loads.
 __device__ inline int wave_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// Lane mask of !(s > v) for a wave-uniform s: one v_cmp_ngt_f32 writing an
-// SGPR pair (true for unordered operands).
-__device__ inline uint64_t mask_not_gt(float s, float v)
+// Wave-uniform reads of data the kernel never writes, through the constant
+// address space so they compile to scalar loads even where alias analysis
+// cannot prove the pointer read-only (device functions, pointers from tables).
+template <typename T>
+__device__ __forceinline__ T ld_uniform(const T* p, size_t i)
 {
-    const float su = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(s)));
-    uint64_t m;
-    asm("v_cmp_ngt_f32_e64 %0, %1, %2" : "=s"(m) : "s"(su), "v"(v));
-    return m;
+    using const_ptr = const __attribute__((address_space(4))) T*;
+    return ((const_ptr)p)[i];   // address-space conversion (a C-style cast performs it)
 }
 
 // Per lane: acc * 2 + (bit `lane` of mask).  One v_addc_co_u32 with the

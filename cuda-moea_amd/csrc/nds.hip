@@ -68,16 +68,6 @@ __host__ __device__ __forceinline__ size_t bword_index(int p, int w, int Wc)
     return ((static_cast<size_t>(p >> 6) * Wc + (w >> 3)) * 64 + (p & 63)) * 8 + (w & 7);
 }
 
-// Wave-uniform reads of data the kernel never writes, through the constant
-// address space so they compile to scalar loads even where alias analysis
-// cannot prove the pointer read-only (device functions, pointers from tables).
-template <typename T>
-__device__ __forceinline__ T ld_uniform(const T* p, size_t i)
-{
-    using const_ptr = const __attribute__((address_space(4))) T*;
-    return ((const_ptr)p)[i];   // address-space conversion (a C-style cast performs it)
-}
-
 __device__ __forceinline__ uint64_t nds_key_of(const float* __restrict__ f, int ldf, const float* __restrict__ cv,
                                       int s, int m)
 {

@@ -9,6 +9,8 @@
 // Arithmetic notes: the partition's rsqrtf (reference_partition.cu:77-78) is
 // evaluated as 1 / sqrtf, and acosf as the deterministic acosf_det, because
 // CUDA's approximate last bits cannot be reproduced.
+#include <algorithm>
+
 #include "common.hpp"
 #include "moea_internal.hpp"
 
@@ -206,35 +208,53 @@ __device__ inline int block_scan_excl(int v, int* s_wave, int& total)
     return res;
 }
 
-// Winner count, survivor flags and the ascending survivor list
-// (generate_newpop_gidx, elitism_selection.cu:272-419; sort at
-// rvea_population_update.cu:281).  Single 1024-thread block.
+// Winner count and the ascending survivor list (generate_newpop_gidx,
+// elitism_selection.cu:272-419; sort at rvea_population_update.cu:281).  One
+// 1024-thread block with the survivor set as nm bits in LDS, words interleaved
+// over the threads so that every pass is contiguous: 64 us with a byte per row
+// in global memory, cleared, set and re-read in strided chunks, against 12 us
+// (nm = 32768).  is_winner is a 0/1 byte per row.  kLds = false keeps the set
+// in the workspace: for more rows than 64 KiB of LDS holds as bits.
+constexpr size_t kChooseMaxLds = 64 * 1024;
+
+template <bool kLds>
 __global__ __launch_bounds__(kScan) void rv_choose(const uint8_t* __restrict__ is_winner, int nm, int n,
                                                    const int32_t* __restrict__ tvals_sorted,
                                                    const int32_t* __restrict__ elit_vals_sorted,
-                                                   uint8_t* __restrict__ flag,
-                                                   int32_t* __restrict__ chosen,
+                                                   uint32_t* __restrict__ g_bits, int32_t* __restrict__ chosen,
                                                    int32_t* __restrict__ meta)
 {
+    extern __shared__ uint32_t s_bits[];        // ceil(nm / 32) words
     __shared__ int s_wave[64];
-    const int chunk = (nm + kScan - 1) / kScan;
-    const int b = threadIdx.x * chunk, e = min(nm, b + chunk);
+    const int words = (nm + 31) / 32;
+    uint32_t* bits = kLds ? s_bits : g_bits;
     int c = 0;
-    for (int i = b; i < e; ++i) c += is_winner[i];
+    const uint32_t* w4 = reinterpret_cast<const uint32_t*>(is_winner);
+    for (int i = threadIdx.x; i < nm / 4; i += kScan) c += __builtin_popcount(w4[i]);
+    if (static_cast<int>(threadIdx.x) < nm % 4) c += is_winner[nm / 4 * 4 + threadIdx.x];
+    for (int i = threadIdx.x; i < words; i += kScan) {
+        if constexpr (kLds) bits[i] = 0u;
+        else st_relaxed_u32(&bits[i], 0u);
+    }
+    drain_memory();
     int winners;
     block_scan_excl(c, s_wave, winners);
-    for (int i = b; i < e; ++i) flag[i] = 0;
-    __syncthreads();
     const int take = (winners == 0) ? n : min(winners, n);
     const int32_t* src = (winners == 0) ? elit_vals_sorted : tvals_sorted;
-    for (int t = threadIdx.x; t < take; t += kScan) flag[src[t]] = 1;
+    for (int t = threadIdx.x; t < take; t += kScan) atomicOr(&bits[src[t] >> 5], 1u << (src[t] & 31));
+    drain_memory();
     __syncthreads();
-    int f = 0;
-    for (int i = b; i < e; ++i) f += flag[i];
-    int tot;
-    int o = block_scan_excl(f, s_wave, tot);
-    for (int i = b; i < e; ++i)
-        if (flag[i] && o < n) chosen[o++] = i;
+    int done = 0;
+    for (int base = 0; base < words; base += kScan) {
+        const int i = base + static_cast<int>(threadIdx.x);
+        uint32_t b = 0u;
+        if (i < words) b = kLds ? bits[i] : ld_relaxed_u32(&bits[i]);
+        int tot;
+        int o = done + block_scan_excl(__builtin_popcount(b), s_wave, tot);
+        done += tot;
+        for (; b; b &= b - 1, ++o)
+            if (o < n) chosen[o] = i * 32 + __builtin_ctz(b);
+    }
     if (threadIdx.x == 0) {
         meta[kRWinners] = winners;
         meta[kRActive] = take;
@@ -271,23 +291,93 @@ __global__ __launch_bounds__(256) void rv_gather(const int32_t* __restrict__ cho
 }
 
 // gamma_j = acos(max_{q != j} v_j . v_q), pi when there is no other direction
-// (gamma_phase1/2_kernel, angle_penalized_distance.cu:196-362).
+// (gamma_phase1/2_kernel, angle_penalized_distance.cu:196-362).  A maximum does
+// not depend on its order, so the k^2 products are cut into tiles: a workgroup
+// takes 512 directions j (two a thread) against `per` directions q, read as
+// scalars, and raises each j's maximum, kept in gamma as an order-preserving
+// integer between the first and the last of the three launches.  M fused
+// multiply-adds and half a maximum a pair.  A thread per direction against all
+// others put 59 workgroups on 256 CUs and waited on every q: 2226 us at
+// k = 14950, M = 5, against 48 us.
+constexpr int kGammaRows = 512;
+constexpr int kGammaGroup = 8;
+
+__global__ void rv_gamma_init(uint32_t* __restrict__ key, int k)
+{
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j < k) key[j] = order_key(-INFINITY);
+}
+
 template <int M>
-__global__ void rv_gamma(const float* __restrict__ v, int k, float* __restrict__ gamma)
+__global__ __launch_bounds__(256) void rv_gamma_tiles(const float* __restrict__ v, int k, int per,
+                                                      uint32_t* __restrict__ key)
+{
+    const int j0 = blockIdx.x * kGammaRows + static_cast<int>(threadIdx.x), j1 = j0 + 256;
+    const int w0 = blockIdx.x * kGammaRows + wave_uniform(static_cast<int>(threadIdx.x >> 6)) * 64, w1 = w0 + 256;
+    const int o0 = blockIdx.y * per, o1 = min(k, o0 + per);
+    float q0[M], q1[M];
+#pragma unroll
+    for (int c = 0; c < M; ++c) {
+        q0[c] = v[static_cast<size_t>(c) * k + min(j0, k - 1)];
+        q1[c] = v[static_cast<size_t>(c) * k + min(j1, k - 1)];
+    }
+    float m0 = -INFINITY, m1 = -INFINITY;
+    const auto one = [&](int o, const float* u) {
+        float d0 = 0.0f, d1 = 0.0f;
+#pragma unroll
+        for (int c = 0; c < M; ++c) {
+            d0 = fmaf(q0[c], u[c], d0);
+            d1 = fmaf(q1[c], u[c], d1);
+        }
+        if (o != j0) m0 = fmaxf(m0, d0);
+        if (o != j1) m1 = fmaxf(m1, d1);
+    };
+    int o = o0;
+    for (; o + kGammaGroup <= o1; o += kGammaGroup) {
+        float u[M][kGammaGroup];
+#pragma unroll
+        for (int c = 0; c < M; ++c)
+#pragma unroll
+            for (int i = 0; i < kGammaGroup; ++i) u[c][i] = ld_uniform(v, static_cast<size_t>(c) * k + o + i);
+        if ((o + kGammaGroup > w0 && o < w0 + 64) || (o + kGammaGroup > w1 && o < w1 + 64)) {
+            // the group holds one of the wave's own directions
+#pragma unroll
+            for (int i = 0; i < kGammaGroup; ++i) {
+                float t[M];
+#pragma unroll
+                for (int c = 0; c < M; ++c) t[c] = u[c][i];
+                one(o + i, t);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < kGammaGroup; ++i) {
+                float d0 = 0.0f, d1 = 0.0f;
+#pragma unroll
+                for (int c = 0; c < M; ++c) {
+                    d0 = fmaf(q0[c], u[c][i], d0);
+                    d1 = fmaf(q1[c], u[c][i], d1);
+                }
+                m0 = fmaxf(m0, d0);
+                m1 = fmaxf(m1, d1);
+            }
+        }
+    }
+    for (; o < o1; ++o) {
+        float t[M];
+#pragma unroll
+        for (int c = 0; c < M; ++c) t[c] = ld_uniform(v, static_cast<size_t>(c) * k + o);
+        one(o, t);
+    }
+    if (j0 < k) atomicMax(&key[j0], order_key(m0));
+    if (j1 < k) atomicMax(&key[j1], order_key(m1));
+}
+
+__global__ void rv_gamma_finish(float* gamma, int k)
 {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= k) return;
-    float q[M];
-#pragma unroll
-    for (int c = 0; c < M; ++c) q[c] = v[static_cast<size_t>(c) * k + j];
-    float mx = -INFINITY;
-    for (int o = 0; o < k; ++o) {
-        if (o == j) continue;
-        float dot = 0.0f;
-#pragma unroll
-        for (int c = 0; c < M; ++c) dot = fmaf(q[c], v[static_cast<size_t>(c) * k + o], dot);
-        mx = fmaxf(mx, dot);
-    }
+    const uint32_t u = __float_as_uint(gamma[j]);
+    const float mx = __uint_as_float((u & 0x80000000u) ? u & 0x7FFFFFFFu : ~u);
     gamma[j] = (mx > -INFINITY) ? acosf_det(fminf(fmaxf(mx, 0.0f), 1.0f)) : 3.14159265358979323846f;
 }
 
@@ -354,7 +444,7 @@ __global__ void rv_adapt(const float* __restrict__ v0, const float* __restrict__
 struct RLayout {
     float* fm; float* cvm; float* tf; float* part_cos; int32_t* part_idx;
     uint64_t* k0; uint64_t* k1; int32_t* v0; int32_t* v1;
-    uint64_t* t0; uint64_t* t1; int32_t* tv0; int32_t* tv1; uint8_t* win; uint8_t* flag;
+    uint64_t* t0; uint64_t* t1; int32_t* tv0; int32_t* tv1; uint8_t* win; uint32_t* bits;
     int32_t* chosen; int32_t* meta; void* sort_tmp; size_t sort_bytes;
 };
 
@@ -372,7 +462,8 @@ RLayout rcarve(int n, int m, int k, Carve& c)
     L.v0 = c.take<int32_t>(nm); L.v1 = c.take<int32_t>(nm);
     L.t0 = c.take<uint64_t>(nm); L.t1 = c.take<uint64_t>(nm);
     L.tv0 = c.take<int32_t>(nm); L.tv1 = c.take<int32_t>(nm);
-    L.win = c.take<uint8_t>(nm); L.flag = c.take<uint8_t>(nm);
+    L.win = c.take<uint8_t>(nm);
+    L.bits = c.take<uint32_t>((static_cast<size_t>(nm) + 31) / 32);
     L.chosen = c.take<int32_t>(n);
     L.meta = c.take<int32_t>(kRLen);
     L.sort_bytes = sort_pairs_temp_bytes(nm);
@@ -421,8 +512,13 @@ int rvea_select(const moea_rvea_select_args& A)
                        L.win);
     MOEA_HIP(hipGetLastError());
     MOEA_CHECK(sort_pairs(L.sort_tmp, L.sort_bytes, L.t0, L.t1, L.tv0, L.tv1, nm, st));
-    hipLaunchKernelGGL(rv_choose, dim3(1), dim3(kScan), 0, st, L.win, nm, n, L.tv1, L.v1, L.flag,
-                       L.chosen, L.meta);
+    const size_t set_bytes = (static_cast<size_t>(nm) + 31) / 32 * 4;
+    if (set_bytes <= kChooseMaxLds)
+        hipLaunchKernelGGL(rv_choose<true>, dim3(1), dim3(kScan), set_bytes, st, L.win, nm, n, L.tv1, L.v1, L.bits,
+                           L.chosen, L.meta);
+    else
+        hipLaunchKernelGGL(rv_choose<false>, dim3(1), dim3(kScan), 0, st, L.win, nm, n, L.tv1, L.v1, L.bits, L.chosen,
+                           L.meta);
     hipLaunchKernelGGL(rv_gather, dim3(ceil_div(n, 4)), dim3(256), 0, st, L.chosen, L.meta, n, d, m,
                        A.parents.x, A.offspring.x, L.fm, L.cvm, A.next.x, A.next.f, A.next.cv,
                        A.out_active);
@@ -433,8 +529,14 @@ int rvea_select(const moea_rvea_select_args& A)
 int rvea_gamma(const float* v, int m, int k, float* gamma, hipStream_t stream)
 {
     if (!v || !gamma || m <= 0 || m > kMaxM || k <= 0) return fail(kInvalidArgument, "rvea_gamma: invalid arguments");
-    const dim3 g(ceil_div(k, 256)), b(256);
-    MOEA_LAUNCH_M(m, rv_gamma, g, b, 0, stream, v, k, gamma);
+    // about 1024 workgroups, at least 32 directions q each
+    const int rows = ceil_div(k, kGammaRows);
+    const int per = std::max(32, ceil_div(ceil_div(k, std::max(1, 1024 / rows)), kGammaGroup) * kGammaGroup);
+    uint32_t* key = reinterpret_cast<uint32_t*>(gamma);
+    const dim3 g(ceil_div(k, 256)), gt(rows, ceil_div(k, per)), b(256);
+    hipLaunchKernelGGL(rv_gamma_init, g, b, 0, stream, key, k);
+    MOEA_LAUNCH_M(m, rv_gamma_tiles, gt, b, 0, stream, v, k, per, key);
+    hipLaunchKernelGGL(rv_gamma_finish, g, b, 0, stream, gamma, k);
     MOEA_HIP(hipGetLastError());
     return kOk;
 }
