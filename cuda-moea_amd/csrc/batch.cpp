@@ -30,7 +30,6 @@ namespace moea {
 
 namespace {
 
-constexpr int kAssocChunkB = 1024;   // association chunk (directions per LDS stage)
 constexpr int kStateFree = 0, kStateRunning = 1, kStateAdmitted = 2, kStateFinished = 3;
 
 int bitlen(long long v)
@@ -41,7 +40,7 @@ int bitlen(long long v)
 }
 
 struct InstSizes {
-    int n, m, d, k, nm, W, Wc, npad, nchunks, nb, hidden;
+    int n, m, d, k, nm, W, Wc, npad, nb, hidden;
 };
 
 InstSizes sizes_of(const moea_batch_problem& p)
@@ -52,7 +51,6 @@ InstSizes sizes_of(const moea_batch_problem& p)
     z.W = ceil_div(z.nm, 64);
     z.Wc = ceil_div(z.W, 8);
     z.npad = z.W * 64;
-    z.nchunks = ceil_div(p.k, kAssocChunkB);
     z.nb = ceil_div(z.nm, 256);
     z.hidden = (p.problem == MOEA_PROBLEM_MLP) ? p.hidden : 0;
     return z;
@@ -82,8 +80,6 @@ void carve_instance(Carve& c, const moea_batch_problem& p, BInst& I)
     I.asf_idx = c.take<int32_t>(static_cast<size_t>(z.nb) * z.m);
     I.row_max = c.take<float>(static_cast<size_t>(z.nb) * z.m);
     I.a = c.take<float>(kMaxM);
-    I.part_d2 = c.take<float>(static_cast<size_t>(z.nchunks) * z.nm);
-    I.part_idx = c.take<int32_t>(static_cast<size_t>(z.nchunks) * z.nm);
     I.dist = c.take<float>(z.nm);
     I.ref = c.take<int32_t>(z.nm);
     I.rho = c.take<int32_t>(z.k);
@@ -124,7 +120,6 @@ void fill_record(const moea_batch_problem& p, BInst& I)
     I.n = z.n; I.m = z.m; I.d = z.d; I.k = z.k;
     I.nm = z.nm; I.W = z.W; I.Wc = z.Wc; I.npad = z.npad;
     I.max_gen = p.max_generations;
-    I.nchunks = z.nchunks;
     I.ddiv = fast_div_make(static_cast<uint32_t>(z.d));
     I.seed = p.seed;
     I.sbx_eta0 = p.sbx_eta[0]; I.sbx_eta1 = p.sbx_eta[1];
@@ -246,7 +241,7 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
         }
         prep[m][i] = nb;
         if (I.cones) apr[m][i] = ceil_div(nm, 4);
-        else assoc[m][i] = static_cast<long long>(nb) * I.nchunks;
+        else assoc[m][i] = ceil_div(nm, 64);
         n0_rows[i] = ceil_div(n, 256);
         n0_prep[i] = static_cast<long long>(Wc0) * m;
         dom0[m][i] = static_cast<long long>(Wc0) * ceil_div(W0, kBatchDomSeg);

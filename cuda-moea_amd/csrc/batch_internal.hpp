@@ -20,7 +20,7 @@
 namespace moea {
 
 constexpr int kBatchPeelStateWords = 1024 + 64;   // per instance: peel group barrier flags and totals
-constexpr int kBatchDomSeg = 64;                   // row blocks per dominance workgroup
+constexpr int kBatchDomSeg = 16;                   // row blocks per dominance workgroup
 constexpr int kBatchPeelMaxLds = 80 * 1024;        // LDS bound of one batched peel block
 
 struct BInst {
@@ -31,7 +31,6 @@ struct BInst {
     int n, m, d, k;
     int nm, W, Wc, npad;          // NDS over the 2n merged rows
     int max_gen;
-    int nchunks;                  // association chunks of 1024 directions
     FastDiv ddiv;                 // division by d (reproduction element indices)
     uint64_t seed;
     float sbx_eta0, sbx_eta1, sbx_prob, sbx_copy, pm_eta0, pm_eta1, pm_prob;
@@ -62,8 +61,6 @@ struct BInst {
     int32_t* asf_idx;             // (ceil(nm / 256), m)
     float* row_max;               // (ceil(nm / 256), m)
     float* a;                     // (kMaxM)
-    float* part_d2;               // (nchunks, nm)
-    int32_t* part_idx;            // (nchunks, nm)
     float* dist;                  // (nm)
     int32_t* ref;                 // (nm)
     int32_t* rho;                 // (k)
@@ -146,7 +143,7 @@ struct BSelGrids {
     BGrid rows4;                  // n rows per instance, one wave per row
     BGrid objectives;             // one 1024-thread block per objective per instance
     BGrid norm_prep[kMaxM + 1];   // ceil(2n / 256) blocks, instances with m objectives
-    BGrid assoc[kMaxM + 1];       // ceil(2n / 256) x association chunks, instances with m objectives
+    BGrid assoc[kMaxM + 1];       // ceil(2n / 64) blocks, instances with m objectives and no cone tables
     BGrid assoc_pruned[kMaxM + 1];// ceil(2n / 4), instances with m objectives and cone tables
     int ref_bits;                 // bits of a direction index (with the two sentinels)
     int rank_bits;                // bits of rho + rank (with the sentinel)

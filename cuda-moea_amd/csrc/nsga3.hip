@@ -591,85 +591,94 @@ __global__ __launch_bounds__(kSolveThreads) void norm_solve(const float* __restr
     norm_solve_body(fn, nm, m, asf_val, asf_idx, row_max, meta, a_out, gidx, out_ext, out_a);
 }
 
-// Perpendicular-distance association, one individual per thread against a
-// chunk of directions staged in LDS (association.cu:85-188): dot by an fmaf
-// chain, residual x - dot*w as one fma, d2 by an fmaf chain, first minimum
-// wins.  Grid: (ceil(2n/256), ceil(K/kAssocChunk)).
-constexpr int kAssocChunk = 1024;
+// Perpendicular-distance association against every direction
+// (association.cu:85-188, 397-447): dot by an fmaf chain, residual x - dot*w as
+// one fma, d2 by an fmaf chain, the smallest d2 and of equal ones the first
+// direction.  A workgroup takes 64 individuals, a lane each, and its 16 waves a
+// sixteenth of the directions each, read as scalars (all lanes look at the same
+// direction), so nothing but the waves' minima passes through LDS.  rho
+// (optional): prior-front individuals add one to their direction's count
+// (prior_histogram_kernel, niching.cu:21-33).
+//
+// Bound: VALU, 3M + 3 instructions a pair.  Cutting the directions over the
+// waves of a workgroup, rather than over workgroups in chunks of 1024 with a
+// second kernel for their partial minima, fills the chip from a few thousand
+// individuals on: 50 us -> 14 us at 2048 individuals and 990 directions, M = 3.
+constexpr int kAssocThreads = 1024;
+constexpr int kAssocWaves = kAssocThreads / 64;
 
 template <int M>
-__device__ __forceinline__ void assoc_partial_body(const float* __restrict__ fn, int nm, const float* __restrict__ a,
-                                          const float* __restrict__ w, int k, const int32_t* __restrict__ meta,
-                                          float* __restrict__ part_d2, int32_t* __restrict__ part_idx, int bx,
-                                          int by)
+__device__ __forceinline__ void assoc_all_body(const float* __restrict__ fn, int nm, const float* __restrict__ a,
+                                               const float* __restrict__ w, int k, const int32_t* __restrict__ meta,
+                                               float* __restrict__ dist, int32_t* __restrict__ ref,
+                                               int32_t* __restrict__ rho, int bx)
 {
-    __shared__ float s_w[M][kAssocChunk];
+    constexpr int G = (M <= 5) ? 8 : 4;       // directions per group of scalar loads
+    __shared__ float s_d[kAssocWaves][64];
+    __shared__ int s_j[kAssocWaves][64];
     if (meta[kNRem] <= 0) return;
-    const int n_nds = meta[kNPrior] + meta[kNLast];
-    if (bx * 256 >= n_nds) return;
-    const int j0 = by * kAssocChunk;
-    const int jn = min(kAssocChunk, k - j0);
-    for (int e = threadIdx.x; e < M * kAssocChunk; e += 256) {
-        const int c = e / kAssocChunk, j = e % kAssocChunk;
-        s_w[c][j] = (j < jn) ? w[static_cast<size_t>(c) * k + j0 + j] : 0.0f;
-    }
-    __syncthreads();
-    const int i = bx * 256 + threadIdx.x;
-    if (i >= n_nds) return;
+    const int n_prior = meta[kNPrior];
+    const int n_nds = n_prior + meta[kNLast];
+    if (bx * 64 >= n_nds) return;
+    const int lane = static_cast<int>(threadIdx.x & 63);
+    const int wave = wave_uniform(static_cast<int>(threadIdx.x >> 6));
+    const int i = bx * 64 + lane;
     float x[M];
 #pragma unroll
-    for (int c = 0; c < M; ++c) x[c] = fn[static_cast<size_t>(c) * nm + i] * a[c];
+    for (int c = 0; c < M; ++c) x[c] = fn[static_cast<size_t>(c) * nm + min(i, n_nds - 1)] * a[c];
+    const int per = ((k + kAssocWaves - 1) / kAssocWaves + G - 1) / G * G;
+    const int j0 = wave * per, j1 = min(k, j0 + per);
     float best = INFINITY;
     int bj = -1;
-    for (int j = 0; j < jn; ++j) {
+    const auto one = [&](int j, const float (&u)[M]) {
         float dot = 0.0f;
 #pragma unroll
-        for (int c = 0; c < M; ++c) dot = fmaf(x[c], s_w[c][j], dot);
+        for (int c = 0; c < M; ++c) dot = fmaf(x[c], u[c], dot);
         float d2 = 0.0f;
 #pragma unroll
         for (int c = 0; c < M; ++c) {
-            const float r = fmaf(-dot, s_w[c][j], x[c]);
+            const float r = fmaf(-dot, u[c], x[c]);
             d2 = fmaf(r, r, d2);
         }
-        if (d2 < best) { best = d2; bj = j0 + j; }
+        if (d2 < best) { best = d2; bj = j; }
+    };
+    int j = j0;
+    for (; j + G <= j1; j += G) {
+        float u[G][M];
+#pragma unroll
+        for (int c = 0; c < M; ++c)
+#pragma unroll
+            for (int t = 0; t < G; ++t) u[t][c] = ld_uniform(w, static_cast<size_t>(c) * k + j + t);
+#pragma unroll
+        for (int t = 0; t < G; ++t) one(j + t, u[t]);
     }
-    part_d2[static_cast<size_t>(by) * nm + i] = best;
-    part_idx[static_cast<size_t>(by) * nm + i] = bj;
+    for (; j < j1; ++j) {
+        float u[M];
+#pragma unroll
+        for (int c = 0; c < M; ++c) u[c] = ld_uniform(w, static_cast<size_t>(c) * k + j);
+        one(j, u);
+    }
+    s_d[wave][lane] = best;
+    s_j[wave][lane] = bj;
+    __syncthreads();
+    if (wave != 0 || i >= n_nds) return;
+    // the waves' directions ascend: the first of equal minima is the smallest index
+    for (int v = 1; v < kAssocWaves; ++v)
+        if (s_d[v][lane] < best) { best = s_d[v][lane]; bj = s_j[v][lane]; }
+    dist[i] = (best != INFINITY) ? sqrtf(best) : INFINITY;
+    ref[i] = bj;
+    if (rho && bj >= 0 && i < n_prior) atomicAdd(&rho[bj], 1);
 }
 
 template <int M>
-__global__ __launch_bounds__(256) void associate_partial(const float* __restrict__ fn, int nm,
-                                                         const float* __restrict__ a,
-                                                         const float* __restrict__ w, int k,
-                                                         const int32_t* __restrict__ meta,
-                                                         float* __restrict__ part_d2,
-                                                         int32_t* __restrict__ part_idx)
+__global__ __launch_bounds__(kAssocThreads) void associate_all(const float* __restrict__ fn, int nm,
+                                                               const float* __restrict__ a,
+                                                               const float* __restrict__ w, int k,
+                                                               const int32_t* __restrict__ meta,
+                                                               float* __restrict__ dist, int32_t* __restrict__ ref,
+                                                               int32_t* __restrict__ rho)
 {
-    assoc_partial_body<M>(fn, nm, a, w, k, meta, part_d2, part_idx, static_cast<int>(blockIdx.x),
-                          static_cast<int>(blockIdx.y));
-}
-
-// Reduce the chunk partials in chunk order (association_phase2_kernel, :397-447).
-// rho (optional): prior-front individuals add one to their direction's count
-// (prior_histogram_kernel, niching.cu:21-33).
-__device__ __forceinline__ void assoc_final_body(const float* __restrict__ part_d2, const int32_t* __restrict__ part_idx,
-                                        int nchunks, int nm, const int32_t* __restrict__ meta,
-                                        float* __restrict__ dist, int32_t* __restrict__ ref, int i,
-                                        int32_t* __restrict__ rho = nullptr)
-{
-    if (meta[kNRem] <= 0) return;
-    const int n_nds = meta[kNPrior] + meta[kNLast];
-    if (i >= n_nds) return;
-    float best = INFINITY;
-    int bj = -1;
-    for (int c = 0; c < nchunks; ++c) {
-        const float d = part_d2[static_cast<size_t>(c) * nm + i];
-        const int idx = part_idx[static_cast<size_t>(c) * nm + i];
-        if (d < best || (d == best && idx >= 0 && idx < bj)) { best = d; bj = idx; }
-    }
-    dist[i] = (best != INFINITY) ? sqrtf(best) : INFINITY;
-    ref[i] = bj;
-    if (rho && bj >= 0 && i < meta[kNPrior]) atomicAdd(&rho[bj], 1);
+    assoc_all_body<M>(fn, nm, a, w, k, meta, dist, ref, rho, static_cast<int>(blockIdx.x));
 }
 
 // ------------------------------------------------------ pruned association --
@@ -982,14 +991,6 @@ __global__ __launch_bounds__(256) void associate_pruned(const float* __restrict_
     const int i = static_cast<int>(blockIdx.x) * 4 + wave;
     if (i >= n_nds) return;
     assoc_pruned_body<M>(fn, nm, a, wp, k, perm, cones, meta, dist, ref, i, s_list[wave], rho);
-}
-
-__global__ void associate_final(const float* __restrict__ part_d2, const int32_t* __restrict__ part_idx,
-                                int nchunks, int nm, const int32_t* __restrict__ meta,
-                                float* __restrict__ dist, int32_t* __restrict__ ref, int32_t* __restrict__ rho)
-{
-    assoc_final_body(part_d2, part_idx, nchunks, nm, meta, dist, ref,
-                     static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x), rho);
 }
 
 // Buffers of the cone preparation: direction keys and permutation, the sort
@@ -1899,7 +1900,7 @@ __global__ void quantize_cv_kernel(const float* __restrict__ cv, float* __restri
 struct Layout {
     float* fm; float* cvm; float* cvq; int32_t* fronts; int32_t* meta; int32_t* gidx; float* fn;
     float* asf_val; int32_t* asf_idx; float* row_max; float* a; float* omin;
-    float* part_d2; int32_t* part_idx; float* dist; int32_t* ref; int32_t* rho; ConeBufs cones;
+    float* dist; int32_t* ref; int32_t* rho; ConeBufs cones;
     uint64_t* k0; uint64_t* k1; int32_t* v0; int32_t* v1; void* sort_tmp; size_t sort_bytes;
     uint8_t* flag; int32_t* chosen; int32_t* counts; void* nds_ws; size_t nds_bytes;
 };
@@ -1908,7 +1909,6 @@ Layout carve(void* ws, size_t cap, int n, int m, int k, Carve& c)
 {
     const int nm = 2 * n;
     const int nb = ceil_div(nm, 256);
-    const int nchunks = ceil_div(k, kAssocChunk);
     Layout L{};
     L.fm = c.take<float>(static_cast<size_t>(m) * nm);
     L.cvm = c.take<float>(nm);
@@ -1922,8 +1922,6 @@ Layout carve(void* ws, size_t cap, int n, int m, int k, Carve& c)
     L.row_max = c.take<float>(static_cast<size_t>(nb) * m);
     L.a = c.take<float>(kMaxM);
     L.omin = c.take<float>(static_cast<size_t>(nb) * m);
-    L.part_d2 = c.take<float>(static_cast<size_t>(nchunks) * nm);
-    L.part_idx = c.take<int32_t>(static_cast<size_t>(nchunks) * nm);
     L.dist = c.take<float>(nm);
     L.ref = c.take<int32_t>(nm);
     L.rho = c.take<int32_t>(k);
@@ -2022,27 +2020,24 @@ __global__ void assoc_meta(int32_t* __restrict__ meta, int n)
 }
 
 struct AssocLayout {
-    int32_t* meta; ConeBufs cones; float* part_d2; int32_t* part_idx;
+    int32_t* meta; ConeBufs cones;
 };
 
-AssocLayout carve_assoc(Carve& c, int n, int m, int k)
+AssocLayout carve_assoc(Carve& c, int m, int k)
 {
     AssocLayout L{};
     L.meta = c.take<int32_t>(kMetaLen);
     L.cones = carve_cones(c, m, k);
-    L.part_d2 = c.take<float>(static_cast<size_t>(ceil_div(k, kAssocChunk)) * n);
-    L.part_idx = c.take<int32_t>(static_cast<size_t>(ceil_div(k, kAssocChunk)) * n);
     return L;
 }
 
 }  // namespace
 
-// The brute-force partials are strided by the leading dimension: size by ld.
 size_t associate_workspace_bytes(int ld, int m, int k)
 {
     if (ld <= 0 || m <= 0 || m > kMaxM || k <= 0) return 0;
     Carve c(nullptr, 0);
-    carve_assoc(c, ld, m, k);
+    carve_assoc(c, m, k);
     return c.used;
 }
 
@@ -2055,7 +2050,7 @@ int associate(const float* fn, int ld, int n, int m, const float* a, const float
     const size_t need = associate_workspace_bytes(ld, m, k);
     if (!ws || ws_bytes < need) return fail(kWorkspaceTooSmall, "associate: workspace too small");
     Carve c(ws, ws_bytes);
-    const AssocLayout L = carve_assoc(c, ld, m, k);
+    const AssocLayout L = carve_assoc(c, m, k);
     const int nbk = ceil_div(k, 64);
     const bool prunable = nbk <= kConeMaxBlocks;
     if (method == 2 && !prunable) return fail(kUnsupported, "associate: too many directions for the pruned path");
@@ -2067,11 +2062,8 @@ int associate(const float* fn, int ld, int n, int m, const float* a, const float
         MOEA_LAUNCH_M(m, associate_pruned, dim3(ceil_div(n, 4)), b256, 0, st, fn, ld, a, L.cones.wp, k,
                       L.cones.perm, L.cones.cones, L.meta, dist, ref, nullptr);
     } else {
-        const int nchunks = ceil_div(k, kAssocChunk);
-        MOEA_LAUNCH_M(m, associate_partial, dim3(ceil_div(n, 256), nchunks), b256, 0, st, fn, ld, a, w, k, L.meta,
-                      L.part_d2, L.part_idx);
-        hipLaunchKernelGGL(associate_final, dim3(ceil_div(n, 256)), b256, 0, st, L.part_d2, L.part_idx, nchunks, ld,
-                           L.meta, dist, ref, nullptr);
+        MOEA_LAUNCH_M(m, associate_all, dim3(ceil_div(n, 64)), dim3(kAssocThreads), 0, st, fn, ld, a, w, k, L.meta,
+                      dist, ref, nullptr);
     }
     MOEA_HIP(hipGetLastError());
     return kOk;
@@ -2116,7 +2108,6 @@ int nsga3_select(const moea_nsga3_select_args& A)
     hipStream_t st = static_cast<hipStream_t>(A.stream);
     const int nm = 2 * n;
     const int nb = ceil_div(nm, 256);
-    const int nchunks = ceil_div(k, kAssocChunk);
     const uint32_t gen = static_cast<uint32_t>(A.generation);
     const moea_draws* dr = A.draws;
 
@@ -2141,7 +2132,7 @@ int nsga3_select(const moea_nsga3_select_args& A)
     hipLaunchKernelGGL(front_counts, dim3(nsb), dim3(kScanThreads), 0, st, L.fronts, nm, L.meta, L.counts);
     hipLaunchKernelGGL(front_scatter, dim3(nsb), dim3(kScanThreads), 0, st, L.fronts, nm, n, L.counts, nsb,
                        L.gidx, L.meta, L.flag);
-    const dim3 g_nb(nb), b256(256), g_assoc(nb, nchunks);
+    const dim3 g_nb(nb), b256(256);
     MOEA_LAUNCH_M(m, norm_prep, g_nb, b256, 0, st, L.fm, nm, L.gidx, L.meta, L.fn, L.asf_val, L.asf_idx,
                   L.row_max, L.rho, k, L.omin, nb, A.ideal);
     hipLaunchKernelGGL(norm_solve, dim3(1), dim3(kSolveThreads), 0, st, L.fn, nm, m, L.asf_val,
@@ -2153,10 +2144,8 @@ int nsga3_select(const moea_nsga3_select_args& A)
         MOEA_LAUNCH_M(m, associate_pruned, dim3(ceil_div(nm, 4)), b256, 0, st, L.fn, nm, L.a, L.cones.wp, k,
                       L.cones.perm, L.cones.cones, L.meta, L.dist, L.ref, L.rho);
     } else {
-        MOEA_LAUNCH_M(m, associate_partial, g_assoc, b256, 0, st, L.fn, nm, L.a, A.directions, k,
-                      L.meta, L.part_d2, L.part_idx);
-        hipLaunchKernelGGL(associate_final, dim3(nb), dim3(256), 0, st, L.part_d2, L.part_idx, nchunks,
-                           nm, L.meta, L.dist, L.ref, L.rho);
+        MOEA_LAUNCH_M(m, associate_all, dim3(ceil_div(nm, 64)), dim3(kAssocThreads), 0, st, L.fn, nm, L.a,
+                      A.directions, k, L.meta, L.dist, L.ref, L.rho);
     }
     stage_end(kStAssociation, st);
     stage_begin(kStNiching, st);
@@ -2239,28 +2228,26 @@ __global__ __launch_bounds__(kScanThreads) void b_split(const BInst* __restrict_
         }
         return;
     }
-    int tp = 0, tl = 0;
-    for (int base = 0; base < I.nm; base += kScanThreads) {
-        const int t = base + static_cast<int>(threadIdx.x);
-        const int fr = t < I.nm ? I.fronts_mix[t] : -1;
-        int cp, cl;
-        block_exclusive_scan((fr >= 0 && fr < mf) ? 1 : 0, s_wave, cp);
-        block_exclusive_scan((fr == mf) ? 1 : 0, s_wave, cl);
-        tp += cp;
-        tl += cl;
+    int cp = 0, cl = 0, tp, tl;
+    for (int t = static_cast<int>(threadIdx.x); t < I.nm; t += kScanThreads) {
+        const int fr = I.fronts_mix[t];
+        cp += (fr >= 0 && fr < mf) ? 1 : 0;
+        cl += (fr == mf) ? 1 : 0;
     }
+    block_exclusive_scan(cp, s_wave, tp);
+    block_exclusive_scan(cl, s_wave, tl);
     int op = 0, ol = 0;
     for (int base = 0; base < I.nm; base += kScanThreads) {
         const int t = base + static_cast<int>(threadIdx.x);
         const int fr = t < I.nm ? I.fronts_mix[t] : -1;
         const int fp = (fr >= 0 && fr < mf) ? 1 : 0, fl = (fr == mf) ? 1 : 0;
-        int cp, cl;
-        const int ep = block_exclusive_scan(fp, s_wave, cp);
-        const int el = block_exclusive_scan(fl, s_wave, cl);
-        if (fp) I.gidx[op + ep] = t;
-        if (fl) I.gidx[tp + ol + el] = t;
-        op += cp;
-        ol += cl;
+        // both positions from one scan: a chunk's counts fit 16 bits each
+        int c;
+        const int e = block_exclusive_scan(fp | (fl << 16), s_wave, c);
+        if (fp) I.gidx[op + (e & 0xFFFF)] = t;
+        if (fl) I.gidx[tp + ol + (e >> 16)] = t;
+        op += c & 0xFFFF;
+        ol += c >> 16;
     }
     if (threadIdx.x == 0) {
         I.meta[kNPrior] = tp;
@@ -2288,6 +2275,9 @@ __global__ __launch_bounds__(256) void b_norm_prep(const BInst* __restrict__ ins
     int local;
     const int i = bmap_find(mp, static_cast<int>(blockIdx.x), local);
     const BInst& I = insts[i];
+    // the niche counts start at zero (the association adds the prior front)
+    const int nb = (I.nm + 255) / 256;
+    for (int j = local * 256 + static_cast<int>(threadIdx.x); j < I.k; j += nb * 256) I.rho[j] = 0;
     norm_prep_body<M>(I.fm, I.nm, I.gidx, I.ideal, I.meta, I.fn, I.asf_val, I.asf_idx, I.row_max, local);
 }
 
@@ -2299,13 +2289,12 @@ __global__ __launch_bounds__(kSolveThreads) void b_norm_solve(const BInst* __res
 }
 
 template <int M>
-__global__ __launch_bounds__(256) void b_assoc_partial(const BInst* __restrict__ insts, BMap mp)
+__global__ __launch_bounds__(kAssocThreads) void b_assoc_all(const BInst* __restrict__ insts, BMap mp)
 {
     int local;
     const int i = bmap_find(mp, static_cast<int>(blockIdx.x), local);
     const BInst& I = insts[i];
-    const int nbx = (I.nm + 255) / 256;
-    assoc_partial_body<M>(I.fn, I.nm, I.a, I.dirs, I.k, I.meta, I.part_d2, I.part_idx, local % nbx, local / nbx);
+    assoc_all_body<M>(I.fn, I.nm, I.a, I.dirs, I.k, I.meta, I.dist, I.ref, I.rho, local);
 }
 
 // One wave per individual of the instances with cone tables.
@@ -2322,32 +2311,7 @@ __global__ __launch_bounds__(256) void b_assoc_pruned(const BInst* __restrict__ 
     const int p = local * 4 + wave;
     if (p >= n_nds) return;
     assoc_pruned_body<M>(I.fn, I.nm, I.a, I.wp, I.k, I.cperm, I.cones, I.meta, I.dist, I.ref, p, s_list[wave],
-                         nullptr);
-}
-
-__global__ void b_assoc_final(const BInst* __restrict__ insts, BMap mp)
-{
-    int local;
-    const int i = bmap_find(mp, static_cast<int>(blockIdx.x), local);
-    const BInst& I = insts[i];
-    if (I.cones) return;                       // associated by b_assoc_pruned
-    const int t = local * 256 + static_cast<int>(threadIdx.x);
-    if (t < I.nm) assoc_final_body(I.part_d2, I.part_idx, I.nchunks, I.nm, I.meta, I.dist, I.ref, t);
-}
-
-// rho_prior of one instance per workgroup (rho_clear + rho_hist).
-__global__ __launch_bounds__(1024) void b_rho(const BInst* __restrict__ insts)
-{
-    const BInst& I = insts[blockIdx.x];
-    if (I.state != 1) return;
-    for (int j = threadIdx.x; j < I.k; j += blockDim.x) I.rho[j] = 0;
-    __syncthreads();
-    if (I.meta[kNRem] <= 0) return;
-    const int n_prior = I.meta[kNPrior];
-    for (int t = threadIdx.x; t < n_prior; t += blockDim.x) {
-        const int r = I.ref[t];
-        if (r >= 0 && r < I.k) atomicAdd(&I.rho[r], 1);
-    }
+                         I.rho);
 }
 
 __global__ void b_niche_keys1(const BInst* __restrict__ insts, BMap mp, int ref_bits, uint64_t* __restrict__ keys,
@@ -2506,20 +2470,17 @@ int batch_select(const BatchLaunch& L, const BSelGrids& G, const BNdsGrids& NG, 
     stage_begin(kStAssociation, st);
     for (int m = 1; m <= kMaxM; ++m) {
         if (G.assoc[m].blocks <= 0) continue;
-        const dim3 grid(G.assoc[m].blocks), block(256);
-        MOEA_LAUNCH_M(m, b_assoc_partial, grid, block, 0, st, L.insts, G.assoc[m].map);
+        const dim3 grid(G.assoc[m].blocks), block(kAssocThreads);
+        MOEA_LAUNCH_M(m, b_assoc_all, grid, block, 0, st, L.insts, G.assoc[m].map);
     }
     for (int m = 1; m <= kMaxM; ++m) {
         if (G.assoc_pruned[m].blocks <= 0) continue;
         const dim3 grid(G.assoc_pruned[m].blocks), block(256);
         MOEA_LAUNCH_M(m, b_assoc_pruned, grid, block, 0, st, L.insts, G.assoc_pruned[m].map);
     }
-    hipLaunchKernelGGL(b_assoc_final, dim3(G.merged256.blocks), dim3(256), 0, st, L.insts, G.merged256.map);
     MOEA_HIP(hipGetLastError());
     stage_end(kStAssociation, st);
     stage_begin(kStNiching, st);
-    hipLaunchKernelGGL(b_rho, dim3(L.count), dim3(1024), 0, st, L.insts);
-    MOEA_HIP(hipGetLastError());
     // one workgroup per instance while every instance is small (2n <= 8192);
     // larger runs (many objectives put most of 2n in the last front) sort
     // faster device-wide
