@@ -340,39 +340,53 @@ __device__ __forceinline__ double readlane_f64(double v, int lane)
     return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
 }
 
-// LDS of the one-wave hyperplane solve: A and V row-major (kMaxM x kMaxM),
-// three sum rows, and the column weights.
+// LDS of the one-wave hyperplane solve: A and V column by column (column p at
+// p * kMaxM), the pairs of each residue, and the column weights.
 struct SolveLds {
     double a[kMaxM * kMaxM];
     double v[kMaxM * kMaxM];
-    double sums[3][16];
     double w[kMaxM];
     int skip[kMaxM];
+    int pair[kMaxM][kMaxM / 2];   // p | q << 8 with (p + q) mod m = residue, or -1
 };
 
-// hyperplane_fp64 (common.hpp) on one wave, bit-identical to it: the same
-// rotation sequence, every element update the same expression, every sum
-// accumulated in the same order.  Lane i < m updates row i of A and V (in
-// LDS); each rotation's three column sums are taken by lanes 0, 1, 2, each
-// summing its row of products in order, and broadcast by lane reads; the
-// rotation parameters are then computed redundantly by every lane.  The
-// singular values and weights are computed by lane j for column j.  The code
-// is a compact loop: a fully unrolled 10 x 10 sweep does not fit the
-// instruction cache once other kernels' code shares it, and then runs several
-// times slower.  Returns 1 for the row-max fallback (the scalar solve's
-// conditions); lane r < m gets a_out[r] in `a_lane`.
+// hyperplane_fp64 (common.hpp) on one wave, bit-identical to it: every element
+// update the same expression, every sum accumulated in the same order.  The
+// scalar sweep takes the pairs (0,1), (0,2), .., (1,2), .. one after another,
+// but a rotation reads and writes its own two columns only, so it need wait
+// only for the earlier ones that share a column.  Pair (p, q) of sweep s runs at
+// step s m + p + q: every earlier rotation of columns p and q, of this sweep
+// and the last, has a smaller step, and the pairs of a step, those with
+// (p + q) mod m = step mod m (p + q >= m: still of the sweep before), are
+// disjoint.  So a sweep of m (m - 1) / 2 rotations takes m steps of up to m / 2
+// rotations: lane g m + i works on row i of the step's pair g, every lane of a
+// pair forming the three sums and the rotation for itself from the two columns
+// in LDS.  What limits it is the chain of three divisions and two roots in
+// double of each step, about 0.4 us.  When a sweep ends without a rotation, the
+// next one's first steps have run already: they met the same columns and
+// rotated nothing.  The code is a compact loop: a fully unrolled 10 x 10 sweep
+// does not fit the instruction cache once other kernels' code shares it, and
+// then runs several times slower.  One rotation at a time took 182 us at M = 10
+// (N = 8190), this 76 us.  kCols: an even bound of m.  Returns 1 for the row-max fallback (the scalar
+// solve's conditions); lane r < m gets a_out[r] in `a_lane`.
+template <int kCols>
 __device__ __forceinline__ int hyperplane_fp64_wave(int m, SolveLds& L, double& a_lane)
 {
     const int lane = static_cast<int>(threadIdx.x & 63);
     const bool own = lane < m;
-    double* ra = L.a + lane * kMaxM;
-    double* rv = L.v + lane * kMaxM;
     bool bad = false;
-    if (own)
+    if (own) {
         for (int j = 0; j < m; ++j) {
-            bad = bad || !isfinite(ra[j]);
-            rv[j] = (lane == j) ? 1.0 : 0.0;
+            bad = bad || !isfinite(L.a[j * kMaxM + lane]);
+            L.v[j * kMaxM + lane] = (lane == j) ? 1.0 : 0.0;
         }
+        int g = 0;
+        for (int p = 0; p < m; ++p) {
+            const int q = lane >= p ? lane - p : lane - p + m;
+            if (p < q) L.pair[lane][g++] = p | (q << 8);
+        }
+        for (; g < kMaxM / 2; ++g) L.pair[lane][g] = -1;
+    }
     if (__ballot(bad)) return 1;
     // Two equal rows (the same individual extreme on two axes, as a rule at
     // M >= 8) make the result the fallback whatever the sweeps do: rotations
@@ -385,50 +399,71 @@ __device__ __forceinline__ int hyperplane_fp64_wave(int m, SolveLds& L, double& 
     if (own)
         for (int i = 0; i < lane; ++i) {
             bool eq = true;
-            for (int j = 0; j < m; ++j) eq = eq && (L.a[i * kMaxM + j] == ra[j]);
+            for (int j = 0; j < m; ++j) eq = eq && (L.a[j * kMaxM + i] == L.a[j * kMaxM + lane]);
             dup = dup || eq;
         }
     if (__ballot(dup)) return 1;
-    int converged = 0;
-    for (int sweep = 0; sweep < 60 && !converged; ++sweep) {
-        int rotated = 0;
-        for (int p = 0; p < m - 1; ++p) {
-            for (int q = p + 1; q < m; ++q) {
-                const double ap = own ? ra[p] : 0.0, aq = own ? ra[q] : 0.0;
-                if (own) {
-                    L.sums[0][lane] = ap * ap;
-                    L.sums[1][lane] = aq * aq;
-                    L.sums[2][lane] = ap * aq;
-                }
-                __builtin_amdgcn_wave_barrier();
-                double acc = 0.0;
-                if (lane < 3) {
-                    double t[kMaxM];
+    const int grp = lane / m, row = lane - grp * m;
+    int converged = m < 2 ? 1 : 0;
+    bool rot_now = false, rot_last = false;      // a rotation of this sweep, of the last
+    for (int sweep = 0; !converged; ++sweep) {
+        // sweep s ends in block s + 1 (m = 2: in its own block)
+        bool stop = false;
+        for (int r = 0; r < m; ++r) {
+            const int pq = grp < m / 2 ? L.pair[r][grp] : -1;
+            const int p = pq & 0xff, q = (pq >> 8) & 0xff;
+            const bool of_last = p + q >= m;
+            const bool act = pq >= 0 && !(of_last && sweep == 0);
+            bool rot = false;
+            if (act) {
+                const double2* cp = reinterpret_cast<const double2*>(L.a + p * kMaxM);
+                const double2* cq = reinterpret_cast<const double2*>(L.a + q * kMaxM);
+                double2 x[kCols / 2], y[kCols / 2];
 #pragma unroll
-                    for (int i = 0; i < kMaxM; ++i) t[i] = L.sums[lane][i];
+                for (int i = 0; i < kCols / 2; ++i) { x[i] = cp[i]; y[i] = cq[i]; }
+                double alpha = 0.0, beta = 0.0, gamma = 0.0;
 #pragma unroll
-                    for (int i = 0; i < kMaxM; ++i)
-                        if (i < m) acc = acc + t[i];
+                for (int i = 0; i < kCols; ++i) {
+                    if (i < m) {
+                        const double ai = (i & 1) ? x[i >> 1].y : x[i >> 1].x;
+                        const double bi = (i & 1) ? y[i >> 1].y : y[i >> 1].x;
+                        alpha = alpha + ai * ai;
+                        beta = beta + bi * bi;
+                        gamma = gamma + ai * bi;
+                    }
                 }
-                const double alpha = readlane_f64(acc, 0), beta = readlane_f64(acc, 1),
-                             gamma = readlane_f64(acc, 2);
-                __builtin_amdgcn_wave_barrier();
-                if (gamma == 0.0 || fabs(gamma) <= 1e-15 * sqrt(alpha * beta)) continue;
-                rotated = 1;
+                // formed whether or not the pair rotates: the test's root and
+                // the rotation's first division run side by side
                 const double zeta = (beta - alpha) / (2.0 * gamma);
+                rot = !(gamma == 0.0 || fabs(gamma) <= 1e-15 * sqrt(alpha * beta));
                 const double t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
                 const double c = 1.0 / sqrt(1.0 + t * t);
                 const double sn = c * t;
-                if (own) {
-                    ra[p] = c * ap - sn * aq;
-                    ra[q] = sn * ap + c * aq;
-                    const double vp = rv[p], vq = rv[q];
-                    rv[p] = c * vp - sn * vq;
-                    rv[q] = sn * vp + c * vq;
+                if (rot) {
+                    double* a = L.a + row;
+                    double* v = L.v + row;
+                    const double ap = a[p * kMaxM], aq = a[q * kMaxM];
+                    const double vp = v[p * kMaxM], vq = v[q * kMaxM];
+                    a[p * kMaxM] = c * ap - sn * aq;
+                    a[q * kMaxM] = sn * ap + c * aq;
+                    v[p * kMaxM] = c * vp - sn * vq;
+                    v[q * kMaxM] = sn * vp + c * vq;
                 }
             }
+            __builtin_amdgcn_wave_barrier();
+            rot_now = rot_now || __ballot(rot && !of_last) != 0;
+            rot_last = rot_last || __ballot(rot && of_last) != 0;
+            const int done = m == 2 ? (r == 1 ? sweep : -1) : (r == m - 3 ? sweep - 1 : -1);
+            if (done >= 0) {
+                const bool any = m == 2 ? rot_now : rot_last;
+                if (!any) converged = 1;
+                stop = !any || done == 59;
+                if (stop) break;
+            }
         }
-        if (!rotated) converged = 1;
+        if (stop) break;
+        rot_last = rot_now;
+        rot_now = false;
     }
     if (!converged) return 1;
     // lane j: singular value of column j, then its weight
@@ -436,7 +471,7 @@ __device__ __forceinline__ int hyperplane_fp64_wave(int m, SolveLds& L, double& 
     if (own) {
         double ss = 0.0;
         for (int i = 0; i < m; ++i) {
-            const double e = L.a[i * kMaxM + lane];
+            const double e = L.a[lane * kMaxM + i];
             ss = ss + e * e;
         }
         sig = sqrt(ss);
@@ -456,7 +491,7 @@ __device__ __forceinline__ int hyperplane_fp64_wave(int m, SolveLds& L, double& 
         double w = 0.0;
         if (use) {
             double usum = 0.0;
-            for (int i = 0; i < m; ++i) usum = usum + L.a[i * kMaxM + lane] / sig;
+            for (int i = 0; i < m; ++i) usum = usum + L.a[lane * kMaxM + i] / sig;
             w = usum / sig;
         }
         L.w[lane] = w;
@@ -466,7 +501,7 @@ __device__ __forceinline__ int hyperplane_fp64_wave(int m, SolveLds& L, double& 
     double out = 0.0;
     if (own)
         for (int j = 0; j < m; ++j)
-            if (!L.skip[j]) out = out + rv[j] * L.w[j];
+            if (!L.skip[j]) out = out + L.v[j * kMaxM + lane] * L.w[j];
     a_lane = out;
     return 0;
 }
@@ -490,12 +525,12 @@ __device__ __forceinline__ void norm_solve_tail(const float* __restrict__ fn, in
         if (lane == i) { my_ext = ext[i]; my_rmax = rmax[i]; }
     if (lane < m)
         for (int k = 0; k < m; ++k)
-            L.a[lane * kMaxM + k] = (my_ext >= 0 && my_ext < n_nds)
+            L.a[k * kMaxM + lane] = (my_ext >= 0 && my_ext < n_nds)
                                         ? static_cast<double>(fn[static_cast<size_t>(k) * nm + my_ext])
                                         : static_cast<double>(INFINITY);
     __builtin_amdgcn_wave_barrier();
     double a = 0.0;
-    const int ill = hyperplane_fp64_wave(m, L, a);
+    const int ill = m <= 4 ? hyperplane_fp64_wave<4>(m, L, a) : hyperplane_fp64_wave<kMaxM>(m, L, a);
     if (lane >= m) return;
     if (ill) a = (my_rmax > 1e-10f) ? 1.0 / static_cast<double>(fmaxf(my_rmax, 1e-6f)) : 1.0;
     if (out_a) out_a[lane] = a;
@@ -573,7 +608,7 @@ __device__ __forceinline__ void norm_solve_body(const float* __restrict__ fn, in
         ext[j] = bi;
         rmax[j] = rm;
     }
-    __shared__ SolveLds s_solve;
+    __shared__ __align__(16) SolveLds s_solve;
     if (m >= 1 && m <= kMaxM)
         norm_solve_tail(fn, nm, m, n_nds, ext, rmax, s_solve, meta, a_out, gidx, out_ext, out_a);
 }
@@ -1371,52 +1406,46 @@ __device__ void niche_body(const Bufs& B, const NicheArgs& A, NicheShared& S, in
 // (phase-4 low word, sort-1 position) for sort 2.  Sort 3 only decides which
 // n_rem members come first: its keys (rho + rank, draw_b, sort-2 position) are
 // distinct, so an 8-round radix select of the n_rem-th smallest finds the
-// chosen set exactly.  A niche of more than kBucketMaxRun members (counting
-// would be quadratic) or more than 65535 members in all (16-bit positions)
-// takes the radix sorts instead.
+// chosen set exactly (a count of the smaller keys for few members).
+//
+// Every key is one 64-bit word, so a counted pair is an LDS word read, a
+// compare and an add: about 46 us for a million pairs on the one CU, where the
+// radix sorts take about 50 ns a member.  They therefore stay for niches so
+// large that a member would be compared with more than kBucketMaxPairs others
+// on average (few directions, most of the last front in a few niches), and for
+// more than 65535 members in all (16-bit positions).
 constexpr int kNicheLdsBytes = 162816;
-constexpr int kBucketMaxRun = 128;
-constexpr int kBucketSlotBytes = 10;   // LDS: t, r / p2, p1 / lev: 2 B each; a0 / db: 4 B
-constexpr int kBucketRegs = 10;        // members a thread holds through the sort-2 step (LDS case)
+constexpr uint32_t kBucketMaxPairs = 512;
+constexpr int kBucketSlotBytes = 12;   // LDS: the key 8 B, last-front index and direction word 2 B each
+constexpr int kBucketRegs = 10;        // members a thread holds between two steps (LDS case)
+constexpr int kSelectCount = 384;      // members up to which the n_rem smallest are found by counting
 
 struct BucketSlots {
+    uint64_t* key;   // distance bits | t; then phase-4 low word | sort-1 position; then level | draw_b | sort-2 position
+    uint64_t* alt;   // workspace case: the second key array
     uint16_t* t;     // last-front index
     uint16_t* r;     // direction word (k: unassociated)
-    uint32_t* a0;    // distance bits, then the phase-4 low word
-    uint16_t* p1;    // sort-1 position
-    uint16_t* lev;   // rho + rank in the niche
-    uint32_t* db;    // draw_b
-    uint16_t* p2;    // sort-2 position
 };
 
-// LDS: four arrays of `cap` members; the sort-2 step replaces a0 by db, p1 by
-// lev and r by p2 (its results wait in registers until every member's inputs
-// are read).
 __device__ __forceinline__ BucketSlots bucket_slots(unsigned char* base, int cap)
 {
     BucketSlots v;
-    v.a0 = reinterpret_cast<uint32_t*>(base);
-    v.db = v.a0;
-    v.t = reinterpret_cast<uint16_t*>(v.a0 + cap);
+    v.key = reinterpret_cast<uint64_t*>(base);
+    v.alt = v.key;
+    v.t = reinterpret_cast<uint16_t*>(v.key + cap);
     v.r = v.t + cap;
-    v.p2 = v.r;
-    v.p1 = v.r + cap;
-    v.lev = v.p1;
     return v;
 }
 
-// Workspace (members past the LDS capacity): a0 and db in k0, the 16-bit
-// arrays in k1 and v0, each of 2n slots (8, 8 and 4 bytes a slot).
+// Workspace (members past the LDS capacity): the keys in k0 and k1, the 16-bit
+// arrays in v0, each of 2n slots.
 __device__ __forceinline__ BucketSlots bucket_slots_global(uint64_t* k0, uint64_t* k1, int32_t* v0, int nm)
 {
     BucketSlots v;
-    v.a0 = reinterpret_cast<uint32_t*>(k0);
-    v.db = v.a0 + nm;
-    v.t = reinterpret_cast<uint16_t*>(k1);
+    v.key = k0;
+    v.alt = k1;
+    v.t = reinterpret_cast<uint16_t*>(v0);
     v.r = v.t + nm;
-    v.p1 = v.r + nm;
-    v.lev = v.p1 + nm;
-    v.p2 = reinterpret_cast<uint16_t*>(v0);
     return v;
 }
 
@@ -1426,8 +1455,19 @@ __device__ __forceinline__ int half_get(const uint32_t* table, int r)
     return static_cast<int>((r & 1) ? (w >> 16) : (w & 0xFFFFu));
 }
 
+// Members of keys[st, en) below mine.
+__device__ __forceinline__ int count_below(const uint64_t* keys, int st, int en, uint64_t mine)
+{
+    int rank = 0;
+#pragma unroll 4
+    for (int u = st; u < en; ++u) rank += keys[u] < mine ? 1 : 0;
+    return rank;
+}
+
 // Slots and ranks, then the selection; table holds each niche's start (16-bit).
-// kShared: V aliases the sort-2 outputs onto its inputs (n_last <= 1024 kBucketRegs).
+// kShared: the keys sit in LDS and each step replaces them in place, its
+// results waiting in registers until every member's inputs are read
+// (n_last <= 1024 kBucketRegs); else two arrays take turns.
 template <bool kShared>
 __device__ __forceinline__ void bucket_finish(const NicheArgs& A, uint32_t* table, int32_t* misc,
                                               const BucketSlots& V, int n_prior, int n_last, int n_rem)
@@ -1442,88 +1482,76 @@ __device__ __forceinline__ void bucket_finish(const NicheArgs& A, uint32_t* tabl
         const int slot = static_cast<int>((r & 1) ? (old >> 16) : (old & 0xFFFFu));
         V.t[slot] = static_cast<uint16_t>(t);
         V.r[slot] = static_cast<uint16_t>(r);
-        V.a0[slot] = __float_as_uint(A.dist[n_prior + t]);
+        V.key[slot] = (static_cast<uint64_t>(__float_as_uint(A.dist[n_prior + t])) << 32) | static_cast<uint32_t>(t);
     }
     __syncthreads();
-    // sort 1: rank by (distance bits, t) inside the niche
-    for (int s = tid; s < n_last; s += kNicheThreads) {
+    // sort 1: rank by (distance bits, t) inside the niche, and from it the
+    // phase-4 key (low word, sort-1 position)
+    auto sort1 = [&](int s) {
         const int r = V.r[s];
         const int st = r ? half_get(table, r - 1) : 0, en = half_get(table, r);
-        const uint32_t d = V.a0[s];
-        const int t = V.t[s];
-        int rank = 0;
-        for (int u = st; u < en; ++u) {
-            const uint32_t du = V.a0[u];
-            rank += (du < d || (du == d && static_cast<int>(V.t[u]) < t)) ? 1 : 0;
-        }
-        V.p1[s] = static_cast<uint16_t>(st + rank);
-    }
-    __syncthreads();
-    // phase 4 low word
-    for (int s = tid; s < n_last; s += kNicheThreads) {
-        const int r = V.r[s];
-        const int st = r ? half_get(table, r - 1) : 0;
-        const int p1 = V.p1[s];
+        const int p1 = st + count_below(V.key, st, en, V.key[s]);
         const int rh = (r < k) ? A.rho[r] : 0;
-        V.a0[s] = (rh == 0 && p1 == st) ? 0u : (niche_draw(A.inj_a, 0, p1, A.seed, A.gen) | 1u);
-    }
-    __syncthreads();
-    // sort 2: rank by (low, p1) inside the niche; phase-5 level and draw
-    auto sort2 = [&](int s, int& lev, uint32_t& db, int& p2) {
-        const int r = V.r[s];
-        const int st = r ? half_get(table, r - 1) : 0, en = half_get(table, r);
-        const uint32_t lo = V.a0[s];
-        const int p1 = V.p1[s];
-        int rank = 0;
-        for (int u = st; u < en; ++u) {
-            const uint32_t lu = V.a0[u];
-            rank += (lu < lo || (lu == lo && static_cast<int>(V.p1[u]) < p1)) ? 1 : 0;
-        }
-        const int rh = (r < k) ? A.rho[r] : 0;
-        p2 = st + rank;
-        lev = rh + rank;
-        db = niche_draw(A.inj_b, 1, p2, A.seed, A.gen);
+        const uint32_t lo = (rh == 0 && p1 == st) ? 0u : (niche_draw(A.inj_a, 0, p1, A.seed, A.gen) | 1u);
+        return (static_cast<uint64_t>(lo) << 32) | static_cast<uint32_t>(p1);
     };
+    // sort 2: rank by that key inside the niche; the phase-5 key
+    // (level << 48 | draw_b << 16 | sort-2 position)
+    auto sort2 = [&](const uint64_t* keys, int s) {
+        const int r = V.r[s];
+        const int st = r ? half_get(table, r - 1) : 0, en = half_get(table, r);
+        const int rank = count_below(keys, st, en, keys[s]);
+        const int rh = (r < k) ? A.rho[r] : 0;
+        const uint32_t db = niche_draw(A.inj_b, 1, st + rank, A.seed, A.gen);
+        return (static_cast<uint64_t>(static_cast<uint16_t>(rh + rank)) << 48) | (static_cast<uint64_t>(db) << 16) |
+               static_cast<uint64_t>(st + rank);
+    };
+    const uint64_t* keys = V.key;
     if (kShared) {
-        int lev[kBucketRegs], p2[kBucketRegs];
-        uint32_t db[kBucketRegs];
+        uint64_t out[kBucketRegs];
 #pragma unroll
         for (int j = 0; j < kBucketRegs; ++j) {
             const int s = tid + j * kNicheThreads;
-            if (s < n_last) sort2(s, lev[j], db[j], p2[j]);
+            if (s < n_last) out[j] = sort1(s);
         }
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < kBucketRegs; ++j) {
             const int s = tid + j * kNicheThreads;
-            if (s < n_last) {
-                V.lev[s] = static_cast<uint16_t>(lev[j]);
-                V.db[s] = db[j];
-                V.p2[s] = static_cast<uint16_t>(p2[j]);
-            }
+            if (s < n_last) V.key[s] = out[j];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kBucketRegs; ++j) {
+            const int s = tid + j * kNicheThreads;
+            if (s < n_last) out[j] = sort2(V.key, s);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kBucketRegs; ++j) {
+            const int s = tid + j * kNicheThreads;
+            if (s < n_last) V.key[s] = out[j];
         }
     } else {
-        for (int s = tid; s < n_last; s += kNicheThreads) {
-            int lev, p2;
-            uint32_t db;
-            sort2(s, lev, db, p2);
-            V.lev[s] = static_cast<uint16_t>(lev);
-            V.db[s] = db;
-            V.p2[s] = static_cast<uint16_t>(p2);
-        }
+        for (int s = tid; s < n_last; s += kNicheThreads) V.alt[s] = sort1(s);
+        __syncthreads();
+        for (int s = tid; s < n_last; s += kNicheThreads) V.key[s] = sort2(V.alt, s);
     }
     __syncthreads();
+    const int take = n_rem < n_last ? n_rem : n_last;
+    if (n_last <= kSelectCount) {
+        if (tid < n_last && count_below(keys, 0, n_last, keys[tid]) < take) A.flag[A.gidx[n_prior + V.t[tid]]] = 1;
+        return;
+    }
     // sort 3 as a selection: the n_rem-th smallest of the distinct keys
     // (lev << 48 | draw_b << 16 | p2), 8 bits a round from the first byte in
     // which the keys differ, until one candidate is left
-    const int take = n_rem < n_last ? n_rem : n_last;
     int32_t* hist = misc;              // 256
     int32_t* pick = misc + 256;        // digit, count below, its count
     uint64_t* ext = reinterpret_cast<uint64_t*>(misc + 264);   // per wave min, max
     uint64_t kmin = ~0ull, kmax = 0;
     for (int s = tid; s < n_last; s += kNicheThreads) {
-        const uint64_t key = (static_cast<uint64_t>(V.lev[s]) << 48) | (static_cast<uint64_t>(V.db[s]) << 16) |
-                             static_cast<uint64_t>(V.p2[s]);
+        const uint64_t key = keys[s];
         kmin = key < kmin ? key : kmin;
         kmax = key > kmax ? key : kmax;
     }
@@ -1553,8 +1581,7 @@ __device__ __forceinline__ void bucket_finish(const NicheArgs& A, uint32_t* tabl
         if (tid < 256) hist[tid] = 0;
         __syncthreads();
         for (int s = tid; s < n_last; s += kNicheThreads) {
-            const uint64_t key = (static_cast<uint64_t>(V.lev[s]) << 48) | (static_cast<uint64_t>(V.db[s]) << 16) |
-                                 static_cast<uint64_t>(V.p2[s]);
+            const uint64_t key = keys[s];
             if ((key & mask) == prefix) atomicAdd(&hist[(key >> sh) & 255u], 1);
         }
         __syncthreads();
@@ -1594,8 +1621,7 @@ __device__ __forceinline__ void bucket_finish(const NicheArgs& A, uint32_t* tabl
     // chosen: every key whose masked value does not exceed the target's (with
     // one candidate left, or the full mask, exactly the `take` smallest)
     for (int s = tid; s < n_last; s += kNicheThreads) {
-        const uint64_t key = (static_cast<uint64_t>(V.lev[s]) << 48) | (static_cast<uint64_t>(V.db[s]) << 16) |
-                             static_cast<uint64_t>(V.p2[s]);
+        const uint64_t key = keys[s];
         if ((key & mask) <= prefix) A.flag[A.gidx[n_prior + V.t[s]]] = 1;
     }
 }
@@ -1619,7 +1645,7 @@ __device__ __forceinline__ void niche_last(const NicheArgs& A, const int32_t* __
     const int fixed = 4 * words + 4 * misc_ints;
     int cap_b = (fixed < kNicheLdsBytes) ? ((kNicheLdsBytes - fixed) / kBucketSlotBytes) & ~15 : 0;
     cap_b = min(cap_b, kBucketRegs * kNicheThreads);
-    if (A.bucket && fixed <= kNicheLdsBytes && n_last <= 65535 && n_prior <= 65535 - kBucketMaxRun) {
+    if (A.bucket && fixed <= kNicheLdsBytes && n_last <= 65535 && n_prior <= 65535) {
         uint32_t* table = reinterpret_cast<uint32_t*>(s_raw);
         int32_t* misc = reinterpret_cast<int32_t*>(s_raw + 4 * words);
         for (int j = tid; j < words; j += kNicheThreads) table[j] = 0;
@@ -1633,6 +1659,7 @@ __device__ __forceinline__ void niche_last(const NicheArgs& A, const int32_t* __
         const int lane = tid & 63, w = tid >> 6;
         uint4* mine = reinterpret_cast<uint4*>(table + tid * wpt);
         int sum = 0, run_max = 0;
+        uint32_t pairs = 0;            // members counted against each other: sum of the squares
         for (int j = 0; j < wpt / 4; ++j) {
             const uint4 v = mine[j];
             const uint32_t e[4] = {v.x, v.y, v.z, v.w};
@@ -1641,16 +1668,27 @@ __device__ __forceinline__ void niche_last(const NicheArgs& A, const int32_t* __
                 const int c0 = static_cast<int>(e[i] & 0xFFFFu), c1 = static_cast<int>(e[i] >> 16);
                 sum += c0 + c1;
                 run_max = max(run_max, max(c0, c1));
+                pairs += static_cast<uint32_t>(c0 * c0) + static_cast<uint32_t>(c1 * c1);
             }
         }
 #pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) run_max = max(run_max, __shfl_xor(run_max, o));
-        if (lane == 0) misc[w] = run_max;
+        for (int o = 32; o >= 1; o >>= 1) {
+            run_max = max(run_max, __shfl_xor(run_max, o));
+            pairs += static_cast<uint32_t>(__shfl_xor(static_cast<int>(pairs), o));
+        }
+        if (lane == 0) {
+            misc[w] = run_max;
+            misc[kNicheWaves + w] = static_cast<int>(pairs);
+        }
         int total;
         int at = block_exclusive_scan(sum, s_wave, total);   // its barriers also publish misc
         int big = 0;
+        uint32_t all_pairs = 0;
 #pragma unroll
-        for (int j = 0; j < kNicheWaves; ++j) big = max(big, misc[j]);
+        for (int j = 0; j < kNicheWaves; ++j) {
+            big = max(big, misc[j]);
+            all_pairs += static_cast<uint32_t>(misc[kNicheWaves + j]);
+        }
         for (int j = 0; j < wpt / 4; ++j) {
             const uint4 v = mine[j];
             uint32_t e[4] = {v.x, v.y, v.z, v.w};
@@ -1663,7 +1701,8 @@ __device__ __forceinline__ void niche_last(const NicheArgs& A, const int32_t* __
             mine[j] = make_uint4(e[0], e[1], e[2], e[3]);
         }
         __syncthreads();
-        if (big <= kBucketMaxRun) {
+        // (levels fit 16 bits: rho <= n_prior, rank < big)
+        if (big <= 65535 - n_prior && all_pairs <= static_cast<uint32_t>(n_last) * kBucketMaxPairs) {
             if (n_last <= cap_b && n_last <= lds_cap)
                 bucket_finish<true>(A, table, misc, bucket_slots(s_raw + fixed, cap_b), n_prior, n_last, n_rem);
             else
@@ -2086,7 +2125,7 @@ bool niching_one_block(const moea_niching& c) { return c.mode != 2; }
 int niching_buckets(const moea_niching& c) { return c.mode == 3 ? 0 : 1; }
 // each path also stops at its own LDS capacity
 int niching_lds_cap(const moea_niching& c) { return c.lds_cap > 0 ? c.lds_cap : (1 << 30); }
-constexpr int kBatchNicheMaxNm = 8192;
+constexpr int kBatchNicheMaxNm = 16384;
 }  // namespace
 
 int nsga3_select(const moea_nsga3_select_args& A)
