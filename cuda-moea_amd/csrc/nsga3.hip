@@ -1358,8 +1358,11 @@ struct NicheArgs {
     int bucket;   // 0: always the radix sorts
 };
 
+// Out of line with its arguments by value: inlined, or taking them by
+// reference, it would put the caller's in scratch on the usual path too.
 template <class Bufs>
-__device__ void niche_body(const Bufs& B, const NicheArgs& A, NicheShared& S, int n_prior, int n_last, int n_rem)
+__device__ __attribute__((noinline)) void niche_body(Bufs B, NicheArgs A, NicheShared& S, int n_prior, int n_last,
+                                                     int n_rem)
 {
     const int tid = static_cast<int>(threadIdx.x);
     const int k = A.k;
@@ -1409,13 +1412,17 @@ __device__ void niche_body(const Bufs& B, const NicheArgs& A, NicheShared& S, in
 // chosen set exactly (a count of the smaller keys for few members).
 //
 // Every key is one 64-bit word, so a counted pair is an LDS word read, a
-// compare and an add: about 46 us for a million pairs on the one CU, where the
-// radix sorts take about 50 ns a member.  They therefore stay for niches so
-// large that a member would be compared with more than kBucketMaxPairs others
-// on average (few directions, most of the last front in a few niches), and for
-// more than 65535 members in all (16-bit positions).
+// compare and an add.  Where a member would be compared with more than
+// kBucketMaxPairs others of its niche on average (few directions, or a last
+// front gathered in a few niches), each niche is first cut into as many parts
+// as it has members by a linear map of the key's value (niche_refine): members
+// are then counted against their own part only.  The radix sorts remain for
+// values too unevenly spread for that, for a last front past the LDS capacity
+// with large niches, and for more than 65535 members (16-bit positions).  On a
+// batch of 256 runs whose largest gather 8192 members in a few of 91 niches the
+// radix sorts took 218 us, counting without the cut 1484 us, this 71 us.
 constexpr int kNicheLdsBytes = 162816;
-constexpr uint32_t kBucketMaxPairs = 512;
+constexpr uint32_t kBucketMaxPairs = 96;
 constexpr int kBucketSlotBytes = 12;   // LDS: the key 8 B, last-front index and direction word 2 B each
 constexpr int kBucketRegs = 10;        // members a thread holds between two steps (LDS case)
 constexpr int kSelectCount = 384;      // members up to which the n_rem smallest are found by counting
@@ -1464,80 +1471,43 @@ __device__ __forceinline__ int count_below(const uint64_t* keys, int st, int en,
     return rank;
 }
 
-// Slots and ranks, then the selection; table holds each niche's start (16-bit).
-// kShared: the keys sit in LDS and each step replaces them in place, its
-// results waiting in registers until every member's inputs are read
-// (n_last <= 1024 kBucketRegs); else two arrays take turns.
-template <bool kShared>
-__device__ __forceinline__ void bucket_finish(const NicheArgs& A, uint32_t* table, int32_t* misc,
-                                              const BucketSlots& V, int n_prior, int n_last, int n_rem)
+// Keys of the three sorts: distance bits << 16 | last-front index; phase-4 low
+// word << 16 | sort-1 position; level << 48 | draw_b << 16 | sort-2 position.
+__device__ __forceinline__ uint64_t niche_key2(int rh, const uint32_t* inj, uint64_t seed, uint32_t gen, int st, int p1)
 {
-    const int tid = static_cast<int>(threadIdx.x);
-    const int k = A.k;
-    // place each member in its niche (order inside a niche does not matter:
-    // the ranks below break ties explicitly); afterwards table holds the ends
-    for (int t = tid; t < n_last; t += kNicheThreads) {
-        const int r = static_cast<int>(ref_word(A.ref[n_prior + t], k));
+    const uint32_t lo = (rh == 0 && p1 == st) ? 0u : (niche_draw(inj, 0, p1, seed, gen) | 1u);
+    return (static_cast<uint64_t>(lo) << 16) | static_cast<uint32_t>(p1);
+}
+
+__device__ __forceinline__ uint64_t niche_key3(int rh, const uint32_t* inj, uint64_t seed, uint32_t gen, int st, int p2)
+{
+    const uint32_t db = niche_draw(inj, 1, p2, seed, gen);
+    return (static_cast<uint64_t>(static_cast<uint16_t>(rh + p2 - st)) << 48) | (static_cast<uint64_t>(db) << 16) |
+           static_cast<uint64_t>(p2);
+}
+
+// Places each member in its niche (order inside a niche does not matter: the
+// ranks break ties explicitly); table, the niches' starts, ends as their ends.
+__device__ __forceinline__ void niche_place(const NicheArgs& A, uint32_t* table, const BucketSlots& V, int n_prior,
+                                            int n_last)
+{
+    for (int t = static_cast<int>(threadIdx.x); t < n_last; t += kNicheThreads) {
+        const int r = static_cast<int>(ref_word(A.ref[n_prior + t], A.k));
         const uint32_t old = atomicAdd(&table[r >> 1], (r & 1) ? 0x10000u : 1u);
         const int slot = static_cast<int>((r & 1) ? (old >> 16) : (old & 0xFFFFu));
         V.t[slot] = static_cast<uint16_t>(t);
         V.r[slot] = static_cast<uint16_t>(r);
-        V.key[slot] = (static_cast<uint64_t>(__float_as_uint(A.dist[n_prior + t])) << 32) | static_cast<uint32_t>(t);
+        V.key[slot] = (static_cast<uint64_t>(__float_as_uint(A.dist[n_prior + t])) << 16) | static_cast<uint32_t>(t);
     }
     __syncthreads();
-    // sort 1: rank by (distance bits, t) inside the niche, and from it the
-    // phase-4 key (low word, sort-1 position)
-    auto sort1 = [&](int s) {
-        const int r = V.r[s];
-        const int st = r ? half_get(table, r - 1) : 0, en = half_get(table, r);
-        const int p1 = st + count_below(V.key, st, en, V.key[s]);
-        const int rh = (r < k) ? A.rho[r] : 0;
-        const uint32_t lo = (rh == 0 && p1 == st) ? 0u : (niche_draw(A.inj_a, 0, p1, A.seed, A.gen) | 1u);
-        return (static_cast<uint64_t>(lo) << 32) | static_cast<uint32_t>(p1);
-    };
-    // sort 2: rank by that key inside the niche; the phase-5 key
-    // (level << 48 | draw_b << 16 | sort-2 position)
-    auto sort2 = [&](const uint64_t* keys, int s) {
-        const int r = V.r[s];
-        const int st = r ? half_get(table, r - 1) : 0, en = half_get(table, r);
-        const int rank = count_below(keys, st, en, keys[s]);
-        const int rh = (r < k) ? A.rho[r] : 0;
-        const uint32_t db = niche_draw(A.inj_b, 1, st + rank, A.seed, A.gen);
-        return (static_cast<uint64_t>(static_cast<uint16_t>(rh + rank)) << 48) | (static_cast<uint64_t>(db) << 16) |
-               static_cast<uint64_t>(st + rank);
-    };
+}
+
+// Flags the n_rem members with the smallest phase-5 keys.
+__device__ __forceinline__ void niche_select(const NicheArgs& A, int32_t* misc, const BucketSlots& V, int n_prior,
+                                             int n_last, int n_rem)
+{
+    const int tid = static_cast<int>(threadIdx.x);
     const uint64_t* keys = V.key;
-    if (kShared) {
-        uint64_t out[kBucketRegs];
-#pragma unroll
-        for (int j = 0; j < kBucketRegs; ++j) {
-            const int s = tid + j * kNicheThreads;
-            if (s < n_last) out[j] = sort1(s);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < kBucketRegs; ++j) {
-            const int s = tid + j * kNicheThreads;
-            if (s < n_last) V.key[s] = out[j];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < kBucketRegs; ++j) {
-            const int s = tid + j * kNicheThreads;
-            if (s < n_last) out[j] = sort2(V.key, s);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < kBucketRegs; ++j) {
-            const int s = tid + j * kNicheThreads;
-            if (s < n_last) V.key[s] = out[j];
-        }
-    } else {
-        for (int s = tid; s < n_last; s += kNicheThreads) V.alt[s] = sort1(s);
-        __syncthreads();
-        for (int s = tid; s < n_last; s += kNicheThreads) V.key[s] = sort2(V.alt, s);
-    }
-    __syncthreads();
     const int take = n_rem < n_last ? n_rem : n_last;
     if (n_last <= kSelectCount) {
         if (tid < n_last && count_below(keys, 0, n_last, keys[tid]) < take) A.flag[A.gidx[n_prior + V.t[tid]]] = 1;
@@ -1626,6 +1596,218 @@ __device__ __forceinline__ void bucket_finish(const NicheArgs& A, uint32_t* tabl
     }
 }
 
+// Ranks by counting inside each niche, then the selection; table holds each
+// niche's start (16-bit).
+// kShared: the keys sit in LDS and each step replaces them in place, its
+// results waiting in registers until every member's inputs are read
+// (n_last <= 1024 kBucketRegs); else two arrays take turns.
+template <bool kShared>
+__device__ __forceinline__ void bucket_finish(const NicheArgs& A, uint32_t* table, int32_t* misc,
+                                              const BucketSlots& V, int n_prior, int n_last, int n_rem)
+{
+    const int tid = static_cast<int>(threadIdx.x);
+    const int k = A.k;
+    const int32_t* rho = A.rho;
+    const uint32_t *inj_a = A.inj_a, *inj_b = A.inj_b;
+    const uint64_t seed = A.seed;
+    const uint32_t gen = A.gen;
+    niche_place(A, table, V, n_prior, n_last);
+    // sort 1: rank by (distance bits, t) inside the niche, and from it the
+    // phase-4 key (low word, sort-1 position)
+    auto sort1 = [=](int s) {
+        const int r = V.r[s];
+        const int st = r ? half_get(table, r - 1) : 0, en = half_get(table, r);
+        return niche_key2((r < k) ? rho[r] : 0, inj_a, seed, gen, st, st + count_below(V.key, st, en, V.key[s]));
+    };
+    // sort 2: rank by that key inside the niche; the phase-5 key
+    auto sort2 = [=](const uint64_t* keys, int s) {
+        const int r = V.r[s];
+        const int st = r ? half_get(table, r - 1) : 0, en = half_get(table, r);
+        return niche_key3((r < k) ? rho[r] : 0, inj_b, seed, gen, st, st + count_below(keys, st, en, keys[s]));
+    };
+    if (kShared) {
+        uint64_t out[kBucketRegs];
+#pragma unroll
+        for (int j = 0; j < kBucketRegs; ++j) {
+            const int s = tid + j * kNicheThreads;
+            if (s < n_last) out[j] = sort1(s);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kBucketRegs; ++j) {
+            const int s = tid + j * kNicheThreads;
+            if (s < n_last) V.key[s] = out[j];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kBucketRegs; ++j) {
+            const int s = tid + j * kNicheThreads;
+            if (s < n_last) out[j] = sort2(V.key, s);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kBucketRegs; ++j) {
+            const int s = tid + j * kNicheThreads;
+            if (s < n_last) V.key[s] = out[j];
+        }
+    } else {
+        for (int s = tid; s < n_last; s += kNicheThreads) V.alt[s] = sort1(s);
+        __syncthreads();
+        for (int s = tid; s < n_last; s += kNicheThreads) V.key[s] = sort2(V.alt, s);
+    }
+    __syncthreads();
+    niche_select(A, misc, V, n_prior, n_last, n_rem);
+}
+
+// One sort of the refined path: the members V.key[s] of every niche r (slots
+// [st, en) by table) move to the order of their value (key >> 16), parts first:
+// part = linear map of the value over [lo, lo + range] onto the niche's en - st
+// parts (a monotone float expression, the same for every member of a niche).
+// Each key is then replaced by next(r, st, position), the position broken by the
+// whole key where values tie; V.t travels with the keys.  False (the keys
+// unchanged) when the parts are too uneven.  mm (kUniform: unused): each
+// niche's smallest and largest value.
+constexpr uint32_t kRefineMaxPairs = 64;
+
+template <bool kUniform, class Next>
+__device__ __forceinline__ bool niche_refine(const uint32_t* table, uint32_t* sub, const uint32_t* mm, int32_t* misc,
+                                             int* s_wave, const BucketSlots& V, int n_last, Next next)
+{
+    const int tid = static_cast<int>(threadIdx.x);
+    const int words = (n_last + 1) / 2;
+    const auto part = [=](uint64_t kv, int r) {
+        const int st = r ? half_get(table, r - 1) : 0, size = half_get(table, r) - st;
+        const uint32_t v = static_cast<uint32_t>(kv >> 16);
+        int p;
+        if (kUniform) {
+            p = static_cast<int>((static_cast<uint64_t>(v) * static_cast<uint32_t>(size)) >> 32);
+        } else {
+            const uint32_t lo = mm[2 * r], range = mm[2 * r + 1] - lo;
+            const float scale = static_cast<float>(size) / (static_cast<float>(range) + 1.0f);
+            p = min(static_cast<int>(static_cast<float>(v - lo) * scale), size - 1);
+        }
+        return st + p;
+    };
+    for (int j = tid; j < words; j += kNicheThreads) sub[j] = 0u;
+    __syncthreads();
+    uint64_t key[kBucketRegs];
+    uint32_t tt[kBucketRegs];
+    int pos[kBucketRegs];
+#pragma unroll
+    for (int j = 0; j < kBucketRegs; ++j) {
+        const int s = tid + j * kNicheThreads;
+        if (s < n_last) {
+            key[j] = V.key[s];
+            tt[j] = V.t[s];
+            pos[j] = part(key[j], V.r[s]);
+            atomicAdd(&sub[pos[j] >> 1], (pos[j] & 1) ? 0x10000u : 1u);
+        }
+    }
+    __syncthreads();
+    // the parts' starts in place, thread t over `per` consecutive words
+    const int per = (words + kNicheThreads - 1) / kNicheThreads;
+    const int b = min(words, tid * per), e = min(words, b + per);
+    int sum = 0;
+    uint32_t pairs = 0;
+    for (int j = b; j < e; ++j) {
+        const uint32_t c0 = sub[j] & 0xFFFFu, c1 = sub[j] >> 16;
+        sum += static_cast<int>(c0 + c1);
+        pairs += c0 * c0 + c1 * c1;
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) pairs += static_cast<uint32_t>(__shfl_xor(static_cast<int>(pairs), o));
+    if ((tid & 63) == 0) misc[tid >> 6] = static_cast<int>(pairs);
+    int total;
+    int at = block_exclusive_scan(sum, s_wave, total);   // its barriers also publish misc
+    uint32_t all_pairs = 0;
+#pragma unroll
+    for (int j = 0; j < kNicheWaves; ++j) all_pairs += static_cast<uint32_t>(misc[j]);
+    if (all_pairs > static_cast<uint32_t>(n_last) * kRefineMaxPairs) return false;
+    for (int j = b; j < e; ++j) {
+        const int c0 = static_cast<int>(sub[j] & 0xFFFFu), c1 = static_cast<int>(sub[j] >> 16);
+        sub[j] = static_cast<uint32_t>(at) | (static_cast<uint32_t>(at + c0) << 16);
+        at += c0 + c1;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kBucketRegs; ++j) {
+        const int s = tid + j * kNicheThreads;
+        if (s < n_last) {
+            const uint32_t old = atomicAdd(&sub[pos[j] >> 1], (pos[j] & 1) ? 0x10000u : 1u);
+            const int at_j = static_cast<int>((pos[j] & 1) ? (old >> 16) : (old & 0xFFFFu));
+            V.key[at_j] = key[j];
+            V.t[at_j] = static_cast<uint16_t>(tt[j]);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kBucketRegs; ++j) {
+        const int s = tid + j * kNicheThreads;
+        if (s < n_last) {
+            const uint64_t kv = V.key[s];
+            const int r = V.r[s];
+            const int id = part(kv, r);
+            const int st = id ? half_get(sub, id - 1) : 0, en = half_get(sub, id);
+            key[j] = next(r, r ? half_get(table, r - 1) : 0, st + count_below(V.key, st, en, kv));
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kBucketRegs; ++j) {
+        const int s = tid + j * kNicheThreads;
+        if (s < n_last) V.key[s] = key[j];
+    }
+    __syncthreads();
+    return true;
+}
+
+// bucket_finish for large niches (keys in LDS); false when the values are too
+// uneven for it.
+__device__ __forceinline__ bool refine_finish(const NicheArgs& A, uint32_t* table, uint32_t* sub, uint32_t* mm,
+                                              int32_t* misc, int* s_wave, const BucketSlots& V, int n_prior,
+                                              int n_last, int n_rem)
+{
+    const int tid = static_cast<int>(threadIdx.x);
+    const int lane = tid & 63;
+    const int k = A.k;
+    const int32_t* rho = A.rho;
+    const uint32_t *inj_a = A.inj_a, *inj_b = A.inj_b;
+    const uint64_t seed = A.seed;
+    const uint32_t gen = A.gen;
+    for (int r = tid; r <= k; r += kNicheThreads) { mm[2 * r] = ~0u; mm[2 * r + 1] = 0u; }
+    niche_place(A, table, V, n_prior, n_last);
+    // each niche's smallest and largest distance bits: the wave's slots hold few
+    // niches, reduced one after another
+    for (int s0 = tid - lane; s0 < n_last; s0 += kNicheThreads) {
+        const int s = s0 + lane;
+        const bool valid = s < n_last;
+        const int r = valid ? V.r[s] : -1;
+        const uint32_t v = valid ? static_cast<uint32_t>(V.key[s] >> 16) : 0u;
+        uint64_t left = ballot(valid);
+        while (left) {
+            const int rl = __builtin_amdgcn_readlane(r, __builtin_ctzll(left));
+            const bool mine = valid && r == rl;
+            uint32_t lo = mine ? v : ~0u, hi = mine ? v : 0u;
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) {
+                lo = min(lo, static_cast<uint32_t>(__shfl_xor(static_cast<int>(lo), o)));
+                hi = max(hi, static_cast<uint32_t>(__shfl_xor(static_cast<int>(hi), o)));
+            }
+            if (lane == 0) { atomicMin(&mm[2 * rl], lo); atomicMax(&mm[2 * rl + 1], hi); }
+            left &= ~ballot(mine);
+        }
+    }
+    __syncthreads();
+    if (!niche_refine<false>(table, sub, mm, misc, s_wave, V, n_last,
+                             [=](int r, int st, int p1) { return niche_key2((r < k) ? rho[r] : 0, inj_a, seed, gen, st, p1); }))
+        return false;
+    if (!niche_refine<true>(table, sub, mm, misc, s_wave, V, n_last,
+                            [=](int r, int st, int p2) { return niche_key3((r < k) ? rho[r] : 0, inj_b, seed, gen, st, p2); }))
+        return false;
+    niche_select(A, misc, V, n_prior, n_last, n_rem);
+    return true;
+}
+
 // The last front's niching (rho must hold the prior-front counts).
 __device__ __forceinline__ void niche_last(const NicheArgs& A, const int32_t* __restrict__ meta, int nm,
                                            uint64_t* gk0, uint64_t* gk1, int32_t* gv0, int32_t* gv1, int lds_cap,
@@ -1702,12 +1884,26 @@ __device__ __forceinline__ void niche_last(const NicheArgs& A, const int32_t* __
         }
         __syncthreads();
         // (levels fit 16 bits: rho <= n_prior, rank < big)
-        if (big <= 65535 - n_prior && all_pairs <= static_cast<uint32_t>(n_last) * kBucketMaxPairs) {
-            if (n_last <= cap_b && n_last <= lds_cap)
-                bucket_finish<true>(A, table, misc, bucket_slots(s_raw + fixed, cap_b), n_prior, n_last, n_rem);
-            else
-                bucket_finish<false>(A, table, misc, bucket_slots_global(gk0, gk1, gv0, nm), n_prior, n_last, n_rem);
-            return;
+        if (big <= 65535 - n_prior) {
+            if (all_pairs <= static_cast<uint32_t>(n_last) * kBucketMaxPairs) {
+                if (n_last <= cap_b && n_last <= lds_cap)
+                    bucket_finish<true>(A, table, misc, bucket_slots(s_raw + fixed, cap_b), n_prior, n_last, n_rem);
+                else
+                    bucket_finish<false>(A, table, misc, bucket_slots_global(gk0, gk1, gv0, nm), n_prior, n_last,
+                                         n_rem);
+                return;
+            }
+            // large niches: part counters (2 B a member) and value ranges (8 B a niche) beside the slots
+            const int cap = (n_last + 15) & ~15;
+            const int extra = fixed + cap * kBucketSlotBytes;
+            if (extra + cap * 2 + (k + 1) * 8 <= kNicheLdsBytes && n_last <= kBucketRegs * kNicheThreads &&
+                n_last <= lds_cap) {
+                uint32_t* sub = reinterpret_cast<uint32_t*>(s_raw + extra);
+                if (refine_finish(A, table, sub, sub + cap / 2, misc, s_wave, bucket_slots(s_raw + fixed, cap), n_prior,
+                                  n_last, n_rem))
+                    return;
+                __syncthreads();
+            }
         }
     }
     NicheShared& S = *reinterpret_cast<NicheShared*>(s_raw);
