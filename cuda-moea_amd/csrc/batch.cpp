@@ -234,7 +234,7 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
         objectives[i] = m;
         rows4[i] = ceil_div(n, 4);
         if (I.problem == MOEA_PROBLEM_MLP) {
-            mlp_tiles[i] = mlp_tile_count(n, I.hidden);
+            mlp_tiles[i] = mlp_tile_count(n, I.hidden, true);
             h4[m][i] = ceil_div(n, 4);
         } else {
             q4[m][i] = ceil_div(n, 4);
@@ -265,6 +265,12 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
         G.eval.quad_rows4[m] = T.add(q4[m]);
         G.eval.mlp_rows4[m] = T.add(h4[m]);
     }
+    long long big_tiles = 0;
+    for (long long t : mlp_tiles) big_tiles += t;
+    G.eval.mlp_big = mlp_fills(big_tiles);
+    if (!G.eval.mlp_big)
+        for (int i = 0; i < count; ++i)
+            if (mlp_tiles[i]) mlp_tiles[i] = mlp_tile_count(host[i].n, host[i].hidden, false);
     G.eval.mlp_tiles = T.add(mlp_tiles);
     G.sel.merged256 = T.add(merged256);
     G.sel.rows4 = T.add(rows4);

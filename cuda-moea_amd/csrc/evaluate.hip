@@ -93,18 +93,46 @@ __global__ __launch_bounds__(256) void b_quadratic_kernel(const BInst* __restric
 }
 
 // MLP hidden layer H = tanh(X W1^T): (n, d) x (hidden, d)^T -> (n, hidden),
-// on the FP32 matrix cores (v_mfma_f32_16x16x4_f32).  A 256-thread block
-// owns a 64 x 128 tile of H; its four waves each own 32 x 64 (2 x 4 MFMA
-// tiles).  K advances in slices of 32 staged in LDS (double-buffered, next
-// slice prefetched into registers during the current one's MFMAs).  Both
-// operands are K-contiguous, so a lane reads four consecutive k of its row
-// with one 16-byte LDS read; lane group g = lane / 16 takes k = 4g + s in MFMA
-// step s (the MFMA sums over its four lane groups), which covers every k of
-// the slice once.  Accumulation is FP32 throughout; the summation order is
-// fixed by the tiling, so a row of H does not depend on anything else in the
-// launch (the batched launch reproduces the single-run values bit for bit).
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-constexpr int kHM = 64, kHN = 128, kHK = 32, kHS = kHK + 4;   // tile rows, cols, k slice, LDS row stride
+// float products on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16).  Every
+// float is split into three bf16 numbers that sum to it exactly (8 + 8 + 8
+// significant bits, each the rounded remainder), and of the nine products of
+// two such sums the six above 2^-24 of the whole are accumulated in FP32,
+// smallest first: hi lo, lo hi, mid mid, mid hi, hi mid, hi hi.  What is left
+// out is below half a unit in the last place of a float product; a step adds
+// 16 products to the accumulator where the FP32 cores' step added 4, and every
+// kMlpFold k the partial sum is folded into a total, so fewer and smaller sums
+// are rounded.
+//   relative error of H against 64 bits (2-norm), FP32 cores -> here:
+//   d = 10: 5.7e-8 -> 3.9e-8, 333: 2.7e-7 -> 2.2e-7, 1333: 5.4e-7 -> 4.6e-7,
+//   20000: 2.1e-6 -> 1.1e-6, 131072: 5.2e-6 -> 1.6e-6.
+// Six bf16 products at 2.5 PFLOP/s peak cost less than one FP32 product at 157
+// TFLOP/s: 16384 x 131072 x 256 takes 6.9 ms instead of 9.7 (160 TFLOP/s of
+// float products, 0.78 of what a plain bf16 product of the library's reaches),
+// 2046 x 1333 x 256 47 us instead of 99.
+//
+// A workgroup owns a BM x BN tile of H, its waves 32-row strips of it.  K
+// advances in slices of 32: the next two slices are in flight in registers, a
+// slice is split on its way to LDS (11 VALU instructions per two numbers, under
+// the other waves' MFMAs), and a lane reads 8 consecutive k of its row with one
+// 16-byte read per part (row stride 80 bytes: no bank conflicts).  A number's
+// place in the order of a sum depends on k alone, not on the tile, so a row of
+// H does not depend on anything else in the launch (the batched launch
+// reproduces the single-run values bit for bit).
+//
+// Infinities, NaN and numbers beyond bf16's largest make the remainders NaN;
+// an element whose sum ends as NaN is summed again by a plain FP32 loop.
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+constexpr int kHK = 32;                 // k slice
+constexpr int kHS = kHK + 8;            // LDS row stride, bf16
+// Tile shapes: large ones read X and W1 least and split each number for 128
+// others; small ones where those would leave CUs without work, with more
+// slices in flight, since a slice then costs less than a trip to memory.
+struct MlpBig { static constexpr int BM = 128, BN = 128, WM = 4, WN = 2, SETS = 2; };
+struct MlpSmall { static constexpr int BM = 64, BN = 64, WM = 2, WN = 2, SETS = 2; };
+constexpr int kMlpFold = 4096;          // k after which a partial sum is folded into the total
+constexpr int kMlpBigTiles = 192;       // tiles of the large shape from which it is used
 
 // (row tile, col tile) of tile index t: the col tiles of one row tile sit
 // 8 indices apart, so a round-robin dispatch over the 8 XCDs puts them on one
@@ -119,39 +147,65 @@ __device__ __forceinline__ bool mlp_tile_of(int t, int nrt, int nct, int& rt, in
 
 }  // namespace
 
-int mlp_tile_count(int n, int hidden)
+bool mlp_fills(long long big_tiles) { return big_tiles >= kMlpBigTiles; }
+
+int mlp_tile_count(int n, int hidden, bool big)
 {
-    const int nrt = (n + kHM - 1) / kHM, nct = (hidden + kHN - 1) / kHN;
+    const int nrt = ceil_div(n, big ? MlpBig::BM : MlpSmall::BM), nct = ceil_div(hidden, big ? MlpBig::BN : MlpSmall::BN);
     return ((nrt + 7) / 8) * 8 * nct;
 }
 
 namespace {
 
+template <class T>
 struct MlpSmem {
-    float a[2][kHM * kHS];
-    float b[2][kHN * kHS];
+    __bf16 part[2][3][(T::BM + T::BN) * kHS];     // buffer, part, rows of X then of W1
 };
+
+// How a matrix's rows are read, four floats at a time: rows that keep 16-byte
+// alignment, any other row length with 16-byte loads of 4-byte alignment (a
+// load near a row's end runs on into the next row; at the matrix's end it is
+// moved back and its numbers shifted into place), or one float at a time where
+// the matrix has fewer than four.  One float at a time for every d that is not
+// a multiple of 4 cost a third more there (2046 x 1333 x 256: 60 us -> 47 us).
+enum MlpLoad : int { kLoadAligned, kLoadAny, kLoadSingle };
 
 // Loads are issued unconditionally from clamped (in-bounds) addresses and the
 // out-of-range elements are zeroed when the registers are stored to LDS, so
 // no load sits behind a branch (a branch join would wait for it).
-// VEC: ld % 4 == 0 (one 16-byte load); otherwise four scalar loads.
-template <bool VEC>
+template <int LOAD>
 __device__ __forceinline__ float4 mlp_raw4(const float* __restrict__ base, int row, int nrows, int ld, int k)
 {
     const float* p = base + static_cast<size_t>(min(row, nrows - 1)) * ld;
-    if (VEC) return *reinterpret_cast<const float4*>(p + min(k, ld - 4));
+    if constexpr (LOAD == kLoadAligned) return *reinterpret_cast<const float4*>(p + min(k, ld - 4));
     float4 v;
-    v.x = p[min(k, ld - 1)];
-    v.y = p[min(k + 1, ld - 1)];
-    v.z = p[min(k + 2, ld - 1)];
-    v.w = p[min(k + 3, ld - 1)];
+    if constexpr (LOAD == kLoadAny) {
+        const float* last = base + (static_cast<size_t>(nrows) * ld - 4);
+        const float* q = p + min(k, ld - 1);
+        __builtin_memcpy(&v, q < last ? q : last, sizeof(v));
+    } else {
+        v.x = p[min(k, ld - 1)];
+        v.y = p[min(k + 1, ld - 1)];
+        v.z = p[min(k + 2, ld - 1)];
+        v.w = p[min(k + 3, ld - 1)];
+    }
     return v;
 }
 
+template <int LOAD>
 __device__ __forceinline__ float4 mlp_mask4(float4 v, int row, int nrows, int ld, int k)
 {
     const bool r = row < nrows;
+    if constexpr (LOAD == kLoadAny) {
+        // the last row's end: loaded up to three places too early
+        const int back = (row == nrows - 1 && k < ld) ? k - (ld - 4) : 0;
+        if (back > 0) {
+            const float e1 = v.y, e2 = v.z, e3 = v.w;
+            v.x = back == 1 ? e1 : back == 2 ? e2 : e3;
+            v.y = back == 1 ? e2 : e3;
+            v.z = e3;
+        }
+    }
     v.x = (r && k < ld) ? v.x : 0.0f;
     v.y = (r && k + 1 < ld) ? v.y : 0.0f;
     v.z = (r && k + 2 < ld) ? v.z : 0.0f;
@@ -164,32 +218,64 @@ __device__ __forceinline__ float4 mlp_mask4(float4 v, int row, int nrows, int ld
 // sums its 4 columns of every slice, then a fixed xor reduction over the 8)
 // and store it in rowsq[row]; the head reads it there instead of reading x
 // again.
-template <bool VEC>
+// Three bf16 parts of four floats, to three LDS rows.
+__device__ __forceinline__ void mlp_split4(float4 v, __bf16* hi, __bf16* mid, __bf16* lo)
+{
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    const f32x2 x[2] = {{v.x, v.y}, {v.z, v.w}};
+    uint32_t out[3][2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        f32x2 r = x[j];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            const uint32_t b = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
+            out[p][j] = b;
+            r[0] = r[0] - __uint_as_float(b << 16);
+            r[1] = r[1] - __uint_as_float(b & 0xFFFF0000u);
+        }
+    }
+    *reinterpret_cast<uint2*>(hi) = make_uint2(out[0][0], out[0][1]);
+    *reinterpret_cast<uint2*>(mid) = make_uint2(out[1][0], out[1][1]);
+    *reinterpret_cast<uint2*>(lo) = make_uint2(out[2][0], out[2][1]);
+}
+
+template <class T, int LOAD>
 __device__ __forceinline__ void mlp_hidden_tile(const float* __restrict__ x, int n, int d,
                                                 const float* __restrict__ w1, int hidden,
-                                                float* __restrict__ h, int r0, int c0, MlpSmem& sm,
+                                                float* __restrict__ h, int r0, int c0, MlpSmem<T>& sm,
                                                 float* __restrict__ rowsq)
 {
+    constexpr int kThreads = 64 * T::WM * T::WN;
+    constexpr int kRows = kThreads / 8;                   // rows a load pass covers, 8 float4 each
+    constexpr int PA = T::BM / kRows, PB = T::BN / kRows;
+    constexpr int TN = T::BN / T::WN / 32;                // 32 x 32 tiles of a wave (one row strip)
+    static_assert(T::BM == 32 * T::WM && PA * kRows == T::BM && PB * kRows == T::BN, "tile shape");
     const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = tid >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
-    const int g = lane >> 4, i = lane & 15;
-    // loader: 8 float4 per 32-float row slice; A 64 rows (2 per thread), B 128 rows (4 per thread)
+    const int wm = wave % T::WM, wn = wave / T::WM;
+    const int g = lane >> 5, i = lane & 31;
     const int lrow = tid >> 3, lk = (tid & 7) * 4;
-    // two register sets: slices s + 1 and s + 2 are in flight while slice s is in LDS
-    float4 pa[2][2], pb[2][4];
+    // register sets: slices s + 1 .. s + SETS are in flight while slice s is in LDS
+    float4 pa[T::SETS][PA], pb[T::SETS][PB];
     auto load = [&](int set, int k0) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) pa[set][j] = mlp_raw4<VEC>(x, r0 + lrow + 32 * j, n, d, k0 + lk);
+        for (int j = 0; j < PA; ++j) pa[set][j] = mlp_raw4<LOAD>(x, r0 + lrow + kRows * j, n, d, k0 + lk);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) pb[set][j] = mlp_raw4<VEC>(w1, c0 + lrow + 32 * j, hidden, d, k0 + lk);
+        for (int j = 0; j < PB; ++j) pb[set][j] = mlp_raw4<LOAD>(w1, c0 + lrow + kRows * j, hidden, d, k0 + lk);
     };
     const bool sq = (c0 == 0);
-    float sqs[2] = {0.0f, 0.0f};
+    float sqs[PA];
+#pragma unroll
+    for (int j = 0; j < PA; ++j) sqs[j] = 0.0f;
+    auto put = [&](int buf, int row, float4 v) {
+        const int at = row * kHS + lk;
+        mlp_split4(v, &sm.part[buf][0][at], &sm.part[buf][1][at], &sm.part[buf][2][at]);
+    };
     auto store = [&](int set, int buf, int k0) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const float4 v = mlp_mask4(pa[set][j], r0 + lrow + 32 * j, n, d, k0 + lk);
-            *reinterpret_cast<float4*>(&sm.a[buf][(lrow + 32 * j) * kHS + lk]) = v;
+        for (int j = 0; j < PA; ++j) {
+            const float4 v = mlp_mask4<LOAD>(pa[set][j], r0 + lrow + kRows * j, n, d, k0 + lk);
+            put(buf, lrow + kRows * j, v);
             if (sq) {
                 const float t0 = v.x - 0.5f, t1 = v.y - 0.5f, t2 = v.z - 0.5f, t3 = v.w - 0.5f;
                 const int kk = k0 + lk;
@@ -200,32 +286,32 @@ __device__ __forceinline__ void mlp_hidden_tile(const float* __restrict__ x, int
             }
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            *reinterpret_cast<float4*>(&sm.b[buf][(lrow + 32 * j) * kHS + lk]) =
-                mlp_mask4(pb[set][j], c0 + lrow + 32 * j, hidden, d, k0 + lk);
+        for (int j = 0; j < PB; ++j)
+            put(buf, T::BM + lrow + kRows * j, mlp_mask4<LOAD>(pb[set][j], c0 + lrow + kRows * j, hidden, d, k0 + lk));
     };
-    f32x4 acc[2][4];
+    f32x16 acc[TN], total[TN];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int u = 0; u < TN; ++u)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) acc[t][u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int r = 0; r < 16; ++r) { acc[u][r] = 0.0f; total[u][r] = 0.0f; }
     auto compute = [&](int buf) {
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            float4 a[2], b[4];
+        for (int ks = 0; ks < kHK; ks += 16) {
+            bf16x8 a[3], b[TN][3];
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
-                a[t] = *reinterpret_cast<const float4*>(&sm.a[buf][(wm * 32 + t * 16 + i) * kHS + half * 16 + 4 * g]);
+            for (int p = 0; p < 3; ++p) {
+                a[p] = *reinterpret_cast<const bf16x8*>(&sm.part[buf][p][(wm * 32 + i) * kHS + ks + 8 * g]);
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-                b[u] = *reinterpret_cast<const float4*>(&sm.b[buf][(wn * 64 + u * 16 + i) * kHS + half * 16 + 4 * g]);
+                for (int u = 0; u < TN; ++u)
+                    b[u][p] = *reinterpret_cast<const bf16x8*>(
+                        &sm.part[buf][p][(T::BM + (wn * TN + u) * 32 + i) * kHS + ks + 8 * g]);
+            }
+            constexpr int pa_of[6] = {0, 2, 1, 1, 0, 0}, pb_of[6] = {2, 0, 1, 0, 1, 0};
 #pragma unroll
-            for (int st = 0; st < 4; ++st)
+            for (int q = 0; q < 6; ++q)
 #pragma unroll
-                for (int t = 0; t < 2; ++t)
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][st], b[u][st], acc[t][u], 0, 0, 0);
+                for (int u = 0; u < TN; ++u)
+                    acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa_of[q]], b[u][pb_of[q]], acc[u], 0, 0, 0);
         }
     };
     // Loads and stores are unconditional (a slice past d loads clamped
@@ -233,55 +319,81 @@ __device__ __forceinline__ void mlp_hidden_tile(const float* __restrict__ x, int
     // same loads in flight and the waits stay exact.
     load(0, 0);
     store(0, 0, 0);
-    load(1, kHK);
-    load(0, 2 * kHK);
+#pragma unroll
+    for (int t = 1; t <= T::SETS; ++t) load(t % T::SETS, t * kHK);
     __syncthreads();
-    // slice s sits in LDS buffer s % 2; slice s + 1 in register set (s + 1) % 2
-    for (int k0 = 0;; k0 += 2 * kHK) {
-        compute(0);                                   // slice k0
-        store(1, 1, k0 + kHK);                        // slice k0 + 32
-        load(1, k0 + 3 * kHK);
-        __syncthreads();
-        if (k0 + kHK >= d) break;
-        compute(1);                                   // slice k0 + 32
-        store(0, 0, k0 + 2 * kHK);                    // slice k0 + 64
-        load(0, k0 + 4 * kHK);
-        __syncthreads();
-        if (k0 + 2 * kHK >= d) break;
+    // slice s sits in LDS buffer s % 2; slice s + 1 in register set (s + 1) % SETS
+    static_assert(T::SETS % 2 == 0 && kMlpFold % (T::SETS * kHK) == 0, "slices of a loop step");
+    bool more = true;
+    for (int k0 = 0; more; k0 += T::SETS * kHK) {
+#pragma unroll
+        for (int t = 0; t < T::SETS; ++t) {
+            compute(t & 1);                                          // slice k0 + 32 t
+            store((t + 1) % T::SETS, (t + 1) & 1, k0 + (t + 1) * kHK);
+            load((t + 1) % T::SETS, k0 + (t + 1 + T::SETS) * kHK);
+            __syncthreads();
+            if (k0 + (t + 1) * kHK >= d) { more = false; break; }
+        }
+        if (!more || (k0 + T::SETS * kHK) % kMlpFold == 0) {
+#pragma unroll
+            for (int u = 0; u < TN; ++u)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) { total[u][r] = total[u][r] + acc[u][r]; acc[u][r] = 0.0f; }
+        }
     }
     if (sq) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < PA; ++j) {
             float v = sqs[j];
             v = v + __shfl_xor(v, 1);
             v = v + __shfl_xor(v, 2);
             v = v + __shfl_xor(v, 4);
-            const int row = r0 + lrow + 32 * j;
+            const int row = r0 + lrow + kRows * j;
             if ((tid & 7) == 0 && row < n) rowsq[row] = v;
         }
     }
-    // D of a 16 x 16 MFMA tile: lane (g, i) holds rows 4g .. 4g+3 of column i
+    // D of a 32 x 32 MFMA tile: lane (g, i) holds rows 8 (r / 4) + 4 g + r % 4 of column i
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int u = 0; u < TN; ++u)
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = r0 + wm * 32 + t * 16 + 4 * g + r;
-                const int col = c0 + wn * 64 + u * 16 + i;
-                if (row < n && col < hidden) h[static_cast<size_t>(row) * hidden + col] = tanhf(acc[t][u][r]);
+        for (int r = 0; r < 16; ++r) {
+            const int row = r0 + wm * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
+            const int col = c0 + (wn * TN + u) * 32 + i;
+            if (row < n && col < hidden) {
+                float v = total[u][r];
+                if (v != v) {
+                    v = 0.0f;
+                    const float* xr = x + static_cast<size_t>(row) * d;
+                    const float* wr = w1 + static_cast<size_t>(col) * d;
+                    for (int k = 0; k < d; ++k) v = fmaf(xr[k], wr[k], v);
+                }
+                h[static_cast<size_t>(row) * hidden + col] = tanhf(v);
             }
+        }
 }
 
-__global__ __launch_bounds__(256) void mlp_hidden_kernel(const float* __restrict__ x, int n, int d,
-                                                         const float* __restrict__ w1, int hidden,
-                                                         float* __restrict__ h, float* __restrict__ rowsq)
+template <class T>
+__device__ __forceinline__ void mlp_hidden_block(const float* __restrict__ x, int n, int d,
+                                                 const float* __restrict__ w1, int hidden, float* __restrict__ h,
+                                                 float* __restrict__ rowsq, int local, MlpSmem<T>& sm)
 {
-    __shared__ __align__(16) MlpSmem sm;
     int rt, ct;
-    if (!mlp_tile_of(static_cast<int>(blockIdx.x), (n + kHM - 1) / kHM, (hidden + kHN - 1) / kHN, rt, ct)) return;
-    if ((d & 3) == 0) mlp_hidden_tile<true>(x, n, d, w1, hidden, h, rt * kHM, ct * kHN, sm, rowsq);
-    else mlp_hidden_tile<false>(x, n, d, w1, hidden, h, rt * kHM, ct * kHN, sm, rowsq);
+    if (!mlp_tile_of(local, (n + T::BM - 1) / T::BM, (hidden + T::BN - 1) / T::BN, rt, ct)) return;
+    const int r0 = rt * T::BM, c0 = ct * T::BN;
+    if ((d & 3) == 0) mlp_hidden_tile<T, kLoadAligned>(x, n, d, w1, hidden, h, r0, c0, sm, rowsq);
+    else if (static_cast<long long>(min(n, hidden)) * d >= 4)
+        mlp_hidden_tile<T, kLoadAny>(x, n, d, w1, hidden, h, r0, c0, sm, rowsq);
+    else mlp_hidden_tile<T, kLoadSingle>(x, n, d, w1, hidden, h, r0, c0, sm, rowsq);
+}
+
+template <class T>
+__global__ __launch_bounds__(64 * T::WM * T::WN) void mlp_hidden_kernel(const float* __restrict__ x, int n, int d,
+                                                                        const float* __restrict__ w1, int hidden,
+                                                                        float* __restrict__ h,
+                                                                        float* __restrict__ rowsq)
+{
+    __shared__ __align__(16) MlpSmem<T> sm;
+    mlp_hidden_block<T>(x, n, d, w1, hidden, h, rowsq, static_cast<int>(blockIdx.x), sm);
 }
 
 // Output head: y = W2 h, f_c = y_c^2 + 0.01 * ||x - 0.5||^2; one wave per row.
@@ -326,19 +438,16 @@ __global__ __launch_bounds__(256) void mlp_head_kernel(int n, const float* __res
 }
 
 // Batched MLP: hidden-layer tiles, then the head rows of the instances with M objectives.
-__global__ __launch_bounds__(256) void b_mlp_hidden_kernel(const BInst* __restrict__ insts, BMap mp, int which)
+template <class T>
+__global__ __launch_bounds__(64 * T::WM * T::WN) void b_mlp_hidden_kernel(const BInst* __restrict__ insts, BMap mp,
+                                                                          int which)
 {
     int local;
     const int i = bmap_find(mp, static_cast<int>(blockIdx.x), local);
     const BInst& I = insts[i];
     const int slot = (I.cur + which) % 3;
-    __shared__ __align__(16) MlpSmem sm;
-    int rt, ct;
-    if (!mlp_tile_of(local, (I.n + kHM - 1) / kHM, (I.hidden + kHN - 1) / kHN, rt, ct)) return;
-    if ((I.d & 3) == 0)
-        mlp_hidden_tile<true>(I.x[slot], I.n, I.d, I.w1, I.hidden, I.hwork, rt * kHM, ct * kHN, sm, I.f[slot]);
-    else
-        mlp_hidden_tile<false>(I.x[slot], I.n, I.d, I.w1, I.hidden, I.hwork, rt * kHM, ct * kHN, sm, I.f[slot]);
+    __shared__ __align__(16) MlpSmem<T> sm;
+    mlp_hidden_block<T>(I.x[slot], I.n, I.d, I.w1, I.hidden, I.hwork, I.f[slot], local, sm);
 }
 
 template <int M>
@@ -624,8 +733,14 @@ int eval_mlp(const float* x, int n, int d, const float* w1, int hidden, const fl
     if (!x || !w1 || !w2 || !f || !hwork || n <= 0 || d <= 0 || hidden <= 0 || m <= 0 || m > kMaxM ||
         ldf < n)
         return fail(kInvalidArgument, "eval_mlp: invalid arguments");
-    hipLaunchKernelGGL(mlp_hidden_kernel, dim3(mlp_tile_count(n, hidden)), dim3(256), 0, stream, x, n, d, w1,
-                       hidden, hwork, f);
+    const bool big = mlp_fills(mlp_tile_count(n, hidden, true));
+    const dim3 tiles(mlp_tile_count(n, hidden, big));
+    if (big)
+        hipLaunchKernelGGL(mlp_hidden_kernel<MlpBig>, tiles, dim3(64 * MlpBig::WM * MlpBig::WN), 0, stream, x, n, d, w1,
+                           hidden, hwork, f);
+    else
+        hipLaunchKernelGGL(mlp_hidden_kernel<MlpSmall>, tiles, dim3(64 * MlpSmall::WM * MlpSmall::WN), 0, stream, x, n,
+                           d, w1, hidden, hwork, f);
     MOEA_HIP(hipGetLastError());
     const dim3 grid(ceil_div(n, 4)), block(256);
     switch (m) {
@@ -663,8 +778,12 @@ int batch_evaluate(const BatchLaunch& L, const BEvalGrids& G, int which)
         MOEA_HIP(hipGetLastError());
     }
     if (G.mlp_tiles.blocks > 0) {
-        hipLaunchKernelGGL(b_mlp_hidden_kernel, dim3(G.mlp_tiles.blocks), dim3(256), 0, L.stream, L.insts,
-                           G.mlp_tiles.map, which);
+        if (G.mlp_big)
+            hipLaunchKernelGGL(b_mlp_hidden_kernel<MlpBig>, dim3(G.mlp_tiles.blocks),
+                               dim3(64 * MlpBig::WM * MlpBig::WN), 0, L.stream, L.insts, G.mlp_tiles.map, which);
+        else
+            hipLaunchKernelGGL(b_mlp_hidden_kernel<MlpSmall>, dim3(G.mlp_tiles.blocks),
+                               dim3(64 * MlpSmall::WM * MlpSmall::WN), 0, L.stream, L.insts, G.mlp_tiles.map, which);
         MOEA_HIP(hipGetLastError());
         for (int m = 1; m <= kMaxM; ++m) {
             if (G.mlp_rows4[m].blocks <= 0) continue;

@@ -1,0 +1,61 @@
+"""The MLP objective against FP64 at the edges of its tiles, slices and loads,
+and its value for infinite and NaN variables."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+if not torch.cuda.is_available():
+    pytest.skip("needs a ROCm GPU", allow_module_level=True)
+
+from cuda_moea import kernels as K  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+
+
+def _case(n, d, hidden, m):
+    g = torch.Generator().manual_seed(n + d)
+    x = torch.rand(n, d, generator=g)
+    w1 = torch.randn(hidden, d, generator=g) / np.sqrt(d)
+    w2 = torch.randn(m, hidden, generator=g) / np.sqrt(hidden)
+    return x, w1, w2
+
+
+def _fp64(x, w1, w2):
+    xd = x.double()
+    y = torch.tanh(xd @ w1.double().t()) @ w2.double().t()
+    return (y.square() + 0.01 * (xd - 0.5).square().sum(1, keepdim=True)).t()
+
+
+# tiles of 64 and 128 rows and columns, slices of 32, rows of every alignment,
+# matrices of fewer than four numbers, folds at 4096, the large tile shape
+@pytest.mark.parametrize("n,d,hidden,m", [(1, 1, 1, 1), (1, 3, 1, 2), (3, 1, 5, 3), (2, 2, 2, 1), (1, 5, 2, 1),
+                                          (63, 31, 64, 3), (64, 32, 65, 5), (65, 33, 63, 2), (128, 35, 128, 10),
+                                          (129, 64, 130, 4), (200, 4095, 100, 3), (130, 4097, 96, 3),
+                                          (127, 8194, 40, 3), (12288, 37, 256, 5), (12289, 66, 255, 5)])
+def test_mlp_sizes_against_fp64(n, d, hidden, m):
+    x, w1, w2 = _case(n, d, hidden, m)
+    print(f"mlp n={n} d={d} hidden={hidden} m={m}", flush=True)
+    f, cv = K.eval_mlp(x.to(DEV), w1.to(DEV), w2.to(DEV))
+    ref = _fp64(x, w1, w2)
+    # float sums of d terms: 64 sqrt(d) 2^-24 (1 + |f|), the objective tests' bound
+    tol = 64 * np.sqrt(d) * 2.0 ** -24 * (1 + ref.abs())
+    assert bool(((f.cpu().double() - ref).abs() <= tol).all())
+    assert not cv.cpu().any()
+
+
+def test_mlp_infinite_and_nan_rows():
+    n, d, hidden, m = 70, 45, 64, 3
+    x, w1, w2 = _case(n, d, hidden, m)
+    w1[3, 7] = 0.0
+    x[5, 7], x[6, 9], x[7, 2], x[8, 4] = np.inf, -np.inf, np.nan, 3.4e38
+    f, _ = K.eval_mlp(x.to(DEV), w1.to(DEV), w2.to(DEV))
+    f = f.cpu()
+    keep = [i for i in range(n) if i not in (5, 6, 7, 8)]
+    ref = _fp64(x[keep], w1, w2)
+    tol = 64 * np.sqrt(d) * 2.0 ** -24 * (1 + ref.abs())
+    assert bool(((f[:, keep].double() - ref).abs() <= tol).all())
+    assert bool(torch.isnan(f[:, 5]).all())               # 0 * inf in hidden unit 3, as in FP32
+    assert bool(torch.isinf(f[:, 6]).all())               # every hidden unit saturates, the distance is infinite
+    assert bool(torch.isnan(f[:, 7]).all())
+    assert bool(torch.isinf(f[:, 8]).all())               # (3.4e38)^2 overflows in the distance only
