@@ -120,7 +120,7 @@ void fill_record(const moea_batch_problem& p, BInst& I)
     I.n = z.n; I.m = z.m; I.d = z.d; I.k = z.k;
     I.nm = z.nm; I.W = z.W; I.Wc = z.Wc; I.npad = z.npad;
     I.max_gen = p.max_generations;
-    I.ddiv = fast_div_make(static_cast<uint32_t>(z.d));
+    I.gdiv = fast_div_make(static_cast<uint32_t>((z.d + 3) / 4));
     I.seed = p.seed;
     I.sbx_eta0 = p.sbx_eta[0]; I.sbx_eta1 = p.sbx_eta[1];
     I.sbx_prob = p.sbx_prob; I.sbx_copy = p.sbx_copy_prob;
@@ -229,7 +229,7 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
         const int nb = ceil_div(nm, 256);
         init256[i] = ceil_div(static_cast<long long>(n) * I.d, 256);
         rows256[i] = ceil_div(n, 256);
-        sbx256[i] = ceil_div(static_cast<long long>(n / 2) * I.d + ((n & 1) ? I.d : 0), 256);
+        sbx256[i] = ceil_div(static_cast<long long>(n / 2) * ((I.d + 3) / 4), 256);
         merged256[i] = nb;
         objectives[i] = m;
         rows4[i] = ceil_div(n, 4);

@@ -31,7 +31,7 @@ struct BInst {
     int n, m, d, k;
     int nm, W, Wc, npad;          // NDS over the 2n merged rows
     int max_gen;
-    FastDiv ddiv;                 // division by d (reproduction element indices)
+    FastDiv gdiv;                 // division by ceil(d / 4) (reproduction thread indices)
     uint64_t seed;
     float sbx_eta0, sbx_eta1, sbx_prob, sbx_copy, pm_eta0, pm_eta1, pm_prob;
     // problem (caller-owned device arrays)

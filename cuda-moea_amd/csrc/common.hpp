@@ -75,6 +75,17 @@ enum DrawStream : uint32_t { kStInit = 1, kStMate = 2, kStSbx = 3, kStPm = 4 };
 
 struct U4 { uint32_t x, y, z, w; };
 
+// a ^ b ^ c, one instruction on gfx950 (the compiler emits two): the xors are
+// a third of a Philox block's instructions.
+__host__ __device__ inline uint32_t xor3(uint32_t a, uint32_t b, uint32_t c)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+    return a ^ b ^ c;
+#endif
+}
+
 __host__ __device__ inline U4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
                                             uint32_t k0, uint32_t k1)
 {
@@ -82,9 +93,9 @@ __host__ __device__ inline U4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c
     for (int r = 0; r < 10; ++r) {
         const uint64_t p0 = static_cast<uint64_t>(0xD2511F53u) * c0;
         const uint64_t p1 = static_cast<uint64_t>(0xCD9E8D57u) * c2;
-        const uint32_t n0 = static_cast<uint32_t>(p1 >> 32) ^ c1 ^ k0;
+        const uint32_t n0 = xor3(static_cast<uint32_t>(p1 >> 32), c1, k0);
         const uint32_t n1 = static_cast<uint32_t>(p1);
-        const uint32_t n2 = static_cast<uint32_t>(p0 >> 32) ^ c3 ^ k1;
+        const uint32_t n2 = xor3(static_cast<uint32_t>(p0 >> 32), c3, k1);
         const uint32_t n3 = static_cast<uint32_t>(p0);
         c0 = n0; c1 = n1; c2 = n2; c3 = n3;
         k0 += 0x9E3779B9u;
@@ -246,13 +257,24 @@ __host__ __device__ inline float powf_det(float x, float y)
 //   2^z = 2^k e^w, k = rint(hi), w = ((hi - k) + lo) ln 2, e^w by its Taylor
 //     polynomial to w^8 / 8! (A&S 4.2.1), |w| <= 0.35.
 // Identical on host and device (fmaf, IEEE division, no contraction).
-__host__ __device__ inline float powf_root(float x, float y)
+// powf_root_normal is its core for normal x, scaled by 2^e.
+
+// 1 / d rounded to nearest for normal d and 1 / d: the hardware's reciprocal
+// (within 1 ulp) and one Newton step in fused arithmetic.  Equal to IEEE
+// division for every mantissa (checked over all floats of [1, 4); a power of
+// two changes nothing) at a third of its instructions.
+__host__ __device__ inline float recip_normal(float d)
 {
-    if (!(x > 0.0f)) return x == 0.0f ? 0.0f : NAN;
-    if (x == 1.0f) return 1.0f;
-    if (x == INFINITY) return INFINITY;
-    int e = 0;
-    if (x < 1.17549435e-38f) { x = x * 16777216.0f; e = -24; }      // subnormal: scale by 2^24
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float r = __builtin_amdgcn_rcpf(d);
+    return fmaf(fmaf(-d, r, 1.0f), r, r);
+#else
+    return 1.0f / d;
+#endif
+}
+
+__host__ __device__ inline float powf_root_normal(float x, float y, int e = 0)
+{
     const uint32_t b = __builtin_bit_cast(uint32_t, x);
     e += static_cast<int>((b >> 23) & 0xffu) - 127;
     float m = __builtin_bit_cast(float, (b & 0x007fffffu) | 0x3f800000u);   // [1, 2)
@@ -260,7 +282,7 @@ __host__ __device__ inline float powf_root(float x, float y)
     const float num = m - 1.0f;                           // exact
     const float den = m + 1.0f;
     const float den_lo = m - (den - 1.0f);                // den + den_lo = m + 1 exactly
-    const float rden = 1.0f / den;                        // one IEEE reciprocal for s and s_lo
+    const float rden = recip_normal(den);                 // one IEEE reciprocal for s and s_lo
     const float s = num * rden;
     float rem = fmaf(-s, den, num);                       // remainder, to a rounding of 2^-24 of itself
     rem = fmaf(-s, den_lo, rem);
@@ -299,6 +321,15 @@ __host__ __device__ inline float powf_root(float x, float y)
     q = fmaf(q, w, 1.0f);
     q = fmaf(q, w, 1.0f);
     return ldexpf(q, static_cast<int>(k));
+}
+
+__host__ __device__ inline float powf_root(float x, float y)
+{
+    if (!(x > 0.0f)) return x == 0.0f ? 0.0f : NAN;
+    if (x == 1.0f) return 1.0f;
+    if (x == INFINITY) return INFINITY;
+    if (x < 1.17549435e-38f) return powf_root_normal(x * 16777216.0f, y, -24);   // subnormal: scaled by 2^24
+    return powf_root_normal(x, y);
 }
 
 // cos(t) in double for |t| <= 2^20 with one fixed operation sequence:

@@ -91,9 +91,19 @@ __device__ __forceinline__ float pm_one(float value, float ug, float ud, float l
     return fminf(fmaxf(fmaf(delta, range, value), lo), hi);
 }
 
+// The same out of line: inlined in a loop, the double constants of its power
+// stay in registers over the whole kernel and halve the waves in flight.
+__device__ __attribute__((noinline)) float pm_call(float value, float ud, float lo, float hi, float exponent,
+                                                   float inv_exponent)
+{
+    return pm_one(value, -1.0f, ud, lo, hi, exponent, inv_exponent, 0.0f);
+}
+
 struct RepArgs {
     int n, d, pairs;
     FastDiv dd;          // division by d
+    int groups;          // groups of four variables per row: ceil(d / 4)
+    FastDiv gd;          // division by groups
     int small;           // pairs * d + d < 2^31: element indices fit the fast division
     const float* px;
     const int32_t* winners;
@@ -208,11 +218,145 @@ __device__ __forceinline__ void sbx_pm_elem(const RepArgs& R, long long e)
     }
 }
 
-// One thread per (pair, variable).
+// One thread per element from `first` on: injected draws, and the tail row.
 template <int kWinners, bool kSmall>
-__global__ __launch_bounds__(256) void sbx_pm_kernel(RepArgs R)
+__global__ __launch_bounds__(256) void sbx_pm_kernel(RepArgs R, long long first)
 {
-    sbx_pm_elem<kWinners, kSmall>(R, static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x);
+    sbx_pm_elem<kWinners, kSmall>(R, first + static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x);
+}
+
+// In-kernel draws: thread t takes up to four neighbouring variables of a pair,
+// so the row addresses, the winners and the index division are shared and rows
+// move in 16-byte pieces (of 4-byte alignment: any d, any view), and its
+// mutations, rare for large d, one after another from a list: a wave runs the
+// mutation as often as its busiest lane needs, not once per variable.  The
+// draws are at least 2^-23 or 0, so SBX needs no special cases of the root.
+// Bound: VALU, most of it the draws (20 64-bit products a variable of a pair).
+// One variable a thread took 6.26 ms at n = 16384, d = 131072, this 5.30 ms; the
+// batch of 256 runs 235 us, now 147 us (it also formed its instance's terms
+// and a 64-bit counter per variable).  An odd tail row is a launch of its own:
+// inlined here, its mutation's constants cost the registers of three waves.
+template <int kWinners, bool kSmall>
+__device__ __forceinline__ void sbx_pm_quad(const RepArgs& R, long long t)
+{
+    const long long paired = static_cast<long long>(R.pairs) * R.groups;
+    if (t >= paired) return;
+    int pair, j0;
+    if (kSmall) {
+        const uint32_t t32 = static_cast<uint32_t>(t);
+        pair = static_cast<int>(fast_div(t32, R.gd));
+        j0 = static_cast<int>(t32 - static_cast<uint32_t>(pair) * static_cast<uint32_t>(R.groups)) * 4;
+    } else {
+        pair = static_cast<int>(t / R.groups);
+        j0 = static_cast<int>(t - static_cast<long long>(pair) * R.groups) * 4;
+    }
+    const int cnt = min(4, R.d - j0);
+    const float* p1 = R.px + static_cast<size_t>(winner_of<kWinners>(R, 2 * pair)) * R.d + j0;
+    const float* p2 = R.px + static_cast<size_t>(winner_of<kWinners>(R, 2 * pair + 1)) * R.d + j0;
+    const float* pb = R.bounds + 2 * static_cast<size_t>(j0);
+    float x1[4], x2[4], bd[8];
+    if (cnt == 4) {
+        __builtin_memcpy(x1, p1, sizeof(x1));
+        __builtin_memcpy(x2, p2, sizeof(x2));
+        __builtin_memcpy(bd, pb, sizeof(bd));
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int s = min(i, cnt - 1);
+            x1[i] = p1[s];
+            x2[i] = p2[s];
+            bd[2 * i] = pb[2 * s];
+            bd[2 * i + 1] = pb[2 * s + 1];
+        }
+    }
+    const uint64_t e0 = static_cast<uint64_t>(pair) * static_cast<uint32_t>(R.d) + static_cast<uint32_t>(j0);
+    const auto draw = [&](int i, uint32_t stream) {
+        const uint64_t e = e0 + static_cast<uint32_t>(i);
+        return draw4(R.seed, kSmall ? static_cast<uint64_t>(static_cast<uint32_t>(e)) : e, R.gen, stream);
+    };
+    float ca[4], cb[4];
+    uint32_t pending = 0;              // mutations: bit i child a, bit 4 + i child b
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const U4 rs = draw(i, kStSbx);
+        const float ub = u01(rs.x), up = u01(rs.y), uc = u01(rs.z);
+        const bool lower = ub < 0.5f;
+        const float twice = 2.0f * ub;
+        const float base = lower ? twice : recip_normal(2.0f - twice);
+        float beta = powf_root_normal(base, R.power_c);
+        beta = (base == 0.0f) ? 0.0f : beta;
+        beta = beta * static_cast<float>(2 * sbx_direction(rs) - 1);
+        const float lo = bd[2 * i], hi = bd[2 * i + 1];
+        const float mid = 0.5f * (x1[i] + x2[i]);
+        const float delta = 0.5f * beta * (x1[i] - x2[i]);
+        const bool copy = up >= R.prob_c || uc < R.copy_c;
+        ca[i] = copy ? x1[i] : fminf(fmaxf(mid + delta, lo), hi);
+        cb[i] = copy ? x2[i] : fminf(fmaxf(mid - delta, lo), hi);
+        if (i < cnt) {
+            pending |= (u01(rs.w) < R.rate_m) ? 1u << i : 0u;
+            pending |= (gate_b(rs) < R.rate_m) ? 16u << i : 0u;
+        }
+    }
+    if (!R.mutate) pending = 0;
+    while (pending) {
+        const int s = __builtin_ctz(pending), i = s & 3;
+        pending &= pending - 1;
+        const U4 rp = draw(i, kStPm);
+        float v = ca[0], lo = bd[0], hi = bd[1];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            v = (s == q) ? ca[q] : (s == 4 + q) ? cb[q] : v;
+            lo = (i == q) ? bd[2 * q] : lo;
+            hi = (i == q) ? bd[2 * q + 1] : hi;
+        }
+        v = pm_call(v, u01(s < 4 ? rp.x : rp.y), lo, hi, R.exp_m, R.inv_exp_m);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            ca[q] = (s == q) ? v : ca[q];
+            cb[q] = (s == 4 + q) ? v : cb[q];
+        }
+    }
+    float* oa = R.ox + static_cast<size_t>(2 * pair) * R.d + j0;
+    float* ob = oa + R.d;
+    if (cnt == 4) {
+        __builtin_memcpy(oa, ca, sizeof(ca));
+        __builtin_memcpy(ob, cb, sizeof(cb));
+    } else {
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            if (i < cnt) { oa[i] = ca[i]; ob[i] = cb[i]; }
+    }
+}
+
+template <int kWinners, bool kSmall>
+__global__ __launch_bounds__(256) void sbx_pm_quads(RepArgs R)
+{
+    sbx_pm_quad<kWinners, kSmall>(R, static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x);
+}
+
+template <int kWinners>
+int launch_sbx_pm(RepArgs& R, hipStream_t st)
+{
+    R.groups = (R.d + 3) / 4;
+    R.gd = fast_div_make(static_cast<uint32_t>(R.groups));
+    const bool injected = R.sbx_u || R.pm_gate;
+    const long long paired = static_cast<long long>(R.pairs) * R.d;
+    const long long tail = (R.n & 1) ? R.d : 0;
+    const dim3 block(256);
+    if (!injected && R.pairs > 0) {
+        const dim3 grid(static_cast<unsigned>((static_cast<long long>(R.pairs) * R.groups + 255) / 256));
+        if (R.small) hipLaunchKernelGGL((sbx_pm_quads<kWinners, true>), grid, block, 0, st, R);
+        else hipLaunchKernelGGL((sbx_pm_quads<kWinners, false>), grid, block, 0, st, R);
+        MOEA_HIP(hipGetLastError());
+    }
+    const long long first = injected ? 0 : paired, count = paired + tail - first;
+    if (count > 0) {
+        const dim3 grid(static_cast<unsigned>((count + 255) / 256));
+        if (R.small) hipLaunchKernelGGL((sbx_pm_kernel<kWinners, true>), grid, block, 0, st, R, first);
+        else hipLaunchKernelGGL((sbx_pm_kernel<kWinners, false>), grid, block, 0, st, R, first);
+    }
+    MOEA_HIP(hipGetLastError());
+    return kOk;
 }
 
 // Population::initialize_random (core/population.cu:97-115):
@@ -276,7 +420,8 @@ __global__ __launch_bounds__(256) void b_sbx_pm_kernel(const BInst* __restrict__
     const int cur = I.cur, off = (I.cur + 1) % 3, gen = I.gen;
     RepArgs R{};
     R.n = I.n; R.d = I.d; R.pairs = I.n / 2;
-    R.dd = I.ddiv;
+    R.groups = (I.d + 3) / 4;
+    R.gd = I.gdiv;
     R.small = (static_cast<long long>(R.pairs) + 1) * R.d < (1ll << 31);
     R.px = I.x[cur]; R.winners = I.winners; R.bounds = I.bounds;
     R.eta_c = annealed_hd(I.sbx_eta0, I.sbx_eta1, gen, I.max_gen);
@@ -286,7 +431,9 @@ __global__ __launch_bounds__(256) void b_sbx_pm_kernel(const BInst* __restrict__
     R.rate_m = I.pm_prob / static_cast<float>(I.d);
     R.seed = I.seed; R.gen = static_cast<uint32_t>(gen); R.ox = I.x[off];
     set_derived(R);
-    sbx_pm_elem<0>(R, static_cast<long long>(local) * blockDim.x + threadIdx.x);
+    const long long t = static_cast<long long>(local) * blockDim.x + threadIdx.x;
+    if (R.small) sbx_pm_quad<0, true>(R, t);
+    else sbx_pm_quad<0, false>(R, t);
 }
 
 }  // namespace
@@ -329,12 +476,7 @@ int mutate_rows(const float* x_in, float* x_out, int n, int d, const float* boun
     R.mutate = 1; R.eta_m = pm_eta; R.rate_m = pm_prob / static_cast<float>(d);
     R.seed = seed; R.gen = static_cast<uint32_t>(generation); R.ox = x_out;
     set_derived(R);
-    const long long total = static_cast<long long>(R.pairs) * d + ((n & 1) ? d : 0);
-    const dim3 grid(static_cast<unsigned>((total + 255) / 256));
-    if (R.small) hipLaunchKernelGGL((sbx_pm_kernel<2, true>), grid, dim3(256), 0, st, R);
-    else hipLaunchKernelGGL((sbx_pm_kernel<2, false>), grid, dim3(256), 0, st, R);
-    MOEA_HIP(hipGetLastError());
-    return kOk;
+    return launch_sbx_pm<2>(R, st);
 }
 
 int reproduce(const moea_reproduce_args& A)
@@ -368,17 +510,7 @@ int reproduce(const moea_reproduce_args& A)
             return fail(kInvalidArgument, "reproduce: partially injected draw set");
     }
     R.seed = A.seed; R.gen = gen; R.ox = A.offspring_x;
-    const long long total = static_cast<long long>(R.pairs) * A.d + ((A.n & 1) ? A.d : 0);
-    const dim3 grid(static_cast<unsigned>((total + 255) / 256));
-    if (A.mating == MOEA_MATING_GIVEN) {
-        if (R.small) hipLaunchKernelGGL((sbx_pm_kernel<1, true>), grid, dim3(256), 0, st, R);
-        else hipLaunchKernelGGL((sbx_pm_kernel<1, false>), grid, dim3(256), 0, st, R);
-    } else {
-        if (R.small) hipLaunchKernelGGL((sbx_pm_kernel<0, true>), grid, dim3(256), 0, st, R);
-        else hipLaunchKernelGGL((sbx_pm_kernel<0, false>), grid, dim3(256), 0, st, R);
-    }
-    MOEA_HIP(hipGetLastError());
-    return kOk;
+    return A.mating == MOEA_MATING_GIVEN ? launch_sbx_pm<1>(R, st) : launch_sbx_pm<0>(R, st);
 }
 
 int init_population(float* x, int n, int d, const float* bounds, uint64_t seed, hipStream_t stream)
