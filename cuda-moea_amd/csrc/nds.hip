@@ -752,9 +752,16 @@ __device__ __forceinline__ bool peel_body(const PeelArgs& P, int g, int G, uint6
         if (rb >= nblk) continue;
         const int p = rb * 64 + lane;
         s_cur[j * 64 + lane] = (P.rend && p < P.n) ? P.rend[p] : P.hi[rb] + 1;
-        if (lane == 0) { st_relaxed_u64(&P.A0[rb], 0ull); st_relaxed_u64(&P.A1[rb], 0ull); }
+        if (G > 1 && lane == 0) { st_relaxed_u64(&P.A0[rb], 0ull); st_relaxed_u64(&P.A1[rb], 0ull); }
     }
-    if (!coherent_barrier(P.state, g, G, phase, P.spin_limit)) { peel_fail(P); return false; }
+    // a group of one keeps the assigned set and the total to itself, in LDS
+    if (G == 1) {
+        for (int w = threadIdx.x; w < nblk; w += kPeelThreads) s_A[w] = 0ull;
+        __syncthreads();
+    } else if (!coherent_barrier(P.state, g, G, phase, P.spin_limit)) {
+        peel_fail(P);
+        return false;
+    }
     if (nf == 0) {
         peel_finish(P, g, G, nf, ne, -1, true, s_front, s_A);
         return true;
@@ -764,7 +771,8 @@ __device__ __forceinline__ bool peel_body(const PeelArgs& P, int g, int G, uint6
     for (int k = 0;; ++k) {
         const uint64_t* Acur = (k & 1) ? P.A1 : P.A0;
         uint64_t* Anext = (k & 1) ? P.A0 : P.A1;
-        for (int w = threadIdx.x; w < nblk; w += kPeelThreads) s_A[w] = ld_relaxed_u64(&Acur[w]);
+        if (G > 1)
+            for (int w = threadIdx.x; w < nblk; w += kPeelThreads) s_A[w] = ld_relaxed_u64(&Acur[w]);
         if (threadIdx.x == 0) { s_count = 0; s_nq[0] = 0; s_nq[1] = 0; }
         __syncthreads();
 
@@ -851,10 +859,14 @@ __device__ __forceinline__ bool peel_body(const PeelArgs& P, int g, int G, uint6
         __syncthreads();
         for (int j = threadIdx.x; j < bpg; j += kPeelThreads) {
             const int rb = g + j * G;
-            if (rb < nblk) st_relaxed_u64(&Anext[rb], s_A[rb] | s_next[j]);
+            if (rb < nblk) {
+                const uint64_t now = s_A[rb] | s_next[j];
+                if (G == 1) s_A[rb] = now;
+                else st_relaxed_u64(&Anext[rb], now);
+            }
             s_next[j] = 0ull;
         }
-        if (threadIdx.x == 0 && s_count)
+        if (G > 1 && threadIdx.x == 0 && s_count)
             __hip_atomic_fetch_add(&P.state[kPeelTotal], static_cast<uint32_t>(s_count), __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
         // the running total is read from the snapshot block 0 takes inside
@@ -862,8 +874,16 @@ __device__ __forceinline__ bool peel_body(const PeelArgs& P, int g, int G, uint6
         // faster blocks already add for the next round, or the blocks could
         // disagree about stopping and strand each other at the next barrier
         const int snap = kPeelTotal + 4 + (k & 1);
-        if (!coherent_barrier(P.state, g, G, phase, P.spin_limit, kPeelTotal, snap)) { peel_fail(P); return false; }
-        const int total = static_cast<int>(ld_relaxed_u32(&P.state[snap]));
+        int total = total_prev + s_count;
+        if (G == 1) {
+            __syncthreads();
+        } else {
+            if (!coherent_barrier(P.state, g, G, phase, P.spin_limit, kPeelTotal, snap)) {
+                peel_fail(P);
+                return false;
+            }
+            total = static_cast<int>(ld_relaxed_u32(&P.state[snap]));
+        }
         if (total >= P.stop_at || total == total_prev || total >= nf) {
             // the infeasible rows follow once every feasible one is assigned
             peel_finish(P, g, G, nf, ne, (total == total_prev) ? k - 1 : k, total >= nf && total < P.stop_at, s_front,
@@ -878,6 +898,20 @@ __global__ __launch_bounds__(kPeelThreads) void nds_peel(PeelArgs P)
 {
     extern __shared__ uint64_t s_dyn[];
     peel_body(P, static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x), s_dyn);
+}
+
+// The same with one workgroup, which needs no grid barrier and so no
+// cooperative launch (that leaves the device idle for about 10 us on each
+// side).  Up to kOneGroupBlocks row blocks its 16 waves hold two blocks each,
+// and the rounds cost less than the barriers of more workgroups: the sort's
+// peel stage of 184 rows took 28 us cooperatively, now 7 us, of 2048 rows 32 us,
+// now 20 us.
+constexpr int kOneGroupBlocks = 32;
+
+__global__ __launch_bounds__(kPeelThreads) void nds_peel_one(PeelArgs P)
+{
+    extern __shared__ uint64_t s_dyn[];
+    peel_body(P, 0, 1, s_dyn);
 }
 
 // ---------------------------------------------------------------- batched --
@@ -1144,7 +1178,7 @@ int nds_run(const float* f, int ldf, const float* cv, int n, int m, int stop_at,
     MOEA_HIP(hipGetLastError());
     stage_end(kStDominance, stream);
 
-    const int grid = peel_grid_size(W);
+    const int grid = W <= kOneGroupBlocks ? 1 : peel_grid_size(W);
     if (grid <= 0) return fail(kUnsupported, "nds: peel kernel cannot be resident on this device");
     const int bpg = ceil_div(W, grid);
     const size_t lds = peel_lds_bytes(W, bpg);
@@ -1152,7 +1186,10 @@ int nds_run(const float* f, int ldf, const float* cv, int n, int m, int stop_at,
                   peel_spin_limit(), error, L.gmask, L.info};
     void* kargs[] = {&args};
     stage_begin(kStPeel, stream);
-    MOEA_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(nds_peel), dim3(grid),
+    if (grid == 1)
+        hipLaunchKernelGGL(nds_peel_one, dim3(1), dim3(kPeelThreads), static_cast<unsigned>(lds), stream, args);
+    else
+        MOEA_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(nds_peel), dim3(grid),
                                         dim3(kPeelThreads), kargs, static_cast<unsigned>(lds), stream));
     MOEA_HIP(hipGetLastError());
     stage_end(kStPeel, stream);
