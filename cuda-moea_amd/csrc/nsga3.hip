@@ -626,6 +626,162 @@ __global__ __launch_bounds__(kSolveThreads) void norm_solve(const float* __restr
     norm_solve_body(fn, nm, m, asf_val, asf_idx, row_max, meta, a_out, gidx, out_ext, out_a);
 }
 
+// The stages between the sort and the association (front_counts, front_scatter,
+// norm_prep, norm_solve) in one workgroup, for small populations: the four
+// launches take 3 to 8 us each, mostly latency.  kRows merged rows a thread, all
+// in registers: 2 up to 2n = 2048, 4 up to 2n = 4096 (two there cost the smaller
+// sizes nothing, eight cost them 5 us).  Stage time, four launches -> one, in us:
+//     2n      M = 2          M = 3          M = 5          M = 10
+//     128     24.0 -> 11.8   32.6 -> 19.3   52.9 -> 33.0   94.3 -> 72.7
+//     2048    25.1 -> 15.2   33.6 -> 23.3   53.1 -> 38.6   96.7 -> 84.3
+//     4096    29.5 -> 20.2   37.8 -> 28.2   55.8 -> 42.9   103 -> 93.1
+// At 8192 rows (eight a thread) it is 3 us for M <= 3 and a loss of 2 us at
+// M = 10, so the line lies at 4096.
+constexpr int kPrepThreads = 1024;
+constexpr int kPrepOneMaxNm = 4 * kPrepThreads;
+constexpr int kPrepWaves = kPrepThreads / 64;
+
+template <int M, int kRows>
+__global__ __launch_bounds__(kPrepThreads) void select_prep_one(
+    const float* __restrict__ fm, int nm, int n, const int32_t* __restrict__ fronts, int32_t* __restrict__ meta,
+    int32_t* __restrict__ gidx, uint8_t* __restrict__ flag, float* __restrict__ fn, int32_t* __restrict__ rho, int k,
+    const float* __restrict__ omin, int nbo, float* __restrict__ ideal_io, float* __restrict__ a_out,
+    int32_t* __restrict__ out_ext, double* __restrict__ out_a)
+{
+    __shared__ int s_wave[64];
+    __shared__ int s_gidx[kRows * kPrepThreads];
+    __shared__ float s_ideal[M];
+    __shared__ float s_best[kPrepWaves][M], s_max[kPrepWaves][M];
+    __shared__ int s_bidx[kPrepWaves][M];
+    __shared__ __align__(16) SolveLds s_solve;
+    const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = tid >> 6;
+    const int mf = meta[kMaxFront];
+    for (int j = tid; j < k; j += kPrepThreads) rho[j] = 0;
+    // running ideal from merge_objectives' per-block minima (norm_prep)
+    if (tid < M) {
+        float z = INFINITY;
+        for (int b = 0; b < nbo; ++b) z = fminf(z, omin[b * M + tid]);
+        z = fminf(ideal_io[tid], z);
+        s_ideal[tid] = z;
+        ideal_io[tid] = z;
+    }
+    // prior and last front, each ascending; both positions from one scan (front_scatter)
+    int fr[kRows], packed = 0;
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) {
+        const int i = tid + u * kPrepThreads;
+        fr[u] = i < nm ? fronts[i] : -1;
+        if (i < nm) flag[i] = prior_survivor(fr[u], mf, i, n) ? 1 : 0;
+        packed += ((fr[u] >= 0 && fr[u] < mf) ? 1 : 0) + ((fr[u] == mf) ? 0x10000 : 0);
+    }
+    if (mf < 0) {
+        // the sort failed on the device: keep the parents, and flag it
+        for (int i = tid; i < n; i += kPrepThreads) gidx[i] = i;
+        if (tid == 0) {
+            meta[kNPrior] = n;
+            meta[kNLast] = 0;
+            meta[kNRem] = 0;
+            meta[kIll] = -1;
+            meta[kDevError] = 1;
+        }
+        return;
+    }
+    int total;
+    block_exclusive_scan(packed, s_wave, total);
+    const int n_prior = total & 0xFFFF, n_last = total >> 16;
+    int op = 0, ol = n_prior;
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) {
+        const int i = tid + u * kPrepThreads;
+        const int fp = (fr[u] >= 0 && fr[u] < mf) ? 1 : 0, fl = (i < nm && fr[u] == mf) ? 1 : 0;
+        int c;
+        const int e = block_exclusive_scan(fp | (fl << 16), s_wave, c);
+        const int at = fp ? op + (e & 0xFFFF) : ol + (e >> 16);
+        if (fp | fl) {
+            gidx[at] = i;
+            s_gidx[at] = i;
+        }
+        op += c & 0xFFFF;
+        ol += c >> 16;
+    }
+    const int n_nds = n_prior + n_last;
+    if (tid == 0) {
+        meta[kNPrior] = n_prior;
+        meta[kNLast] = n_last;
+        meta[kNRem] = n - n_prior;
+        meta[kIll] = -1;
+        meta[kDevError] = 0;
+    }
+    if (n - n_prior <= 0) return;
+    __syncthreads();
+    // translated objectives, extreme-point and row-max candidates (norm_prep)
+    float best[M], rm[M];
+    int bi[M];
+#pragma unroll
+    for (int j = 0; j < M; ++j) { best[j] = INFINITY; rm[j] = -INFINITY; bi[j] = -1; }
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) {
+        const int i = tid + u * kPrepThreads;
+        if (i >= n_nds) continue;
+        const int s = s_gidx[i];
+        float v[M];
+#pragma unroll
+        for (int c = 0; c < M; ++c) {
+            float t = fm[static_cast<size_t>(c) * nm + s] - s_ideal[c];
+            if (isfinite(t)) t = fmaxf(t, 0.0f);
+            v[c] = t;
+            fn[static_cast<size_t>(c) * nm + i] = t;
+        }
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            float mx = -INFINITY;
+#pragma unroll
+            for (int c = 0; c < M; ++c) {
+                const float t = (v[c] != v[c]) ? INFINITY : v[c];
+                mx = fmaxf(mx, t * ((c == j) ? 1.0f : 1e6f));
+            }
+            if (mx < best[j]) { best[j] = mx; bi[j] = i; }
+            rm[j] = fmaxf(rm[j], (v[j] != v[j]) ? -INFINITY : v[j]);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) {
+            const float ov = __shfl_xor(best[j], o);
+            const int oi = __shfl_xor(bi[j], o);
+            if (oi >= 0 && (bi[j] < 0 || ov < best[j] || (ov == best[j] && oi < bi[j]))) { best[j] = ov; bi[j] = oi; }
+            rm[j] = fmaxf(rm[j], __shfl_xor(rm[j], o));
+        }
+        if (lane == 0) { s_best[wave][j] = best[j]; s_bidx[wave][j] = bi[j]; s_max[wave][j] = rm[j]; }
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    int ext[kMaxM];
+    float rmax[kMaxM];
+#pragma unroll
+    for (int j = 0; j < kMaxM; ++j) { ext[j] = -1; rmax[j] = -INFINITY; }
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+        float b = INFINITY, r = -INFINITY;
+        int e = -1;
+        for (int w = 0; w < kPrepWaves; ++w) {
+            const float ov = s_best[w][j];
+            const int oi = s_bidx[w][j];
+            if (oi >= 0 && (e < 0 || ov < b || (ov == b && oi < e))) { b = ov; e = oi; }
+            r = fmaxf(r, s_max[w][j]);
+        }
+        ext[j] = e;
+        rmax[j] = r;
+    }
+    norm_solve_tail(fn, nm, M, n_nds, ext, rmax, s_solve, meta, a_out, gidx, out_ext, out_a);
+}
+
+template <int M>
+constexpr auto select_prep_2rows = select_prep_one<M, 2>;
+template <int M>
+constexpr auto select_prep_4rows = select_prep_one<M, 4>;
+
 // Perpendicular-distance association against every direction
 // (association.cu:85-188, 397-447): dot by an fmaf chain, residual x - dot*w as
 // one fma, d2 by an fmaf chain, the smallest d2 and of equal ones the first
@@ -2364,14 +2520,22 @@ int nsga3_select(const moea_nsga3_select_args& A)
                        A.stats ? reinterpret_cast<uint32_t*>(A.stats + kDevError) : nullptr, keys_in_merge));
     stage_begin(kStSelectPrep, st);
     const int nsb = ceil_div(nm, kScanThreads);
-    hipLaunchKernelGGL(front_counts, dim3(nsb), dim3(kScanThreads), 0, st, L.fronts, nm, L.meta, L.counts);
-    hipLaunchKernelGGL(front_scatter, dim3(nsb), dim3(kScanThreads), 0, st, L.fronts, nm, n, L.counts, nsb,
-                       L.gidx, L.meta, L.flag);
     const dim3 g_nb(nb), b256(256);
-    MOEA_LAUNCH_M(m, norm_prep, g_nb, b256, 0, st, L.fm, nm, L.gidx, L.meta, L.fn, L.asf_val, L.asf_idx,
-                  L.row_max, L.rho, k, L.omin, nb, A.ideal);
-    hipLaunchKernelGGL(norm_solve, dim3(1), dim3(kSolveThreads), 0, st, L.fn, nm, m, L.asf_val,
-                       L.asf_idx, L.row_max, L.meta, L.a, L.gidx, A.out_extremes, A.out_intercepts);
+    if (nm <= 2 * kPrepThreads) {
+        MOEA_LAUNCH_M(m, select_prep_2rows, dim3(1), dim3(kPrepThreads), 0, st, L.fm, nm, n, L.fronts, L.meta, L.gidx,
+                      L.flag, L.fn, L.rho, k, L.omin, nb, A.ideal, L.a, A.out_extremes, A.out_intercepts);
+    } else if (nm <= kPrepOneMaxNm) {
+        MOEA_LAUNCH_M(m, select_prep_4rows, dim3(1), dim3(kPrepThreads), 0, st, L.fm, nm, n, L.fronts, L.meta, L.gidx,
+                      L.flag, L.fn, L.rho, k, L.omin, nb, A.ideal, L.a, A.out_extremes, A.out_intercepts);
+    } else {
+        hipLaunchKernelGGL(front_counts, dim3(nsb), dim3(kScanThreads), 0, st, L.fronts, nm, L.meta, L.counts);
+        hipLaunchKernelGGL(front_scatter, dim3(nsb), dim3(kScanThreads), 0, st, L.fronts, nm, n, L.counts, nsb,
+                           L.gidx, L.meta, L.flag);
+        MOEA_LAUNCH_M(m, norm_prep, g_nb, b256, 0, st, L.fm, nm, L.gidx, L.meta, L.fn, L.asf_val, L.asf_idx,
+                      L.row_max, L.rho, k, L.omin, nb, A.ideal);
+        hipLaunchKernelGGL(norm_solve, dim3(1), dim3(kSolveThreads), 0, st, L.fn, nm, m, L.asf_val,
+                           L.asf_idx, L.row_max, L.meta, L.a, L.gidx, A.out_extremes, A.out_intercepts);
+    }
     stage_end(kStSelectPrep, st);
     stage_begin(kStAssociation, st);
     if (assoc_prunable(k, m)) {
