@@ -1203,7 +1203,7 @@ int nds_run(const float* f, int ldf, const float* cv, int n, int m, int stop_at,
 // process ends; host code reaches it only through the address that
 // hipGetSymbolAddress reports for the current device (the array's name is a
 // host-side stand-in, not a device address).  Nothing in it needs clearing
-// between calls: nds_block_prep zeroes the peel state and the peel
+// between calls: nds_prep zeroes the peel state and the peel
 // initializes cursors, fronts and the assigned sets.  Calls that overlap on
 // one GPU share the array and race.
 constexpr size_t kStaticScratchBytes = size_t{16} << 20;

@@ -169,11 +169,12 @@ int moea_quantize_cv(const float* cv, float* out, int n, const moea_cv_quantizat
 typedef struct moea_niching {
     int mode;      /* 0 automatic, 1 one workgroup over only the last front's
                       members, grouped by direction (a niche of more than 128
-                      members falls back to that workgroup's radix sorts),
+                      members is cut into parts by value first, or falls back
+                      to that workgroup's radix sorts),
                       2 three device-wide sorts of all 2n slots, 3 the one
                       workgroup's radix sorts only.  The batched and served
                       engines take one workgroup per instance in mode 1, and
-                      in mode 0 while every instance has 2n <= 8192. */
+                      in mode 0 while every instance has 2n <= 16384. */
     int lds_cap;   /* one-workgroup paths: last-front members kept in LDS at
                       most (0: as many as the path's LDS holds, about 9500 for
                       the grouping at K = 32640, 5888 for the radix sorts);
