@@ -218,7 +218,7 @@ __device__ __forceinline__ void sbx_pm_elem(const RepArgs& R, long long e)
     }
 }
 
-// One thread per element from `first` on: injected draws, and the tail row.
+// One thread per element from `first` on: injected draws, smaller calls, the tail row.
 template <int kWinners, bool kSmall>
 __global__ __launch_bounds__(256) void sbx_pm_kernel(RepArgs R, long long first)
 {
@@ -334,22 +334,29 @@ __global__ __launch_bounds__(256) void sbx_pm_quads(RepArgs R)
     sbx_pm_quad<kWinners, kSmall>(R, static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x);
 }
 
+// Four variables a thread from this many pair-variables on.  Below, a variable
+// a thread fills the chip with shorter chains, and an odd last row needs no
+// launch of its own (2.7 us).  One reproduce call, a variable a thread against
+// four: 17.1 / 18.2 us at 4000 x 1000, 77.1 / 82.1 at 8000 x 4000, 88.3 / 86.9 at
+// 32768 x 1024, 191 / 171 at 16384 x 4096, 6296 / 5288 at 16384 x 131072.
+constexpr long long kQuadMinPaired = 1ll << 24;
+
 template <int kWinners>
 int launch_sbx_pm(RepArgs& R, hipStream_t st)
 {
     R.groups = (R.d + 3) / 4;
     R.gd = fast_div_make(static_cast<uint32_t>(R.groups));
-    const bool injected = R.sbx_u || R.pm_gate;
     const long long paired = static_cast<long long>(R.pairs) * R.d;
     const long long tail = (R.n & 1) ? R.d : 0;
+    const bool quads = !R.sbx_u && !R.pm_gate && paired >= kQuadMinPaired;
     const dim3 block(256);
-    if (!injected && R.pairs > 0) {
+    if (quads) {
         const dim3 grid(static_cast<unsigned>((static_cast<long long>(R.pairs) * R.groups + 255) / 256));
         if (R.small) hipLaunchKernelGGL((sbx_pm_quads<kWinners, true>), grid, block, 0, st, R);
         else hipLaunchKernelGGL((sbx_pm_quads<kWinners, false>), grid, block, 0, st, R);
         MOEA_HIP(hipGetLastError());
     }
-    const long long first = injected ? 0 : paired, count = paired + tail - first;
+    const long long first = quads ? paired : 0, count = paired + tail - first;
     if (count > 0) {
         const dim3 grid(static_cast<unsigned>((count + 255) / 256));
         if (R.small) hipLaunchKernelGGL((sbx_pm_kernel<kWinners, true>), grid, block, 0, st, R, first);

@@ -1,8 +1,8 @@
-"""Reproduction with its own draws where four variables go to a thread: rows of
-1 to 9 variables and others that four does not divide, an odd last row, parents
-that begin off a 16-byte line, equal parents, variables at their bounds, with and
-without copying and with up to every variable mutated; offspring bit for bit against the
-oracle."""
+"""Reproduction with its own draws, one and four variables a thread: rows of 1 to
+9 variables and others that four does not divide, an odd last row, parents that
+begin off a 16-byte line, equal parents, variables at their bounds, with and
+without copying and with up to every variable mutated; offspring bit for bit
+against the oracle."""
 import numpy as np
 import pytest
 
@@ -21,10 +21,14 @@ def _f(a):
     return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
 
 
-@pytest.mark.parametrize("d", [1, 2, 3, 4, 5, 7, 8, 9, 63, 254, 1030])
-@pytest.mark.parametrize("n,shift,copy_p,pm_p", [(1, 0, 0.0, 1.0), (2, 1, 0.0, 1.0), (7, 1, 0.5, 40.0),
-                                                 (64, 2, 0.5, 1.0), (101, 3, 0.0, 4.0)])
-def test_reproduce_rows(d, n, shift, copy_p, pm_p):
+# the last two have the 2^24 pair-variables from which four go to a thread
+SIZES = [(n, d, shift, copy_p, pm_p) for d in (1, 2, 3, 4, 5, 7, 8, 9, 63, 254, 1030)
+         for n, shift, copy_p, pm_p in ((1, 0, 0.0, 1.0), (2, 1, 0.0, 1.0), (7, 1, 0.5, 40.0), (64, 2, 0.5, 1.0),
+                                        (101, 3, 0.0, 4.0))] + [(8193, 4099, 1, 0.5, 4.0), (131074, 257, 0, 0.0, 1.0)]
+
+
+@pytest.mark.parametrize("n,d,shift,copy_p,pm_p", SIZES)
+def test_reproduce_rows(n, d, shift, copy_p, pm_p):
     rng = np.random.default_rng(n * 2048 + d)
     lo, hi = np.float32(-1.5), np.float32(2.25)
     x = (lo + (hi - lo) * rng.random((n, d), dtype=np.float32)).astype(np.float32)
