@@ -164,10 +164,12 @@ struct MlpSmem {
 
 // How a matrix's rows are read, four floats at a time: rows that keep 16-byte
 // alignment, any other row length with 16-byte loads of 4-byte alignment (a
-// load near a row's end runs on into the next row; at the matrix's end it is
-// moved back and its numbers shifted into place), or one float at a time where
-// the matrix has fewer than four.  One float at a time for every d that is not
-// a multiple of 4 cost a third more there (2046 x 1333 x 256: 60 us -> 47 us).
+// load near a row's end runs on into the next row; in the last row it is moved
+// back from the matrix's end and its numbers shifted into place), or one float
+// at a time where the matrix has fewer than four numbers, or rows of one: there
+// the loads of the two rows before the last would run past the end as well.  One
+// float at a time for every d that is not a multiple of 4 cost a third more there
+// (2046 x 1333 x 256: 60 us -> 47 us).
 enum MlpLoad : int { kLoadAligned, kLoadAny, kLoadSingle };
 
 // Loads are issued unconditionally from clamped (in-bounds) addresses and the
@@ -381,7 +383,7 @@ __device__ __forceinline__ void mlp_hidden_block(const float* __restrict__ x, in
     if (!mlp_tile_of(local, (n + T::BM - 1) / T::BM, (hidden + T::BN - 1) / T::BN, rt, ct)) return;
     const int r0 = rt * T::BM, c0 = ct * T::BN;
     if ((d & 3) == 0) mlp_hidden_tile<T, kLoadAligned>(x, n, d, w1, hidden, h, r0, c0, sm, rowsq);
-    else if (static_cast<long long>(min(n, hidden)) * d >= 4)
+    else if (d > 1 && static_cast<long long>(min(n, hidden)) * d >= 4)
         mlp_hidden_tile<T, kLoadAny>(x, n, d, w1, hidden, h, r0, c0, sm, rowsq);
     else mlp_hidden_tile<T, kLoadSingle>(x, n, d, w1, hidden, h, r0, c0, sm, rowsq);
 }

@@ -28,11 +28,14 @@ def _fp64(x, w1, w2):
 
 
 # tiles of 64 and 128 rows and columns, slices of 32, rows of every alignment,
-# matrices of fewer than four numbers, folds at 4096, the large tile shape
+# matrices of fewer than four numbers, rows of one to three numbers beside their
+# matrix's end, folds at 4096, the large tile shape
 @pytest.mark.parametrize("n,d,hidden,m", [(1, 1, 1, 1), (1, 3, 1, 2), (3, 1, 5, 3), (2, 2, 2, 1), (1, 5, 2, 1),
                                           (63, 31, 64, 3), (64, 32, 65, 5), (65, 33, 63, 2), (128, 35, 128, 10),
                                           (129, 64, 130, 4), (200, 4095, 100, 3), (130, 4097, 96, 3),
-                                          (127, 8194, 40, 3), (12288, 37, 256, 5), (12289, 66, 255, 5)])
+                                          (127, 8194, 40, 3), (12288, 37, 256, 5), (12289, 66, 255, 5),
+                                          (4, 1, 4, 2), (5, 1, 3, 1), (9, 1, 64, 3), (70, 1, 65, 3), (300, 1, 256, 5),
+                                          (24577, 1, 256, 3), (4, 2, 4, 1), (70, 2, 64, 3), (4, 3, 5, 2), (70, 3, 65, 3)])
 def test_mlp_sizes_against_fp64(n, d, hidden, m):
     x, w1, w2 = _case(n, d, hidden, m)
     print(f"mlp n={n} d={d} hidden={hidden} m={m}", flush=True)
