@@ -1574,7 +1574,8 @@ __device__ __attribute__((noinline)) void niche_body(Bufs B, NicheArgs A, NicheS
 // as it has members by a linear map of the key's value (niche_refine): members
 // are then counted against their own part only.  The radix sorts remain for
 // values too unevenly spread for that, for a last front past the LDS capacity
-// with large niches, and for more than 65535 members (16-bit positions).  On a
+// with large niches, and for more than 65535 members or directions (16-bit
+// positions and direction words).  On a
 // batch of 256 runs whose largest gather 8192 members in a few of 91 niches the
 // radix sorts took 218 us, counting without the cut 1484 us, this 71 us.
 constexpr int kNicheLdsBytes = 162816;
@@ -1983,7 +1984,7 @@ __device__ __forceinline__ void niche_last(const NicheArgs& A, const int32_t* __
     const int fixed = 4 * words + 4 * misc_ints;
     int cap_b = (fixed < kNicheLdsBytes) ? ((kNicheLdsBytes - fixed) / kBucketSlotBytes) & ~15 : 0;
     cap_b = min(cap_b, kBucketRegs * kNicheThreads);
-    if (A.bucket && fixed <= kNicheLdsBytes && n_last <= 65535 && n_prior <= 65535) {
+    if (A.bucket && fixed <= kNicheLdsBytes && n_last <= 65535 && n_prior <= 65535 && k <= 65535) {
         uint32_t* table = reinterpret_cast<uint32_t*>(s_raw);
         int32_t* misc = reinterpret_cast<int32_t*>(s_raw + 4 * words);
         for (int j = tid; j < words; j += kNicheThreads) table[j] = 0;
