@@ -141,7 +141,7 @@ __device__ __forceinline__ void tie_runs(const uint64_t* __restrict__ keys, int 
     const int first = b * 64, end = min(n, first + 64);
     const int t = first + lane;
     const uint64_t key = keys[min(t, n - 1)];
-    const uint64_t prev = t > 0 ? keys[min(t, n - 1) - 1] : ~key;
+    const uint64_t prev = (t > 0 && t < n) ? keys[t - 1] : ~key;
     const uint64_t starts = ballot(t < end && prev != key);
     const uint64_t key_last = keys[end - 1];
     const bool seg0_first = ((keys[first] >> 32) & 3u) == 0, seg0_last = ((key_last >> 32) & 3u) == 0;
