@@ -2007,7 +2007,8 @@ __device__ __forceinline__ void niche_last(const NicheArgs& A, const int32_t* __
                 const int c0 = static_cast<int>(e[i] & 0xFFFFu), c1 = static_cast<int>(e[i] >> 16);
                 sum += c0 + c1;
                 run_max = max(run_max, max(c0, c1));
-                pairs += static_cast<uint32_t>(c0 * c0) + static_cast<uint32_t>(c1 * c1);
+                pairs += static_cast<uint32_t>(c0) * static_cast<uint32_t>(c0) +
+                         static_cast<uint32_t>(c1) * static_cast<uint32_t>(c1);
             }
         }
 #pragma unroll

@@ -51,3 +51,24 @@ def test_few_directions_equal_oracle(n, m, parts, kind):
         nxt, nfr, _ = K.nsga3_select(par, ofs, _f(w), _f(ideal0), seed=5, generation=3, niching=(1, cap))
         np.testing.assert_array_equal(nxt.x[:, 0].cpu().numpy().astype(np.int64), chosen)
         np.testing.assert_array_equal(nfr.cpu().numpy(), fr_mix[chosen])
+
+
+def test_one_direction_65532_members():
+    """The largest niche whose members' positions fit 16 bits (its square needs 32)."""
+    n, m = 32766, 3
+    rng = np.random.default_rng(1)
+    fm = _objectives(rng, "plane", m, 2 * n)
+    cvm = np.zeros(2 * n, np.float32)
+    xm = np.zeros((2 * n, 2), np.float32)
+    xm[:, 0] = np.arange(2 * n, dtype=np.float32)
+    w = np.full((m, 1), 1 / np.sqrt(3), np.float32)
+    ideal0 = fm[:, :n].min(axis=1).astype(np.float32)
+    ua, ub = O.draw_niche(5, 3, 2 * n)
+    chosen, fr_mix, st, _ = O.nsga3_select(fm, cvm, w, ideal0, ua, ub)
+    print(f"niching one direction: n_prior={st[1]} n_last={st[2]}", flush=True)
+    assert st[2] > 46341
+    par = K.Population(_f(xm[:n]), _f(fm[:, :n]), _f(cvm[:n]))
+    ofs = K.Population(_f(xm[n:]), _f(fm[:, n:]), _f(cvm[n:]))
+    nxt, nfr, _ = K.nsga3_select(par, ofs, _f(w), _f(ideal0), seed=5, generation=3)
+    np.testing.assert_array_equal(nxt.x[:, 0].cpu().numpy().astype(np.int64), chosen)
+    np.testing.assert_array_equal(nfr.cpu().numpy(), fr_mix[chosen])
