@@ -119,8 +119,12 @@ __global__ __launch_bounds__(256) void b_quadratic_kernel(const BInst* __restric
 // H does not depend on anything else in the launch (the batched launch
 // reproduces the single-run values bit for bit).
 //
-// Infinities, NaN and numbers beyond bf16's largest make the remainders NaN;
-// an element whose sum ends as NaN is summed again by a plain FP32 loop.
+// Infinities, NaN and numbers beyond bf16's largest make the remainders NaN.  A
+// wave whose part of the tile ends with a NaN goes over its rows once more on the
+// FP32 cores (mlp_again), and only its NaN elements take the result, so that no
+// other row changes.  However many such rows there are, that costs about one more
+// pass: 1024 x 2048 x 256 takes 52 us without a NaN and 136 us with one in every
+// row (one lane summing each such element by itself took 3800 us there).
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -194,20 +198,22 @@ __device__ __forceinline__ float4 mlp_raw4(const float* __restrict__ base, int r
     return v;
 }
 
-template <int LOAD>
+// kLoadAny: the last row's end was loaded up to three places too early.
+__device__ __forceinline__ float4 mlp_shift4(float4 v, int row, int nrows, int ld, int k)
+{
+    const int back = (row == nrows - 1 && k < ld) ? k - (ld - 4) : 0;
+    if (back > 0) {
+        const float e1 = v.y, e2 = v.z, e3 = v.w;
+        v.x = back == 1 ? e1 : back == 2 ? e2 : e3;
+        v.y = back == 1 ? e2 : e3;
+        v.z = e3;
+    }
+    return v;
+}
+
 __device__ __forceinline__ float4 mlp_mask4(float4 v, int row, int nrows, int ld, int k)
 {
     const bool r = row < nrows;
-    if constexpr (LOAD == kLoadAny) {
-        // the last row's end: loaded up to three places too early
-        const int back = (row == nrows - 1 && k < ld) ? k - (ld - 4) : 0;
-        if (back > 0) {
-            const float e1 = v.y, e2 = v.z, e3 = v.w;
-            v.x = back == 1 ? e1 : back == 2 ? e2 : e3;
-            v.y = back == 1 ? e2 : e3;
-            v.z = e3;
-        }
-    }
     v.x = (r && k < ld) ? v.x : 0.0f;
     v.y = (r && k + 1 < ld) ? v.y : 0.0f;
     v.z = (r && k + 2 < ld) ? v.z : 0.0f;
@@ -215,11 +221,61 @@ __device__ __forceinline__ float4 mlp_mask4(float4 v, int row, int nrows, int ld
     return v;
 }
 
-// The blocks of column tile 0 also sum (x - 0.5)^2 over each row of their
-// row tile from the x slices they stage (each of the 8 loader lanes of a row
-// sums its 4 columns of every slice, then a fixed xor reduction over the 8)
-// and store it in rowsq[row]; the head reads it there instead of reading x
-// again.
+// The NaN elements of a wave's 32 x (32 TN) part of H at (row0, col0), once more
+// on the FP32 cores, straight from memory: lane group g takes k = 16 g + t of a
+// slice in step t.  No barrier: other waves of the tile may have none.
+template <int TN, int LOAD>
+__device__ __forceinline__ void mlp_again(const float* __restrict__ x, int n, int d, const float* __restrict__ w1,
+                                          int hidden, float* h, int row0, int col0)
+{
+    const int lane = static_cast<int>(threadIdx.x & 63), g = lane >> 5, i = lane & 31;
+    f32x16 sum[TN];
+#pragma unroll
+    for (int u = 0; u < TN; ++u)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum[u][r] = 0.0f;
+#pragma unroll 1
+    for (int k0 = 16 * g; k0 < d + 16 * g; k0 += kHK) {
+        float4 a[4], b[TN][4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            a[t] = mlp_raw4<LOAD>(x, row0 + i, n, d, k0 + 4 * t);
+#pragma unroll
+            for (int u = 0; u < TN; ++u) b[u][t] = mlp_raw4<LOAD>(w1, col0 + 32 * u + i, hidden, d, k0 + 4 * t);
+        }
+        if (LOAD == kLoadAny) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                a[t] = mlp_shift4(a[t], row0 + i, n, d, k0 + 4 * t);
+#pragma unroll
+                for (int u = 0; u < TN; ++u) b[u][t] = mlp_shift4(b[u][t], col0 + 32 * u + i, hidden, d, k0 + 4 * t);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const float4 p = mlp_mask4(a[t], row0 + i, n, d, k0 + 4 * t);
+#pragma unroll
+            for (int u = 0; u < TN; ++u) {
+                const float4 q = mlp_mask4(b[u][t], col0 + 32 * u + i, hidden, d, k0 + 4 * t);
+                sum[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(p.x, q.x, sum[u], 0, 0, 0);
+                sum[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(p.y, q.y, sum[u], 0, 0, 0);
+                sum[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(p.z, q.z, sum[u], 0, 0, 0);
+                sum[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(p.w, q.w, sum[u], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < TN; ++u)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int row = row0 + 8 * (r >> 2) + 4 * g + (r & 3), col = col0 + 32 * u + i;
+            if (row < n && col < hidden) {
+                float* e = h + static_cast<size_t>(row) * hidden + col;
+                if (*e != *e) *e = tanhf(sum[u][r]);
+            }
+        }
+}
+
 // Three bf16 parts of four floats, to three LDS rows.
 __device__ __forceinline__ void mlp_split4(float4 v, __bf16* hi, __bf16* mid, __bf16* lo)
 {
@@ -242,6 +298,11 @@ __device__ __forceinline__ void mlp_split4(float4 v, __bf16* hi, __bf16* mid, __
     *reinterpret_cast<uint2*>(lo) = make_uint2(out[2][0], out[2][1]);
 }
 
+// The tile of H at (r0, c0).  The blocks of column tile 0 also sum (x - 0.5)^2
+// over each row of their row tile from the x slices they stage (each of the 8
+// loader lanes of a row sums its 4 columns of every slice, then a fixed xor
+// reduction over the 8) and store it in rowsq[row]; the head reads it there
+// instead of reading x again.
 template <class T, int LOAD>
 __device__ __forceinline__ void mlp_hidden_tile(const float* __restrict__ x, int n, int d,
                                                 const float* __restrict__ w1, int hidden,
@@ -274,9 +335,15 @@ __device__ __forceinline__ void mlp_hidden_tile(const float* __restrict__ x, int
         mlp_split4(v, &sm.part[buf][0][at], &sm.part[buf][1][at], &sm.part[buf][2][at]);
     };
     auto store = [&](int set, int buf, int k0) {
+        if (LOAD == kLoadAny && k0 + kHK > d) {            // the slices past the rows' last whole one
+#pragma unroll
+            for (int j = 0; j < PA; ++j) pa[set][j] = mlp_shift4(pa[set][j], r0 + lrow + kRows * j, n, d, k0 + lk);
+#pragma unroll
+            for (int j = 0; j < PB; ++j) pb[set][j] = mlp_shift4(pb[set][j], c0 + lrow + kRows * j, hidden, d, k0 + lk);
+        }
 #pragma unroll
         for (int j = 0; j < PA; ++j) {
-            const float4 v = mlp_mask4<LOAD>(pa[set][j], r0 + lrow + kRows * j, n, d, k0 + lk);
+            const float4 v = mlp_mask4(pa[set][j], r0 + lrow + kRows * j, n, d, k0 + lk);
             put(buf, lrow + kRows * j, v);
             if (sq) {
                 const float t0 = v.x - 0.5f, t1 = v.y - 0.5f, t2 = v.z - 0.5f, t3 = v.w - 0.5f;
@@ -289,7 +356,7 @@ __device__ __forceinline__ void mlp_hidden_tile(const float* __restrict__ x, int
         }
 #pragma unroll
         for (int j = 0; j < PB; ++j)
-            put(buf, T::BM + lrow + kRows * j, mlp_mask4<LOAD>(pb[set][j], c0 + lrow + kRows * j, hidden, d, k0 + lk));
+            put(buf, T::BM + lrow + kRows * j, mlp_mask4(pb[set][j], c0 + lrow + kRows * j, hidden, d, k0 + lk));
     };
     f32x16 acc[TN], total[TN];
 #pragma unroll
@@ -355,23 +422,18 @@ __device__ __forceinline__ void mlp_hidden_tile(const float* __restrict__ x, int
         }
     }
     // D of a 32 x 32 MFMA tile: lane (g, i) holds rows 8 (r / 4) + 4 g + r % 4 of column i
+    bool nan = false;
 #pragma unroll
     for (int u = 0; u < TN; ++u)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int row = r0 + wm * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
             const int col = c0 + (wn * TN + u) * 32 + i;
-            if (row < n && col < hidden) {
-                float v = total[u][r];
-                if (v != v) {
-                    v = 0.0f;
-                    const float* xr = x + static_cast<size_t>(row) * d;
-                    const float* wr = w1 + static_cast<size_t>(col) * d;
-                    for (int k = 0; k < d; ++k) v = fmaf(xr[k], wr[k], v);
-                }
-                h[static_cast<size_t>(row) * hidden + col] = tanhf(v);
-            }
+            const float v = total[u][r];
+            nan = nan || v != v;
+            if (row < n && col < hidden) h[static_cast<size_t>(row) * hidden + col] = tanhf(v);
         }
+    if (ballot(nan)) mlp_again<TN, LOAD>(x, n, d, w1, hidden, h, r0 + wm * 32, c0 + wn * TN * 32);
 }
 
 template <class T>

@@ -62,3 +62,42 @@ def test_mlp_infinite_and_nan_rows():
     assert bool(torch.isinf(f[:, 6]).all())               # every hidden unit saturates, the distance is infinite
     assert bool(torch.isnan(f[:, 7]).all())
     assert bool(torch.isinf(f[:, 8]).all())               # (3.4e38)^2 overflows in the distance only
+
+
+# both tile shapes, each way of loading
+@pytest.mark.parametrize("n,d,hidden,m", [(70, 45, 64, 3), (130, 64, 65, 2), (9, 1, 64, 3), (12289, 66, 255, 5), (12288, 4100, 256, 2)])
+def test_mlp_nan_rows_leave_the_others_alone(n, d, hidden, m):
+    x, w1, w2 = _case(n, d, hidden, m)
+    print(f"mlp nan rows n={n} d={d} hidden={hidden} m={m}", flush=True)
+    clean, _ = K.eval_mlp(x.to(DEV), w1.to(DEV), w2.to(DEV))
+    x[1, d - 1], x[n - 1, 0], x[n // 2, d // 2] = np.nan, np.inf, -np.inf
+    f, _ = K.eval_mlp(x.to(DEV), w1.to(DEV), w2.to(DEV))
+    bad = [1, n // 2, n - 1]
+    ref = _fp64(x[bad], w1, w2)
+    f, clean = f.cpu(), clean.cpu()
+    assert torch.equal(torch.isnan(f[:, bad]), torch.isnan(ref)) and torch.equal(torch.isinf(f[:, bad]), torch.isinf(ref))
+    f[:, bad] = clean[:, bad]
+    assert torch.equal(f, clean)
+
+
+def test_mlp_time_with_nan_rows():
+    """A NaN in every row costs about one more pass (2.6 times the time), not a loop per element (36 times)."""
+    x, w1, w2 = (t.to(DEV) for t in _case(1024, 2048, 256, 3))
+    bad = x.clone()
+    bad[:, 1000] = np.nan
+
+    def best(v):
+        times = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(3):
+                K.eval_mlp(v, w1, w2)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    clean, nan = best(x), best(bad)
+    print(f"mlp 1024 x 2048 x 256: {clean / 3 * 1e3:.0f} us, with NaN rows {nan / 3 * 1e3:.0f} us", flush=True)
+    assert nan < 8 * clean
