@@ -95,7 +95,8 @@ __global__ __launch_bounds__(256) void b_quadratic_kernel(const BInst* __restric
 // MLP hidden layer H = tanh(X W1^T): (n, d) x (hidden, d)^T -> (n, hidden),
 // float products on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16).  Every
 // float is split into three bf16 numbers that sum to it exactly (8 + 8 + 8
-// significant bits, each the rounded remainder), and of the nine products of
+// significant bits, each the rounded remainder; W1 from 2^-110 up, below that
+// to 2^-134), and of the nine products of
 // two such sums the six above 2^-24 of the whole are accumulated in FP32,
 // smallest first: hi lo, lo hi, mid mid, mid hi, hi mid, hi hi.  What is left
 // out is below half a unit in the last place of a float product; a step adds
@@ -119,12 +120,19 @@ __global__ __launch_bounds__(256) void b_quadratic_kernel(const BInst* __restric
 // H does not depend on anything else in the launch (the batched launch
 // reproduces the single-run values bit for bit).
 //
-// Infinities, NaN and numbers beyond bf16's largest make the remainders NaN.  A
-// wave whose part of the tile ends with a NaN goes over its rows once more on the
-// FP32 cores (mlp_again), and only its NaN elements take the result, so that no
-// other row changes.  However many such rows there are, that costs about one more
-// pass: 1024 x 2048 x 256 takes 52 us without a NaN and 136 us with one in every
-// row (one lane summing each such element by itself took 3800 us there).
+// X is scaled by 2^32 before its split and the sums by 2^-32 after it: bf16 has no
+// exponents below FP32's, so the parts of a variable under 2^-110 would lose bits
+// that large weights bring back (hidden sums off by 2e-5 for variables near 2^-118
+// and weights near 2^118).  Weights under 2^-110 matter only against variables
+// whose squared distance then outweighs everything else.
+//
+// Infinities, NaN, variables from 2^95, weights beyond bf16's largest and sums
+// from 2^96 do not end as numbers.  A wave whose part of the tile ends with such
+// a sum goes over its rows once more on the FP32 cores (mlp_again), and only
+// those elements take the result, so that no other row changes.  However many
+// such rows there are, that costs about one more pass: 1024 x 2048 x 256 takes
+// 55 us without a NaN and 137 us with one in every row (one lane summing each such
+// element by itself took 3800 us there).
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -135,6 +143,7 @@ constexpr int kHS = kHK + 8;            // LDS row stride, bf16
 // slices in flight, since a slice then costs less than a trip to memory.
 struct MlpBig { static constexpr int BM = 128, BN = 128, WM = 4, WN = 2, SETS = 2; };
 struct MlpSmall { static constexpr int BM = 64, BN = 64, WM = 2, WN = 2, SETS = 2; };
+constexpr float kMlpScale = 4294967296.0f;   // of X
 constexpr int kMlpFold = 4096;          // k after which a partial sum is folded into the total
 constexpr int kMlpBigTiles = 192;       // tiles of the large shape from which it is used
 
@@ -221,7 +230,7 @@ __device__ __forceinline__ float4 mlp_mask4(float4 v, int row, int nrows, int ld
     return v;
 }
 
-// The NaN elements of a wave's 32 x (32 TN) part of H at (row0, col0), once more
+// The elements left as NaN of a wave's 32 x (32 TN) part of H at (row0, col0), once more
 // on the FP32 cores, straight from memory: lane group g takes k = 16 g + t of a
 // slice in step t.  No barrier: other waves of the tile may have none.
 template <int TN, int LOAD>
@@ -344,7 +353,7 @@ __device__ __forceinline__ void mlp_hidden_tile(const float* __restrict__ x, int
 #pragma unroll
         for (int j = 0; j < PA; ++j) {
             const float4 v = mlp_mask4(pa[set][j], r0 + lrow + kRows * j, n, d, k0 + lk);
-            put(buf, lrow + kRows * j, v);
+            put(buf, lrow + kRows * j, make_float4(v.x * kMlpScale, v.y * kMlpScale, v.z * kMlpScale, v.w * kMlpScale));
             if (sq) {
                 const float t0 = v.x - 0.5f, t1 = v.y - 0.5f, t2 = v.z - 0.5f, t3 = v.w - 0.5f;
                 const int kk = k0 + lk;
@@ -422,18 +431,19 @@ __device__ __forceinline__ void mlp_hidden_tile(const float* __restrict__ x, int
         }
     }
     // D of a 32 x 32 MFMA tile: lane (g, i) holds rows 8 (r / 4) + 4 g + r % 4 of column i
-    bool nan = false;
+    bool again = false;
 #pragma unroll
     for (int u = 0; u < TN; ++u)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int row = r0 + wm * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
             const int col = c0 + (wn * TN + u) * 32 + i;
-            const float v = total[u][r];
-            nan = nan || v != v;
-            if (row < n && col < hidden) h[static_cast<size_t>(row) * hidden + col] = tanhf(v);
+            const float v = total[u][r] * (1.0f / kMlpScale);
+            const bool off = !(fabsf(v) < INFINITY);
+            again = again || off;
+            if (row < n && col < hidden) h[static_cast<size_t>(row) * hidden + col] = off ? NAN : tanhf(v);
         }
-    if (ballot(nan)) mlp_again<TN, LOAD>(x, n, d, w1, hidden, h, r0 + wm * 32, c0 + wn * TN * 32);
+    if (ballot(again)) mlp_again<TN, LOAD>(x, n, d, w1, hidden, h, r0 + wm * 32, c0 + wn * TN * 32);
 }
 
 template <class T>

@@ -47,6 +47,25 @@ def test_mlp_sizes_against_fp64(n, d, hidden, m):
     assert not cv.cpu().any()
 
 
+# variables and weights far from one: parts that would fall under bf16's smallest
+# exponents, subnormal variables, sums past the split's range
+@pytest.mark.parametrize("n,d", [(70, 10), (200, 33), (24576, 64)])
+@pytest.mark.parametrize("xe,we", [(-118, 118), (-126, 124), (-135, 125), (60, -60), (20, -110), (-3, 110)])
+def test_mlp_far_magnitudes(n, d, xe, we):
+    hidden = m = 10
+    x, w1, _ = _case(n, d, hidden, m)
+    x, w1 = torch.ldexp(x, torch.tensor(xe)), torch.ldexp(w1, torch.tensor(we))
+    print(f"mlp far n={n} d={d} xe={xe} we={we}", flush=True)
+    f, _ = K.eval_mlp(x.to(DEV), w1.to(DEV), torch.eye(hidden).to(DEV))
+    xd, wd = x.double(), w1.double()
+    ref = _fp64(x, w1, torch.eye(hidden))
+    # d + 4 roundings of each hidden sum, d + 8 of the distance and the objective
+    tol = 2.0 ** -24 * ((2 * (d + 4) * (xd.abs() @ wd.abs().t()).t()).clamp(max=2.0 ** 24) + (d + 8) * ref)
+    if we == 110:                                    # saturated: the units' signs alone
+        tol = 2.0 ** -24 * (d + 8) * ref
+    assert bool(((f.cpu().double() - ref).abs() <= tol).all())
+
+
 def test_mlp_infinite_and_nan_rows():
     n, d, hidden, m = 70, 45, 64, 3
     x, w1, w2 = _case(n, d, hidden, m)
