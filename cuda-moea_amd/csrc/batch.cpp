@@ -80,6 +80,8 @@ void carve_instance(Carve& c, const moea_batch_problem& p, BInst& I)
     I.asf_idx = c.take<int32_t>(static_cast<size_t>(z.nb) * z.m);
     I.row_max = c.take<float>(static_cast<size_t>(z.nb) * z.m);
     I.a = c.take<float>(kMaxM);
+    I.part_d2 = c.take<float>(static_cast<size_t>(assoc_chunks(z.k, z.m)) * z.nm);
+    I.part_idx = c.take<int32_t>(static_cast<size_t>(assoc_chunks(z.k, z.m)) * z.nm);
     I.dist = c.take<float>(z.nm);
     I.ref = c.take<int32_t>(z.nm);
     I.rho = c.take<int32_t>(z.k);
@@ -120,6 +122,7 @@ void fill_record(const moea_batch_problem& p, BInst& I)
     I.n = z.n; I.m = z.m; I.d = z.d; I.k = z.k;
     I.nm = z.nm; I.W = z.W; I.Wc = z.Wc; I.npad = z.npad;
     I.max_gen = p.max_generations;
+    I.nchunks = assoc_chunks(z.k, z.m);
     I.gdiv = fast_div_make(static_cast<uint32_t>((z.d + 3) / 4));
     I.seed = p.seed;
     I.sbx_eta0 = p.sbx_eta[0]; I.sbx_eta1 = p.sbx_eta[1];
@@ -192,6 +195,7 @@ void fix_grids(Grids& G, const int* base)
         fix(G.eval.mlp_rows4[m], base);
         fix(G.sel.norm_prep[m], base);
         fix(G.sel.assoc[m], base);
+        fix(G.sel.assoc_chunks[m], base);
         fix(G.sel.assoc_pruned[m], base);
         fix(G.nds0.dom[m], base);
         fix(G.nds1.dom[m], base);
@@ -217,7 +221,8 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
     std::vector<std::vector<long long>> q4(kMaxM + 1, std::vector<long long>(count, 0)),
         h4(kMaxM + 1, std::vector<long long>(count, 0)), prep(kMaxM + 1, std::vector<long long>(count, 0)),
         assoc(kMaxM + 1, std::vector<long long>(count, 0)), dom0(kMaxM + 1, std::vector<long long>(count, 0)),
-        dom1(kMaxM + 1, std::vector<long long>(count, 0)), apr(kMaxM + 1, std::vector<long long>(count, 0));
+        dom1(kMaxM + 1, std::vector<long long>(count, 0)), apr(kMaxM + 1, std::vector<long long>(count, 0)),
+        chunks(kMaxM + 1, std::vector<long long>(count, 0));
     int max_k = 1, max_nm = 1;
     std::vector<int> peel_inst, peel_W0, peel_W1;
     long long total_merged = 0, total_n = 0;
@@ -241,6 +246,7 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
         }
         prep[m][i] = nb;
         if (I.cones) apr[m][i] = ceil_div(nm, 4);
+        else if (I.nchunks > 0) chunks[m][i] = static_cast<long long>(nb) * I.nchunks;
         else assoc[m][i] = ceil_div(nm, 64);
         n0_rows[i] = ceil_div(n, 256);
         n0_prep[i] = static_cast<long long>(Wc0) * m;
@@ -278,6 +284,7 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
     for (int m = 1; m <= kMaxM; ++m) {
         G.sel.norm_prep[m] = T.add(prep[m]);
         G.sel.assoc[m] = T.add(assoc[m]);
+        G.sel.assoc_chunks[m] = T.add(chunks[m]);
         G.sel.assoc_pruned[m] = T.add(apr[m]);
     }
     G.sel.ref_bits = bitlen(max_k + 1);
@@ -308,8 +315,8 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
     return total_merged;
 }
 
-// Prefix tables per state: (1 + 3 + 2 kMaxM + 1 + 3 + 3 kMaxM + 2 + 2 + 2 kMaxM) grids.
-constexpr int kGridsPerState = 12 + 7 * kMaxM;
+// Prefix tables per state: (1 + 3 + 2 kMaxM + 1 + 3 + 4 kMaxM + 2 + 2 + 2 kMaxM) grids.
+constexpr int kGridsPerState = 12 + 8 * kMaxM;
 
 }  // namespace
 

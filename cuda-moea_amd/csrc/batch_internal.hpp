@@ -31,6 +31,7 @@ struct BInst {
     int n, m, d, k;
     int nm, W, Wc, npad;          // NDS over the 2n merged rows
     int max_gen;
+    int nchunks;                  // assoc_chunks(k, m)
     FastDiv gdiv;                 // division by ceil(d / 4) (reproduction thread indices)
     uint64_t seed;
     float sbx_eta0, sbx_eta1, sbx_prob, sbx_copy, pm_eta0, pm_eta1, pm_prob;
@@ -61,6 +62,8 @@ struct BInst {
     int32_t* asf_idx;             // (ceil(nm / 256), m)
     float* row_max;               // (ceil(nm / 256), m)
     float* a;                     // (kMaxM)
+    float* part_d2;               // (nchunks, nm) association partials, many directions only
+    int32_t* part_idx;            // (nchunks, nm)
     float* dist;                  // (nm)
     int32_t* ref;                 // (nm)
     int32_t* rho;                 // (k)
@@ -143,7 +146,8 @@ struct BSelGrids {
     BGrid rows4;                  // n rows per instance, one wave per row
     BGrid objectives;             // one 1024-thread block per objective per instance
     BGrid norm_prep[kMaxM + 1];   // ceil(2n / 256) blocks, instances with m objectives
-    BGrid assoc[kMaxM + 1];       // ceil(2n / 64) blocks, instances with m objectives and no cone tables
+    BGrid assoc[kMaxM + 1];       // ceil(2n / 64) blocks, instances with m objectives, no cone tables and no chunks
+    BGrid assoc_chunks[kMaxM + 1];// ceil(2n / 256) x chunks, instances with m objectives and chunks
     BGrid assoc_pruned[kMaxM + 1];// ceil(2n / 4), instances with m objectives and cone tables
     int ref_bits;                 // bits of a direction index (with the two sentinels)
     int rank_bits;                // bits of rho + rank (with the sentinel)

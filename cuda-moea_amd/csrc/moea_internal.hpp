@@ -34,6 +34,8 @@ bool cv_quant_valid(const moea_cv_quantization& q);
 int quantize_cv(const float* cv, float* out, int n, const moea_cv_quantization& q, hipStream_t stream);
 // Cone tables of the pruned association, built once per set of directions.
 bool assoc_prunable(int k, int m);
+// Chunks of directions whose partial minima the selection keeps, 0 when it compares them in one kernel or prunes.
+int assoc_chunks(int k, int m);
 size_t cone_bytes(int m, int k);
 void cone_views(void* buf, int m, int k, float** wp, int32_t** perm, float** cones);
 int cones_build(const float* w, int k, int m, void* buf, hipStream_t st);

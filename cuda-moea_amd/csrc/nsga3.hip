@@ -872,6 +872,96 @@ __global__ __launch_bounds__(kAssocThreads) void associate_all(const float* __re
     assoc_all_body<M>(fn, nm, a, w, k, meta, dist, ref, rho, static_cast<int>(blockIdx.x));
 }
 
+// The same for many directions, which the kernel above has too few workgroups
+// for and reads as 16 streams that no longer fit the scalar cache: an individual
+// a thread against a chunk of directions staged in LDS, partial minima in the
+// workspace, and a second kernel that takes the first of their minima.  Above
+// kAssocAllMaxK directions it wins at every M from 64 to 16384 individuals
+// (M = 5, one kernel / chunks, in us: 4096 x 8192 62 / 68, 64 x 12288 90 / 63,
+// 64 x 65536 478 / 78, 16384 x 32640 236 / 207); below, the one kernel does or
+// loses at most 3 % (65536 x 6000: 154 / 150).
+constexpr int kAssocAllMaxK = 8192;
+constexpr int kAssocChunk = 1024;
+
+template <int M>
+__device__ __forceinline__ void assoc_chunk_body(const float* __restrict__ fn, int nm, const float* __restrict__ a,
+                                                 const float* __restrict__ w, int k, const int32_t* __restrict__ meta,
+                                                 float* __restrict__ part_d2, int32_t* __restrict__ part_idx, int bx,
+                                                 int by)
+{
+    __shared__ float s_w[M][kAssocChunk];
+    if (meta[kNRem] <= 0) return;
+    const int n_nds = meta[kNPrior] + meta[kNLast];
+    if (bx * 256 >= n_nds) return;
+    const int j0 = by * kAssocChunk;
+    const int jn = min(kAssocChunk, k - j0);
+    for (int e = threadIdx.x; e < M * kAssocChunk; e += 256) {
+        const int c = e / kAssocChunk, j = e % kAssocChunk;
+        s_w[c][j] = (j < jn) ? w[static_cast<size_t>(c) * k + j0 + j] : 0.0f;
+    }
+    __syncthreads();
+    const int i = bx * 256 + threadIdx.x;
+    if (i >= n_nds) return;
+    float x[M];
+#pragma unroll
+    for (int c = 0; c < M; ++c) x[c] = fn[static_cast<size_t>(c) * nm + i] * a[c];
+    float best = INFINITY;
+    int bj = -1;
+    for (int j = 0; j < jn; ++j) {
+        float dot = 0.0f;
+#pragma unroll
+        for (int c = 0; c < M; ++c) dot = fmaf(x[c], s_w[c][j], dot);
+        float d2 = 0.0f;
+#pragma unroll
+        for (int c = 0; c < M; ++c) {
+            const float r = fmaf(-dot, s_w[c][j], x[c]);
+            d2 = fmaf(r, r, d2);
+        }
+        if (d2 < best) { best = d2; bj = j0 + j; }
+    }
+    part_d2[static_cast<size_t>(by) * nm + i] = best;
+    part_idx[static_cast<size_t>(by) * nm + i] = bj;
+}
+
+// The chunks' minima in chunk order (association_phase2_kernel, :397-447): the
+// first of equal ones has the smallest direction.
+__device__ __forceinline__ void assoc_merge_body(const float* __restrict__ part_d2, const int32_t* __restrict__ part_idx,
+                                                 int nchunks, int nm, const int32_t* __restrict__ meta,
+                                                 float* __restrict__ dist, int32_t* __restrict__ ref,
+                                                 int32_t* __restrict__ rho, int i)
+{
+    if (meta[kNRem] <= 0 || i >= meta[kNPrior] + meta[kNLast]) return;
+    float best = INFINITY;
+    int bj = -1;
+    for (int c = 0; c < nchunks; ++c) {
+        const float d2 = part_d2[static_cast<size_t>(c) * nm + i];
+        if (d2 < best) { best = d2; bj = part_idx[static_cast<size_t>(c) * nm + i]; }
+    }
+    dist[i] = (best != INFINITY) ? sqrtf(best) : INFINITY;
+    ref[i] = bj;
+    if (rho && bj >= 0 && i < meta[kNPrior]) atomicAdd(&rho[bj], 1);
+}
+
+// Grid (ceil(individuals / 256), chunks).
+template <int M>
+__global__ __launch_bounds__(256) void associate_chunks(const float* __restrict__ fn, int nm,
+                                                        const float* __restrict__ a, const float* __restrict__ w,
+                                                        int k, const int32_t* __restrict__ meta,
+                                                        float* __restrict__ part_d2, int32_t* __restrict__ part_idx)
+{
+    assoc_chunk_body<M>(fn, nm, a, w, k, meta, part_d2, part_idx, static_cast<int>(blockIdx.x),
+                        static_cast<int>(blockIdx.y));
+}
+
+__global__ __launch_bounds__(256) void associate_merge(const float* __restrict__ part_d2,
+                                                       const int32_t* __restrict__ part_idx, int nchunks, int nm,
+                                                       const int32_t* __restrict__ meta, float* __restrict__ dist,
+                                                       int32_t* __restrict__ ref, int32_t* __restrict__ rho)
+{
+    assoc_merge_body(part_d2, part_idx, nchunks, nm, meta, dist, ref, rho,
+                     static_cast<int>(blockIdx.x * 256 + threadIdx.x));
+}
+
 // ------------------------------------------------------ pruned association --
 // Exact association with pruning, for many directions.  Directions are cut
 // into blocks of 64 consecutive indices; each block gets a cone (unit center c
@@ -2293,7 +2383,7 @@ __global__ void quantize_cv_kernel(const float* __restrict__ cv, float* __restri
 struct Layout {
     float* fm; float* cvm; float* cvq; int32_t* fronts; int32_t* meta; int32_t* gidx; float* fn;
     float* asf_val; int32_t* asf_idx; float* row_max; float* a; float* omin;
-    float* dist; int32_t* ref; int32_t* rho; ConeBufs cones;
+    float* dist; int32_t* ref; int32_t* rho; float* part_d2; int32_t* part_idx; ConeBufs cones;
     uint64_t* k0; uint64_t* k1; int32_t* v0; int32_t* v1; void* sort_tmp; size_t sort_bytes;
     uint8_t* flag; int32_t* chosen; int32_t* counts; void* nds_ws; size_t nds_bytes;
 };
@@ -2318,6 +2408,8 @@ Layout carve(void* ws, size_t cap, int n, int m, int k, Carve& c)
     L.dist = c.take<float>(nm);
     L.ref = c.take<int32_t>(nm);
     L.rho = c.take<int32_t>(k);
+    L.part_d2 = c.take<float>(static_cast<size_t>(assoc_chunks(k, m)) * nm);
+    L.part_idx = c.take<int32_t>(static_cast<size_t>(assoc_chunks(k, m)) * nm);
     L.cones = carve_cones(c, m, k);
     L.k0 = c.take<uint64_t>(nm);
     L.k1 = c.take<uint64_t>(nm);
@@ -2341,6 +2433,11 @@ Layout carve(void* ws, size_t cap, int n, int m, int k, Carve& c)
 bool assoc_prunable(int k, int m)
 {
     return m <= kConeAutoMaxM && k >= kConeMinK && ceil_div(k, 64) <= kConeMaxBlocks;
+}
+
+int assoc_chunks(int k, int m)
+{
+    return (k > kAssocAllMaxK && !assoc_prunable(k, m)) ? ceil_div(k, kAssocChunk) : 0;
 }
 
 size_t cone_bytes(int m, int k)
@@ -2413,13 +2510,17 @@ __global__ void assoc_meta(int32_t* __restrict__ meta, int n)
 }
 
 struct AssocLayout {
-    int32_t* meta; ConeBufs cones;
+    int32_t* meta; float* part_d2; int32_t* part_idx; int nchunks; ConeBufs cones;
 };
 
-AssocLayout carve_assoc(Carve& c, int m, int k)
+// ld individuals; by method 1 every direction is compared, also where method 0 prunes
+AssocLayout carve_assoc(Carve& c, int ld, int m, int k)
 {
     AssocLayout L{};
     L.meta = c.take<int32_t>(kMetaLen);
+    L.nchunks = k > kAssocAllMaxK ? ceil_div(k, kAssocChunk) : 0;
+    L.part_d2 = c.take<float>(static_cast<size_t>(L.nchunks) * ld);
+    L.part_idx = c.take<int32_t>(static_cast<size_t>(L.nchunks) * ld);
     L.cones = carve_cones(c, m, k);
     return L;
 }
@@ -2430,7 +2531,7 @@ size_t associate_workspace_bytes(int ld, int m, int k)
 {
     if (ld <= 0 || m <= 0 || m > kMaxM || k <= 0) return 0;
     Carve c(nullptr, 0);
-    carve_assoc(c, m, k);
+    carve_assoc(c, ld, m, k);
     return c.used;
 }
 
@@ -2443,7 +2544,7 @@ int associate(const float* fn, int ld, int n, int m, const float* a, const float
     const size_t need = associate_workspace_bytes(ld, m, k);
     if (!ws || ws_bytes < need) return fail(kWorkspaceTooSmall, "associate: workspace too small");
     Carve c(ws, ws_bytes);
-    const AssocLayout L = carve_assoc(c, m, k);
+    const AssocLayout L = carve_assoc(c, ld, m, k);
     const int nbk = ceil_div(k, 64);
     const bool prunable = nbk <= kConeMaxBlocks;
     if (method == 2 && !prunable) return fail(kUnsupported, "associate: too many directions for the pruned path");
@@ -2454,6 +2555,11 @@ int associate(const float* fn, int ld, int n, int m, const float* a, const float
         MOEA_CHECK(cones_prepare(w, k, m, L.cones, st));
         MOEA_LAUNCH_M(m, associate_pruned, dim3(ceil_div(n, 4)), b256, 0, st, fn, ld, a, L.cones.wp, k,
                       L.cones.perm, L.cones.cones, L.meta, dist, ref, nullptr);
+    } else if (L.nchunks > 0) {
+        MOEA_LAUNCH_M(m, associate_chunks, dim3(ceil_div(n, 256), L.nchunks), b256, 0, st, fn, ld, a, w, k, L.meta,
+                      L.part_d2, L.part_idx);
+        hipLaunchKernelGGL(associate_merge, dim3(ceil_div(n, 256)), b256, 0, st, L.part_d2, L.part_idx, L.nchunks, ld,
+                           L.meta, dist, ref, nullptr);
     } else {
         MOEA_LAUNCH_M(m, associate_all, dim3(ceil_div(n, 64)), dim3(kAssocThreads), 0, st, fn, ld, a, w, k, L.meta,
                       dist, ref, nullptr);
@@ -2547,6 +2653,11 @@ int nsga3_select(const moea_nsga3_select_args& A)
         if (!A.directions_ready) MOEA_CHECK(cones_prepare(A.directions, k, m, L.cones, st));
         MOEA_LAUNCH_M(m, associate_pruned, dim3(ceil_div(nm, 4)), b256, 0, st, L.fn, nm, L.a, L.cones.wp, k,
                       L.cones.perm, L.cones.cones, L.meta, L.dist, L.ref, L.rho);
+    } else if (const int nchunks = assoc_chunks(k, m); nchunks > 0) {
+        MOEA_LAUNCH_M(m, associate_chunks, dim3(nb, nchunks), b256, 0, st, L.fn, nm, L.a, A.directions, k, L.meta,
+                      L.part_d2, L.part_idx);
+        hipLaunchKernelGGL(associate_merge, g_nb, b256, 0, st, L.part_d2, L.part_idx, nchunks, nm, L.meta, L.dist,
+                           L.ref, L.rho);
     } else {
         MOEA_LAUNCH_M(m, associate_all, dim3(ceil_div(nm, 64)), dim3(kAssocThreads), 0, st, L.fn, nm, L.a,
                       A.directions, k, L.meta, L.dist, L.ref, L.rho);
@@ -2699,6 +2810,26 @@ __global__ __launch_bounds__(kAssocThreads) void b_assoc_all(const BInst* __rest
     const int i = bmap_find(mp, static_cast<int>(blockIdx.x), local);
     const BInst& I = insts[i];
     assoc_all_body<M>(I.fn, I.nm, I.a, I.dirs, I.k, I.meta, I.dist, I.ref, I.rho, local);
+}
+
+template <int M>
+__global__ __launch_bounds__(256) void b_assoc_chunks(const BInst* __restrict__ insts, BMap mp)
+{
+    int local;
+    const int i = bmap_find(mp, static_cast<int>(blockIdx.x), local);
+    const BInst& I = insts[i];
+    const int nb = (I.nm + 255) / 256;
+    assoc_chunk_body<M>(I.fn, I.nm, I.a, I.dirs, I.k, I.meta, I.part_d2, I.part_idx, local % nb, local / nb);
+}
+
+__global__ __launch_bounds__(256) void b_assoc_merge(const BInst* __restrict__ insts, BMap mp)
+{
+    int local;
+    const int i = bmap_find(mp, static_cast<int>(blockIdx.x), local);
+    const BInst& I = insts[i];
+    if (I.nchunks > 0)
+        assoc_merge_body(I.part_d2, I.part_idx, I.nchunks, I.nm, I.meta, I.dist, I.ref, I.rho,
+                         local * 256 + static_cast<int>(threadIdx.x));
 }
 
 // One wave per individual of the instances with cone tables.
@@ -2877,6 +3008,15 @@ int batch_select(const BatchLaunch& L, const BSelGrids& G, const BNdsGrids& NG, 
         const dim3 grid(G.assoc[m].blocks), block(kAssocThreads);
         MOEA_LAUNCH_M(m, b_assoc_all, grid, block, 0, st, L.insts, G.assoc[m].map);
     }
+    bool chunked = false;
+    for (int m = 1; m <= kMaxM; ++m) {
+        if (G.assoc_chunks[m].blocks <= 0) continue;
+        const dim3 grid(G.assoc_chunks[m].blocks), block(256);
+        MOEA_LAUNCH_M(m, b_assoc_chunks, grid, block, 0, st, L.insts, G.assoc_chunks[m].map);
+        chunked = true;
+    }
+    if (chunked)
+        hipLaunchKernelGGL(b_assoc_merge, dim3(G.merged256.blocks), dim3(256), 0, st, L.insts, G.merged256.map);
     for (int m = 1; m <= kMaxM; ++m) {
         if (G.assoc_pruned[m].blocks <= 0) continue;
         const dim3 grid(G.assoc_pruned[m].blocks), block(256);
