@@ -41,3 +41,26 @@ def test_ranks_at_edges(n, m, kind):
         fr_g, mf_g = K.nds_rank(torch.from_numpy(f).to(DEV), torch.from_numpy(cv).to(DEV), stop)
         assert mf_g == mf_o
         np.testing.assert_array_equal(fr_g.cpu().numpy(), fr_o)
+
+
+@pytest.mark.parametrize("n,m", [(2000, 1), (2500, 1), (2500, 2), (3001, 3), (2300, 5)])
+@pytest.mark.parametrize("kind", ["band", "two chains"])
+def test_many_fronts(n, m, kind):
+    """Hundreds to thousands of fronts that the assigned set fills in sort order, and one where a second chain
+    stays open below the first, with infeasible rows after both."""
+    rng = np.random.default_rng(n + m)
+    i = np.arange(n, dtype=np.float32)
+    f = np.repeat(i[None], m, 0)
+    if kind == "band":
+        f += rng.uniform(0, 8, (m, n)).astype(np.float32)
+    elif m > 1:                                      # the later half is not dominated by the earlier one
+        f[1, n // 2:] -= n
+    p = rng.permutation(n)
+    f = np.ascontiguousarray(f[:, p])
+    cv = np.where(rng.random(n) < 0.1, rng.integers(1, 9, n), 0).astype(np.float32)
+    for stop in (n, n // 3):
+        print(f"nds many fronts n={n} m={m} kind={kind} stop={stop}", flush=True)
+        fr_o, mf_o = O.nds(f, cv, stop)
+        fr_g, mf_g = K.nds_rank(torch.from_numpy(f).to(DEV), torch.from_numpy(cv).to(DEV), stop)
+        assert mf_g == mf_o
+        np.testing.assert_array_equal(fr_g.cpu().numpy(), fr_o)
