@@ -372,13 +372,44 @@ __global__ __launch_bounds__(256) void rv_gamma_tiles(const float* __restrict__ 
     if (j1 < k) atomicMax(&key[j1], order_key(m1));
 }
 
+__device__ __forceinline__ float gamma_of(float mx)
+{
+    return (mx > -INFINITY) ? acosf_det(fminf(fmaxf(mx, 0.0f), 1.0f)) : 3.14159265358979323846f;
+}
+
 __global__ void rv_gamma_finish(float* gamma, int k)
 {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= k) return;
     const uint32_t u = __float_as_uint(gamma[j]);
     const float mx = __uint_as_float((u & 0x80000000u) ? u & 0x7FFFFFFFu : ~u);
-    gamma[j] = (mx > -INFINITY) ? acosf_det(fminf(fmaxf(mx, 0.0f), 1.0f)) : 3.14159265358979323846f;
+    gamma[j] = gamma_of(mx);
+}
+
+// Few directions: a thread per direction against all others, in one launch where
+// the tiles take three (4 to 5 us).  The line lies where this loop, k (M + 3) long
+// in instructions, takes as long as the two launches it saves (one launch / tiles,
+// in us): 8 / 13 at k = 64, M = 5, 12 / 13 at 64, 10, 11 / 13 at 128, 3, 14 / 13 at
+// 128, 5, 18 / 13 at 200, 3.
+constexpr int kGammaOneMax = 900;
+
+template <int M>
+__global__ __launch_bounds__(256) void rv_gamma_one(const float* __restrict__ v, int k, float* __restrict__ gamma)
+{
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= k) return;
+    float q[M];
+#pragma unroll
+    for (int c = 0; c < M; ++c) q[c] = v[static_cast<size_t>(c) * k + j];
+    float mx = -INFINITY;
+    for (int o = 0; o < k; ++o) {
+        if (o == j) continue;
+        float dot = 0.0f;
+#pragma unroll
+        for (int c = 0; c < M; ++c) dot = fmaf(q[c], v[static_cast<size_t>(c) * k + o], dot);
+        mx = fmaxf(mx, dot);
+    }
+    gamma[j] = gamma_of(mx);
 }
 
 // z range over the active columns, then V = normalize(V0 * range)
@@ -529,6 +560,12 @@ int rvea_select(const moea_rvea_select_args& A)
 int rvea_gamma(const float* v, int m, int k, float* gamma, hipStream_t stream)
 {
     if (!v || !gamma || m <= 0 || m > kMaxM || k <= 0) return fail(kInvalidArgument, "rvea_gamma: invalid arguments");
+    if (static_cast<long long>(k) * (m + 3) <= kGammaOneMax) {
+        const dim3 g(ceil_div(k, 256)), b(256);
+        MOEA_LAUNCH_M(m, rv_gamma_one, g, b, 0, stream, v, k, gamma);
+        MOEA_HIP(hipGetLastError());
+        return kOk;
+    }
     // about 1024 workgroups, at least 32 directions q each
     const int rows = ceil_div(k, kGammaRows);
     const int per = std::max(32, ceil_div(ceil_div(k, std::max(1, 1024 / rows)), kGammaGroup) * kGammaGroup);

@@ -18,7 +18,7 @@ def _f(a):
     return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
 
 
-@pytest.mark.parametrize("k,m", [(1, 3), (2, 2), (31, 5), (33, 4), (256, 3), (511, 10), (512, 3), (513, 6), (1500, 2)])
+@pytest.mark.parametrize("k,m", [(1, 3), (2, 2), (31, 5), (33, 4), (69, 10), (70, 10), (150, 3), (151, 3), (225, 1), (226, 1), (256, 3), (511, 10), (512, 3), (513, 6), (1500, 2)])
 def test_gamma_tile_edges(k, m):
     rng = np.random.default_rng(k)
     v = rng.standard_normal((m, k)).astype(np.float32)       # negative products too
