@@ -336,18 +336,20 @@ __global__ __launch_bounds__(256) void sbx_pm_quads(RepArgs R)
 
 // Four variables a thread where that is the faster way, one reproduce call in us, a
 // variable a thread against four:
-//  - from 2^24 pair-variables, or 2^25 where hardly any variable mutates.  Below, a
+//  - from 2^24 pair-variables, or 2^25 where hardly any variable of a long row
+//    mutates.  Below, a
 //    variable a thread fills the chip with shorter chains, and an odd last row needs
 //    no launch of its own (2.7 us): 17.1 / 18.2 at 4000 x 1000, 77.1 / 82.1 at
 //    8000 x 4000; at 2^24 93.8 / 89.5 at 32768 x 1024 (rate 2^-10), 81 / 86 at
-//    4096 x 8192 (2^-13); above 191 / 171 at 16384 x 4096, 6296 / 5288 at
+//    4096 x 8192 (2^-13), without mutation 80 / 86 at d = 256 and 191 / 180 at 16; above 191 / 171 at 16384 x 4096, 6296 / 5288 at
 //    16384 x 131072.
 //  - up to a mutation rate of a quarter of the variables in use: a thread works its
 //    mutations off one after another.  At 2^24 and d = 1024: 215 / 134 at rate 0.1,
 //    217 / 178 at 0.25, 220 / 223 at 0.5, 226 / 243 at 1; at d = 5, where five of
 //    eight are in use, 670 / 652 at 0.1, 671 / 700 at 0.2, 677 / 837 at 1.
 constexpr long long kQuadMinPaired = 1ll << 24;
-constexpr float kQuadMinRate = 1.0f / 2048.0f;    // for fewer than twice as many
+constexpr float kQuadMinRate = 1.0f / 2048.0f;    // for fewer than twice as many, and rows from
+constexpr int kQuadLongRow = 128;                 // this length
 constexpr float kQuadMaxRate = 0.25f;
 
 template <int kWinners>
@@ -358,7 +360,7 @@ int launch_sbx_pm(RepArgs& R, hipStream_t st)
     const long long paired = static_cast<long long>(R.pairs) * R.d;
     const long long tail = (R.n & 1) ? R.d : 0;
     const float rate = R.mutate ? R.rate_m : 0.0f;
-    const bool quads = !R.sbx_u && !R.pm_gate && paired >= (rate >= kQuadMinRate ? 1 : 2) * kQuadMinPaired &&
+    const bool quads = !R.sbx_u && !R.pm_gate && paired >= (rate >= kQuadMinRate || R.d < kQuadLongRow ? 1 : 2) * kQuadMinPaired &&
                        rate <= kQuadMaxRate * static_cast<float>(R.d) / static_cast<float>(4ll * R.groups);
     const dim3 block(256);
     if (quads) {
