@@ -224,6 +224,7 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
         dom1(kMaxM + 1, std::vector<long long>(count, 0)), apr(kMaxM + 1, std::vector<long long>(count, 0)),
         chunks(kMaxM + 1, std::vector<long long>(count, 0));
     int max_k = 1, max_nm = 1;
+    bool niche_one = true;
     std::vector<int> peel_inst, peel_W0, peel_W1;
     long long total_merged = 0, total_n = 0;
     for (int i = 0; i < count; ++i) {
@@ -256,6 +257,7 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
         dom1[m][i] = static_cast<long long>(I.Wc) * ceil_div(I.W, kBatchDomSeg);
         max_k = std::max(max_k, I.k);
         max_nm = std::max(max_nm, nm);
+        niche_one = niche_one && nm <= batch_niche_max_nm(m);
         peel_inst.push_back(i);
         peel_W0.push_back(W0);
         peel_W1.push_back(I.W);
@@ -290,7 +292,7 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
     G.sel.ref_bits = bitlen(max_k + 1);
     G.sel.rank_bits = bitlen(max_nm);
     G.sel.total_merged = total_merged;
-    G.sel.max_nm = static_cast<int>(max_nm);
+    G.sel.niche_one = niche_one;
     G.nds0.rows256 = T.add(n0_rows);
     G.nds0.prep = T.add(n0_prep);
     G.nds1.rows256 = T.add(n1_rows);

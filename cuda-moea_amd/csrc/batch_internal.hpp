@@ -152,7 +152,7 @@ struct BSelGrids {
     int ref_bits;                 // bits of a direction index (with the two sentinels)
     int rank_bits;                // bits of rho + rank (with the sentinel)
     long long total_merged;       // sum of 2n (sort length)
-    int max_nm;                   // largest 2n of the state's instances
+    bool niche_one;               // every instance niches in a workgroup of its own (batch_niche_max_nm)
 };
 
 struct BNdsScratch {
@@ -187,6 +187,7 @@ int mlp_tile_count(int n, int hidden, bool big);  // blocks of one MLP hidden-la
 bool mlp_fills(long long big_tiles);              // the large tile shape has enough tiles          // evaluate.hip
 size_t batch_nds_sort_bytes(long long total_rows, int inst_bits);                             // nds.hip
 int batch_nds(const BatchLaunch& L, const BNdsGrids& G, const BNdsScratch& S, int mode, int state);  // nds.hip
+int batch_niche_max_nm(int m);                                                                // nsga3.hip
 size_t nds_table_bytes(int nm, int m);                                                        // nds.hip
 int batch_peel_capacity();                                                                    // nds.hip
 int batch_peel_plan(const std::vector<int>& inst, const std::vector<int>& W, int capacity, int rows_per_block,

@@ -2585,11 +2585,20 @@ bool niching_one_block(const moea_niching& c) { return c.mode != 2; }
 int niching_buckets(const moea_niching& c) { return c.mode == 3 ? 0 : 1; }
 // each path also stops at its own LDS capacity
 int niching_lds_cap(const moea_niching& c) { return c.lds_cap > 0 ? c.lds_cap : (1 << 30); }
-// Largest instance (merged rows) of a batch that niches in one workgroup each.
-// 16 served runs of up to 16384 rows: 38 us a step against 135 us with the
-// device-wide sorts; nothing larger is served or batched in the measured mixes.
-constexpr int kBatchNicheMaxNm = 16384;
 }  // namespace
+
+// Largest instance (merged rows) that niches in a workgroup of its own; a batch
+// with a larger one takes the device-wide sorts.  A workgroup is the faster way as
+// long as the last front fits its LDS, which more objectives fill from fewer rows:
+// niching stage in us, a workgroup / device-wide sorts, 1 and 16 runs of
+//     2n       M = 3          M = 4          M = 5          M = 6          M = 8
+//     10000    33/136 37/249  48/139 61/252  63/140 88/253  78/140 97/254  366/141 380/255
+//     13000    36/142 39/355  57/146 110/366 80/150 332/369 411/150        432/150
+//     16384    39/146 44/362  62/151 217/372 157/156 427/375 495/156       535/156
+// (4 runs of 16384 at M = 5: a whole step 650 against 680.)  At 8192 it is 70 to 85
+// against 135 to 235 for M = 6 to 10.  For M <= 3 it wins
+// beyond 16384 too (65536 rows: 116 to 151 against 265 to 443), which is not used yet.
+int batch_niche_max_nm(int m) { return m <= 5 ? 16384 : 8192; }
 
 int nsga3_select(const moea_nsga3_select_args& A)
 {
@@ -3025,10 +3034,7 @@ int batch_select(const BatchLaunch& L, const BSelGrids& G, const BNdsGrids& NG, 
     MOEA_HIP(hipGetLastError());
     stage_end(kStAssociation, st);
     stage_begin(kStNiching, st);
-    // one workgroup per instance up to kBatchNicheMaxNm merged rows; larger
-    // runs (many objectives put most of 2n in the last front) sort faster
-    // device-wide
-    if (niching_one_block(L.niching) && (L.niching.mode == 1 || G.max_nm <= kBatchNicheMaxNm)) {
+    if (niching_one_block(L.niching) && (L.niching.mode == 1 || G.niche_one)) {
         hipLaunchKernelGGL(b_niche, dim3(L.count), dim3(kNicheThreads), 0, st, L.insts, S.keys_in, S.keys_out,
                            S.vals_in, S.vals_out, niching_buckets(L.niching), niching_lds_cap(L.niching));
         MOEA_HIP(hipGetLastError());

@@ -168,13 +168,15 @@ int moea_quantize_cv(const float* cv, float* out, int n, const moea_cv_quantizat
  * counterpart there. */
 typedef struct moea_niching {
     int mode;      /* 0 automatic, 1 one workgroup over only the last front's
-                      members, grouped by direction (a niche of more than 128
-                      members is cut into parts by value first, or falls back
-                      to that workgroup's radix sorts),
+                      members, grouped by direction (where a member would be
+                      compared with more than 96 others of its niche on
+                      average, the niches are cut into parts by value first,
+                      or it falls back to that workgroup's radix sorts),
                       2 three device-wide sorts of all 2n slots, 3 the one
                       workgroup's radix sorts only.  The batched and served
                       engines take one workgroup per instance in mode 1, and
-                      in mode 0 while every instance has 2n <= 16384. */
+                      in mode 0 while every instance has 2n <= 16384 (up to
+                      five objectives) or 8192 (more). */
     int lds_cap;   /* one-workgroup paths: last-front members kept in LDS at
                       most (0: as many as the path's LDS holds, about 9500 for
                       the grouping at K = 32640, 5888 for the radix sorts);

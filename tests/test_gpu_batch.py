@@ -106,3 +106,12 @@ def test_batch_step_and_validation():
         cm.BatchNSGA3([_run(92, 3, 12, 12, 0, 5), _run(92, 3, 12, 12, 0, 6)])
     with pytest.raises(ValueError):
         cm.BatchNSGA3([_run(91, 3, 12, 12, 0, 5)])
+
+
+# about the sizes at which a batch's niching leaves the workgroup of its own
+@pytest.mark.parametrize("mix", [[(8192, 5, 4, 6, 1), (300, 3, 9, 12, 2)], [(8194, 5, 4, 6, 1), (300, 3, 9, 12, 2)],
+                                 [(4096, 8, 3, 3, 3)], [(4098, 8, 3, 3, 3), (64, 3, 5, 12, 4)], [(8192, 4, 3, 8, 5)]])
+def test_batch_niching_lines_equal_single_runs(mix):
+    print(f"batch niching lines {mix}", flush=True)
+    for c, res in zip(mix, cm.BatchNSGA3([_run(*c, 3) for c in mix]).run()):
+        _same(res, _run(*c, 3).run())
