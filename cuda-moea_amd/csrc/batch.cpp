@@ -123,6 +123,7 @@ void fill_record(const moea_batch_problem& p, BInst& I)
     I.nm = z.nm; I.W = z.W; I.Wc = z.Wc; I.npad = z.npad;
     I.max_gen = p.max_generations;
     I.nchunks = assoc_chunks(z.k, z.m);
+    I.ddiv = fast_div_make(static_cast<uint32_t>(z.d));
     I.gdiv = fast_div_make(static_cast<uint32_t>((z.d + 3) / 4));
     I.seed = p.seed;
     I.sbx_eta0 = p.sbx_eta[0]; I.sbx_eta1 = p.sbx_eta[1];
@@ -152,6 +153,7 @@ int validate_problem(const moea_batch_problem& p)
 // Grids of one state (the instances a set of launches serves).
 struct Grids {
     BGrid init256{}, rows256{}, sbx256{};
+    bool sbx_quads = false;       // four variables a thread in sbx256
     BEvalGrids eval{};
     BSelGrids sel{};
     BNdsGrids nds0{}, nds1{};
@@ -226,7 +228,7 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
     int max_k = 1, max_nm = 1;
     bool niche_one = true;
     std::vector<int> peel_inst, peel_W0, peel_W1;
-    long long total_merged = 0, total_n = 0;
+    long long total_merged = 0, total_n = 0, paired = 0;
     for (int i = 0; i < count; ++i) {
         BInst& I = host[i];
         if (I.state != state) continue;
@@ -235,7 +237,7 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
         const int nb = ceil_div(nm, 256);
         init256[i] = ceil_div(static_cast<long long>(n) * I.d, 256);
         rows256[i] = ceil_div(n, 256);
-        sbx256[i] = ceil_div(static_cast<long long>(n / 2) * ((I.d + 3) / 4), 256);
+        paired += static_cast<long long>(n / 2) * I.d;
         merged256[i] = nb;
         objectives[i] = m;
         rows4[i] = ceil_div(n, 4);
@@ -268,6 +270,10 @@ long long build_grids(std::vector<BInst>& host, int state, int peel_capacity, in
     }
     G.init256 = T.add(init256);
     G.rows256 = T.add(rows256);
+    G.sbx_quads = batch_sbx_quads(paired);
+    for (int i = 0; i < count; ++i)
+        if (rows256[i])
+            sbx256[i] = ceil_div(static_cast<long long>(host[i].n / 2) * (G.sbx_quads ? (host[i].d + 3) / 4 : host[i].d), 256);
     G.sbx256 = T.add(sbx256);
     for (int m = 1; m <= kMaxM; ++m) {
         G.eval.quad_rows4[m] = T.add(q4[m]);
@@ -477,7 +483,8 @@ int core_step_launch(BatchCore& C, hipStream_t st)
 {
     BatchLaunch L{C.dev_insts, C.slots, st, C.niching};
     stage_begin(kStReproduce, st);
-    MOEA_CHECK(batch_reproduce(L, C.run.rows256.map, C.run.rows256.blocks, C.run.sbx256.map, C.run.sbx256.blocks));
+    MOEA_CHECK(batch_reproduce(L, C.run.rows256.map, C.run.rows256.blocks, C.run.sbx256.map, C.run.sbx256.blocks,
+                               C.run.sbx_quads));
     stage_end(kStReproduce, st);
     stage_begin(kStEvaluate, st);
     MOEA_CHECK(batch_evaluate(L, C.run.eval, 1));

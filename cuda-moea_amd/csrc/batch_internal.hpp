@@ -32,7 +32,7 @@ struct BInst {
     int nm, W, Wc, npad;          // NDS over the 2n merged rows
     int max_gen;
     int nchunks;                  // assoc_chunks(k, m)
-    FastDiv gdiv;                 // division by ceil(d / 4) (reproduction thread indices)
+    FastDiv ddiv, gdiv;           // division by d and by ceil(d / 4) (reproduction element and thread indices)
     uint64_t seed;
     float sbx_eta0, sbx_eta1, sbx_prob, sbx_copy, pm_eta0, pm_eta1, pm_prob;
     // problem (caller-owned device arrays)
@@ -181,7 +181,8 @@ struct BEvalGrids {
 // population slot: 0 the parents (slot cur), 1 the offspring (slot cur + 1).
 int batch_init_population(const BatchLaunch& L, const BMap& mp, int nblocks);                 // reproduce.hip
 int batch_reproduce(const BatchLaunch& L, const BMap& rows256, int nrows_blocks, const BMap& sbx256,
-                    int nsbx_blocks);                                                         // reproduce.hip
+                    int nsbx_blocks, bool quads);                                             // reproduce.hip
+bool batch_sbx_quads(long long paired);           // four variables a thread for so many pair-variables // reproduce.hip
 int batch_evaluate(const BatchLaunch& L, const BEvalGrids& G, int which);                     // evaluate.hip
 int mlp_tile_count(int n, int hidden, bool big);  // blocks of one MLP hidden-layer launch       // evaluate.hip
 bool mlp_fills(long long big_tiles);              // the large tile shape has enough tiles          // evaluate.hip

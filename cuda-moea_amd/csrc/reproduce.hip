@@ -432,6 +432,15 @@ __global__ void b_mating_kernel(const BInst* __restrict__ insts, BMap mp)
                               nullptr, I.seed, static_cast<uint32_t>(I.gen));
 }
 
+// kQuads: four variables a thread, for batches of kBatchQuadMin pair-variables and
+// more; smaller ones are over sooner with a variable a thread.  Reproduction stage
+// in us, one / four: 12.3 / 15.8 for 1 run of 64 x 5, 13.1 / 16.0 for 16 of 100 x 2,
+// 14.5 / 18.6 for 256 of 64 x 10, 19.0 / 22.5 for 64 of 2048 x 5 (0.3 million), 23.2 /
+// 23.7 for 64 of 2048 x 9 (0.6), 32.6 / 27.4 for 256 of 512 x 17 (1.1), 90.6 / 54.9 for
+// 64 of 2048 x 101 (6.6).
+constexpr long long kBatchQuadMin = 1ll << 20;
+
+template <bool kQuads>
 __global__ __launch_bounds__(256) void b_sbx_pm_kernel(const BInst* __restrict__ insts, BMap mp)
 {
     int local;
@@ -440,6 +449,7 @@ __global__ __launch_bounds__(256) void b_sbx_pm_kernel(const BInst* __restrict__
     const int cur = I.cur, off = (I.cur + 1) % 3, gen = I.gen;
     RepArgs R{};
     R.n = I.n; R.d = I.d; R.pairs = I.n / 2;
+    R.dd = I.ddiv;
     R.groups = (I.d + 3) / 4;
     R.gd = I.gdiv;
     R.small = (static_cast<long long>(R.pairs) + 1) * R.d < (1ll << 31);
@@ -452,8 +462,12 @@ __global__ __launch_bounds__(256) void b_sbx_pm_kernel(const BInst* __restrict__
     R.seed = I.seed; R.gen = static_cast<uint32_t>(gen); R.ox = I.x[off];
     set_derived(R);
     const long long t = static_cast<long long>(local) * blockDim.x + threadIdx.x;
-    if (R.small) sbx_pm_quad<0, true>(R, t);
-    else sbx_pm_quad<0, false>(R, t);
+    if constexpr (kQuads) {
+        if (R.small) sbx_pm_quad<0, true>(R, t);
+        else sbx_pm_quad<0, false>(R, t);
+    } else {
+        sbx_pm_elem<0, true>(R, t);        // fewer than 2^31 elements
+    }
 }
 
 }  // namespace
@@ -551,13 +565,16 @@ int batch_init_population(const BatchLaunch& L, const BMap& mp, int nblocks)
     return kOk;
 }
 
+bool batch_sbx_quads(long long paired) { return paired >= kBatchQuadMin; }
+
 int batch_reproduce(const BatchLaunch& L, const BMap& rows256, int nrows_blocks, const BMap& sbx256,
-                    int nsbx_blocks)
+                    int nsbx_blocks, bool quads)
 {
     if (nrows_blocks <= 0) return kOk;
     hipLaunchKernelGGL(b_mating_kernel, dim3(nrows_blocks), dim3(256), 0, L.stream, L.insts, rows256);
     MOEA_HIP(hipGetLastError());
-    hipLaunchKernelGGL(b_sbx_pm_kernel, dim3(nsbx_blocks), dim3(256), 0, L.stream, L.insts, sbx256);
+    if (quads) hipLaunchKernelGGL(b_sbx_pm_kernel<true>, dim3(nsbx_blocks), dim3(256), 0, L.stream, L.insts, sbx256);
+    else hipLaunchKernelGGL(b_sbx_pm_kernel<false>, dim3(nsbx_blocks), dim3(256), 0, L.stream, L.insts, sbx256);
     MOEA_HIP(hipGetLastError());
     return kOk;
 }

@@ -115,3 +115,11 @@ def test_batch_niching_lines_equal_single_runs(mix):
     print(f"batch niching lines {mix}", flush=True)
     for c, res in zip(mix, cm.BatchNSGA3([_run(*c, 3) for c in mix]).run()):
         _same(res, _run(*c, 3).run())
+
+
+def test_batch_with_four_variables_a_thread_equals_single_runs():
+    """2^20 pair-variables and more: rows of every remainder by four beside a long one."""
+    mix = [(2048, 3, 1030, 12, 1)] + [(100 + 2 * d, 3, d, 12, 10 + d) for d in (1, 2, 3, 4, 5, 6, 7, 8, 9)]
+    print("batch of 2^20 pair-variables", flush=True)
+    for c, res in zip(mix, cm.BatchNSGA3([_run(*c, 4) for c in mix]).run()):
+        _same(res, _run(*c, 4).run())
