@@ -632,18 +632,4 @@ __device__ __forceinline__ T ld_uniform(const T* p, size_t i)
     return ((const_ptr)p)[i];   // address-space conversion (a C-style cast performs it)
 }
 
-// Per lane: acc * 2 + (bit `lane` of mask).  One v_addc_co_u32 with the
-// wave-uniform lane mask as carry-in, i.e. a bit-serial shift of a ballot
-// into a per-lane word.
-__device__ inline uint32_t shift_in(uint32_t acc, uint64_t mask)
-{
-    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(mask)));
-    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(mask >> 32)));
-    const uint64_t m = (static_cast<uint64_t>(hi) << 32) | lo;
-    uint32_t r;
-    uint64_t carry_out;
-    asm("v_addc_co_u32 %0, %1, %2, %2, %3" : "=v"(r), "=s"(carry_out) : "v"(acc), "s"(m));
-    return r;
-}
-
 }  // namespace moea
