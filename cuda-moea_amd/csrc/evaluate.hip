@@ -139,13 +139,16 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 constexpr int kHK = 32;                 // k slice
 constexpr int kHS = kHK + 8;            // LDS row stride, bf16
 // Tile shapes: large ones read X and W1 least and split each number for 128
-// others; small ones where those would leave CUs without work, with more
-// slices in flight, since a slice then costs less than a trip to memory.
+// others; small ones where those would leave CUs without work.
 struct MlpBig { static constexpr int BM = 128, BN = 128, WM = 4, WN = 2, SETS = 2; };
 struct MlpSmall { static constexpr int BM = 64, BN = 64, WM = 2, WN = 2, SETS = 2; };
 constexpr float kMlpScale = 4294967296.0f;   // of X
 constexpr int kMlpFold = 4096;          // k after which a partial sum is folded into the total
-constexpr int kMlpBigTiles = 192;       // tiles of the large shape from which it is used
+// Tiles of the large shape from which it is used; small / large in us at d = 1024 and
+// 8192: 128 tiles (8192 x 256) 46 / 58 and 286 / 354, 160 (10240) 67 / 60 and 427 / 357,
+// 192 (12288) 66 / 61 and 446 / 382, 128 (16384 x 128) 47 / 58 and 312 / 355, 192 (24576 x
+// 128) 69 / 62 and 478 / 403.
+constexpr int kMlpBigTiles = 192;
 
 // (row tile, col tile) of tile index t: the col tiles of one row tile sit
 // 8 indices apart, so a round-robin dispatch over the 8 XCDs puts them on one

@@ -25,9 +25,10 @@
 //  3. nds_dominance: the dominator bitmask B in sorted order, words (p, w) for
 //     w <= hi[p/64], from the rank tables: a search and a table row per
 //     objective give a row's "q_k <= p_k" over a whole chunk.
-//  4. nds_peel: front peeling of the feasible rows with per-row cursors on B
-//     in one cooperative launch; the infeasible rows' fronts follow from their
-//     order alone; fronts are written back in input order.
+//  4. nds_peel: front peeling of the feasible rows with per-row cursors on B,
+//     by one workgroup up to 2048 rows (an ordinary launch) and by cooperating
+//     ones above; the infeasible rows' fronts follow from their order alone;
+//     fronts are written back in input order.
 //
 // Infeasible rows need no bitmask: every feasible row dominates them, among
 // themselves they are ordered by cv alone, and a NaN cv neither dominates nor
@@ -506,7 +507,11 @@ __global__ __launch_bounds__(dom_threads(M)) void nds_dominance(const float* __r
 }
 
 // Row blocks per dominance workgroup: enough workgroups to fill the chip, and
-// enough row blocks in each to pay for loading its tables.
+// enough row blocks in each to pay for loading its tables.  1024 workgroups
+// against 512 and 2048, in us: 33.4 / 34.3 / 29.8 at 32768 rows, M = 3, 160 / 150 /
+// 160 at M = 10; 521 / 522 / 540 at 65536, M = 10; within 1 % below 32768 rows.  At
+// most 64 row blocks against 32 and 128: 101 / 96 / 99 at 65536, M = 3, 521 / 541 / 522
+// at M = 10; at 131072 rows 32 is faster (362 / 287 / 342, 2079 / 1631 / 1999).
 int dom_segment(int W, int Wc, int m)
 {
     const int waves = dom_threads(m) / 64;
@@ -925,9 +930,11 @@ __global__ __launch_bounds__(kPeelThreads) void nds_peel(PeelArgs P)
 // The same with one workgroup, which needs no grid barrier and so no
 // cooperative launch (that leaves the device idle for about 10 us on each
 // side).  Up to kOneGroupBlocks row blocks its 16 waves hold two blocks each,
-// and the rounds cost less than the barriers of more workgroups: the sort's
-// peel stage of 184 rows took 28 us cooperatively, now 7 us, of 2048 rows 32 us,
-// now 20 us.
+// and the rounds cost less than the barriers of more workgroups.  Peel stage in us,
+// one workgroup / cooperating ones (shell of many fronts, then one front): 184
+// rows 7 / 28; 2048 rows M = 2 78 / 132, 19 / 32, M = 10 11 / 29, 9 / 28; 3072 rows M = 3
+// 63 / 63, 35 / 33, M = 10 14 / 30, 10 / 28; 4096 rows M = 3 88 / 71, 52 / 33, M = 10 18 / 30,
+// 12 / 29: above 2048 rows it depends on the fronts.
 constexpr int kOneGroupBlocks = 32;
 
 __global__ __launch_bounds__(kPeelThreads) void nds_peel_one(PeelArgs P)

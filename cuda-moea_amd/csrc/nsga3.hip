@@ -1669,10 +1669,15 @@ __device__ __attribute__((noinline)) void niche_body(Bufs B, NicheArgs A, NicheS
 // batch of 256 runs whose largest gather 8192 members in a few of 91 niches the
 // radix sorts took 218 us, counting without the cut 1484 us, this 71 us.
 constexpr int kNicheLdsBytes = 162816;
+// Pairs a member from which niches are cut; niching stage in us at 32 / 96 / 384 pairs:
+// 8192 members in 45 niches 79 / 79 / 170, 10000 in 45 89 / 89 / 240, in 400 95 / 77 / 77, in 200
+// 85 / 96 / 96, 512 in 15 27 / 24 / 24, 2048 in 91 37 / 30 / 30.
 constexpr uint32_t kBucketMaxPairs = 96;
 constexpr int kBucketSlotBytes = 12;   // LDS: the key 8 B, last-front index and direction word 2 B each
 constexpr int kBucketRegs = 10;        // members a thread holds between two steps (LDS case)
-constexpr int kSelectCount = 384;      // members up to which the n_rem smallest are found by counting
+// Members up to which the n_rem smallest are found by counting; niching stage in us,
+// radix select / counting: 51 members 20 / 17, 184 21 / 19, 307 28.4 / 29.0, 512 22 / 26, 1024 24 / 40.
+constexpr int kSelectCount = 384;
 
 struct BucketSlots {
     uint64_t* key;   // distance bits | t; then phase-4 low word | sort-1 position; then level | draw_b | sort-2 position
@@ -1913,7 +1918,10 @@ __device__ __forceinline__ void bucket_finish(const NicheArgs& A, uint32_t* tabl
 // Each key is then replaced by next(r, st, position), the position broken by the
 // whole key where values tie; V.t travels with the keys.  False (the keys
 // unchanged) when the parts are too uneven.  mm (kUniform: unused): each
-// niche's smallest and largest value.
+// niche's smallest and largest value.  Too uneven: more than kRefineMaxPairs pairs a
+// member.  Niching stage in us at 16 / 64 / 256, last fronts of which a tenth is one
+// point: 2048 members 105 / 42 / 42, 8192 336 / 335 / 103; a fifth: 104 / 104 / 47, 335 / 335 /
+// 335; none: the same (a failed cut costs 6 to 20 us before the radix sorts).
 constexpr uint32_t kRefineMaxPairs = 64;
 
 template <bool kUniform, class Next>

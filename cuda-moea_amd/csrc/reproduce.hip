@@ -337,12 +337,11 @@ __global__ __launch_bounds__(256) void sbx_pm_quads(RepArgs R)
 // Four variables a thread where that is the faster way, one reproduce call in us, a
 // variable a thread against four:
 //  - from 2^24 pair-variables, or 2^25 where hardly any variable of a long row
-//    mutates.  Below, a
-//    variable a thread fills the chip with shorter chains, and an odd last row needs
-//    no launch of its own (2.7 us): 17.1 / 18.2 at 4000 x 1000, 77.1 / 82.1 at
-//    8000 x 4000; at 2^24 93.8 / 89.5 at 32768 x 1024 (rate 2^-10), 81 / 86 at
-//    4096 x 8192 (2^-13), without mutation 80 / 86 at d = 256 and 191 / 180 at 16; above 191 / 171 at 16384 x 4096, 6296 / 5288 at
-//    16384 x 131072.
+//    mutates.  Below, a variable a thread fills the chip with shorter chains, and an
+//    odd last row needs no launch of its own (2.7 us): 17.1 / 18.2 at 4000 x 1000,
+//    77.1 / 82.1 at 8000 x 4000.  At 2^24: 93.8 / 89.5 at 32768 x 1024 (rate 2^-10),
+//    81 / 86 at 4096 x 8192 (2^-13), without mutation 80 / 86 at d = 256 and 191 / 180 at
+//    16.  Above: 191 / 171 at 16384 x 4096, 6296 / 5288 at 16384 x 131072.
 //  - up to a mutation rate of a quarter of the variables in use: a thread works its
 //    mutations off one after another.  At 2^24 and d = 1024: 215 / 134 at rate 0.1,
 //    217 / 178 at 0.25, 220 / 223 at 0.5, 226 / 243 at 1; at d = 5, where five of
