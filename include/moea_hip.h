@@ -178,8 +178,8 @@ typedef struct moea_niching {
                       in mode 0 while every instance has 2n <= 16384 (up to
                       five objectives) or 8192 (more). */
     int lds_cap;   /* one-workgroup paths: last-front members kept in LDS at
-                      most (0: as many as the path's LDS holds, about 9500 for
-                      the grouping at K = 32640, 5888 for the radix sorts);
+                      most (0: as many as the path's LDS holds, 7936 for the
+                      grouping at K = 32640, 5888 for the radix sorts);
                       the others go to the workspace */
 } moea_niching;
 
