@@ -66,12 +66,13 @@ def test_selection_equals_oracle(n, m, k):
     np.testing.assert_array_equal(nfr.cpu().numpy(), fr_mix[chosen])
 
 
-def test_batch_equals_single_runs():
+@pytest.mark.parametrize("graph", [False, True])
+def test_batch_equals_single_runs(graph):
     def runs():                                      # K = 91, 14950, 330 and 2600
         return [cm.NSGA3(population_size=n, max_generations=6, problem=cm.QuadraticCenters(d, m, seed=n), seed=n,
                          reference_directions=cm.DasDennisDirections(partitions=p), print_progress=False)
                 for n, m, d, p in ((100, 3, 10, 12), (130, 5, 20, 22), (64, 8, 9, 4), (200, 4, 16, 23))]
-    batch = cm.BatchNSGA3(runs())
+    batch = cm.BatchNSGA3(runs(), graph=graph)
     batch.initialize()
     batch.step(6)
     for i, alone in enumerate(runs()):
